@@ -512,6 +512,22 @@ size_t workspace_budget()
     return want;
 }
 
+// k_secondary_phase by sample type
+using SecKernel = void (*)(const void*, int, const SecReqDev*, int32_t*);
+SecKernel secondary_kernel(int eltype)
+{
+    switch (eltype) {
+    case FMDBZP_CF32: return k_secondary_phase<FMDBZP_CF32>;
+    case FMDBZP_CF64: return k_secondary_phase<FMDBZP_CF64>;
+    case FMDBZP_I16: return k_secondary_phase<FMDBZP_I16>;
+    case FMDBZP_CI8: return k_secondary_phase<FMDBZP_CI8>;
+    case FMDBZP_CI16: return k_secondary_phase<FMDBZP_CI16>;
+    case FMDBZP_F32: return k_secondary_phase<FMDBZP_F32>;
+    case FMDBZP_F64: return k_secondary_phase<FMDBZP_F64>;
+    default: return k_secondary_phase<FMDBZP_C2BIT>;
+    }
+}
+
 }  // namespace
 
 extern "C" {
@@ -1071,14 +1087,20 @@ int fmdbzp_secondary_phase(fmdbzp_plan* plan, const void* signal, int32_t eltype
         rq[(size_t)i].L = reqs[i].num_rotations;
         rq[(size_t)i].pad = 0;
     }
+    size_t lds_bytes = 0;
+    for (int i = 0; i < nreq; i++) lds_bytes = std::max(lds_bytes, sec_lds(reqs[i].num_rotations));
+    {
+        const int rc = set_lds_attr((const void*)secondary_kernel(eltype), lds_bytes);
+        if (rc) return rc;
+    }
     hipError_t e = hipSuccess;
     if (!dev_sig) e = hipMemcpy(plan->d_signal, signal, sig_bytes, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(d_codes, codes.data(), codes.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(d_secs, secs.data(), secs.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(d_reqs, rq.data(), sizeof(SecReqDev) * (size_t)nreq, hipMemcpyHostToDevice);
     if (e == hipSuccess) {
-        k_secondary_phase<<<nreq, 64, 0, plan->stream>>>(dev_sig ? signal : plan->d_signal, eltype, spc, d_reqs,
-                                                         d_out);
+        secondary_kernel(eltype)<<<nreq, FMDBZP_SEC_NTHR, lds_bytes, plan->stream>>>(
+            dev_sig ? signal : plan->d_signal, spc, d_reqs, d_out);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(out_phase, d_out, sizeof(int32_t) * (size_t)nreq, hipMemcpyDeviceToHost,
@@ -1654,11 +1676,10 @@ int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t elt
                     const int rb4 = (ndop + 4 * FMDBZP_NTHR - 1) / (4 * FMDBZP_NTHR);
                     k_reduce_cols<<<dim3(P->red_nchunk, rb4, cnt), FMDBZP_NTHR, 0, st>>>(
                         acc, P->acc_ps, P->apc, ndop, spc, spc_eff, d.num_secondary_rotations, streamed_rot,
-                        P->red_cw, W.psum + po, W.pbest_v + po, W.pbest_k + po);
+                        P->red_cw, psum, pbest_v, pbest_k);
                     HIP_TRY(hipGetLastError());
-                    k_merge_rows<<<dim3(rb, cnt), FMDBZP_NTHR, 0, st>>>(W.psum + po, W.pbest_v + po,
-                                                                       W.pbest_k + po, P->red_nchunk, ndop,
-                                                                       rowsum, rowbest_v, rowbest_k);
+                    k_merge_rows<<<dim3((ndop + FMDBZP_MERGE_ROWS - 1) / FMDBZP_MERGE_ROWS, cnt), FMDBZP_NTHR, 0, st>>>(
+                        psum, pbest_v, pbest_k, P->red_nchunk, ndop, rowsum, rowbest_v, rowbest_k);
                 } else {
                     k_reduce_rows<<<dim3(ndop, cnt), FMDBZP_NTHR, 0, st>>>(acc, ndop, spc, spc_eff, P->ap,
                                                                            d.num_secondary_rotations, streamed_rot,

@@ -2409,12 +2409,20 @@ k_export_cm(const float* __restrict__ acc, float* __restrict__ out, int ndop, in
 }
 
 // Secondary-code phase of a detected PRN (`_estimate_secondary_code_phase`,
-// src/acquire.jl:503-538), in the reference's order of operations: lane k
-// despreads code period k sequentially, acc += (x * carr) * code with
-// ComplexF32 products (no fused multiply-add) and carr *= dphi, the phasor
-// reset per period from an FP64 sincos; lane 0 then sums the L rotations of
-// the secondary code and keeps the first largest |s|^2. grid (requests),
-// block 64 (L <= 64).
+// src/acquire.jl:503-538), in the reference's order of operations: period k is
+// despread sequentially, acc += (x * carr) * code with ComplexF32 products (no
+// fused multiply-add) and carr *= dphi, the phasor reset per period from an
+// FP64 sincos; the L rotations of the secondary code are then summed in order
+// and the first largest |s|^2 is kept. grid (requests), L <= 64.
+//
+// Two chains are serial by that definition: the phasor of a period (two
+// dependent operations per sample) and its sum (one add). Everything else is
+// not, so the workgroup is a pipeline over chunks of C samples, all periods at
+// once, one barrier per chunk: wave 0 writes the phasors of chunk i to LDS
+// (lane = period), waves 2-7 form the despread products of chunk i - 1 and
+// load the samples of chunk i (lanes along samples: coalesced), wave 1 sums
+// chunk i - 2 (lane = period). The phasor chain bounds it. C is 64 up to 32
+// periods and 32 above, so the four LDS buffers stay within 66 KB.
 struct SecReqDev {
     const int8_t* code;  // spc samples at the estimated code phase
     const int8_t* sec;   // L secondary chips
@@ -2422,67 +2430,127 @@ struct SecReqDev {
     int L;
     int pad;
 };
-__global__ void __launch_bounds__(64)
-k_secondary_phase(const void* __restrict__ sig, int eltype, int spc, const SecReqDev* __restrict__ reqs,
+#define FMDBZP_SEC_NTHR 512
+__host__ __device__ __forceinline__ int sec_chunk(int L) { return L <= 32 ? 64 : 32; }
+__host__ __device__ __forceinline__ int sec_pitch(int L) { return L | 1; }  // odd: lanes along samples spread over the banks
+__host__ __device__ __forceinline__ size_t sec_lds(int L)
+{
+    return (size_t)4 * sec_chunk(L) * sec_pitch(L) * sizeof(float2);
+}
+template <int ELT>
+__global__ void __launch_bounds__(FMDBZP_SEC_NTHR)
+k_secondary_phase(const void* __restrict__ sig, int spc, const SecReqDev* __restrict__ reqs,
                   int32_t* __restrict__ out)
 {
 #pragma clang fp contract(off)
+    constexpr int NPT = FMDBZP_SEC_NTHR - 128;        // product threads
+    constexpr int NI = (64 * 32 + NPT - 1) / NPT;     // products per thread and chunk (C L <= 2048)
     const SecReqDev R = reqs[blockIdx.x];
-    __shared__ float zr[64], zi[64];
-    const int k = threadIdx.x;
-    if (k < R.L) {
-        const int64_t base = (int64_t)k * spc;
-        const double a = R.phase_step * (double)base;
-        float cr = (float)cos(a), ci = (float)sin(a);
-        const float dre = (float)cos(R.phase_step), dim = (float)sin(R.phase_step);
-        float ar = 0.0f, ai = 0.0f;
-        // samples and code chips are loaded 16 at a time ahead of the
-        // recurrence, which then runs over them in order
-        constexpr int B = 16;
-        for (int n0 = 0; n0 < spc; n0 += B) {
-            float2 xs[B];
-            float cs[B];
-#pragma unroll
-            for (int u = 0; u < B; u++) {
-                const int n = min(n0 + u, spc - 1);
-                xs[u] = load_sample(sig, eltype, base + n);
-                cs[u] = (float)R.code[n];
-            }
-#pragma unroll
-            for (int u = 0; u < B; u++) {
-                if (n0 + u < spc) {
-                    const float2 x = xs[u];
-                    const float pr = x.x * cr - x.y * ci, pim = x.x * ci + x.y * cr;
-                    const float c = cs[u];
-                    const float qr = pr * c - pim * 0.0f, qi = pr * 0.0f + pim * c;
-                    ar += qr;
-                    ai += qi;
+    extern __shared__ float2 lds[];
+    __shared__ float zr[64], zi[64], mags[64];
+    const int tid = threadIdx.x, wave = tid >> 6, k = tid & 63;
+    const int L = R.L, C = sec_chunk(L), Lp = sec_pitch(L), lc = C == 64 ? 6 : 5;
+    float2* ph = lds;              // [2][C][Lp] phasors
+    float2* qq = lds + 2 * C * Lp; // [2][C][Lp] despread products
+    const int nch = (spc + C - 1) / C;
+    // wave 0: phasor of period k
+    float cr = 1.0f, ci = 0.0f, dre = 1.0f, dim = 0.0f;
+    if (wave == 0 && k < L) {
+        const double a = R.phase_step * (double)((int64_t)k * spc);
+        cr = (float)cos(a);
+        ci = (float)sin(a);
+        dre = (float)cos(R.phase_step);
+        dim = (float)sin(R.phase_step);
+    }
+    float ar = 0.0f, ai = 0.0f;  // wave 1: sum of period k
+    float2 xs[NI];
+    float cs[NI];
+    for (int i = 0; i < nch + 2; i++) {
+        if (wave == 0) {
+            if (i < nch && k < L) {
+                float2* p = ph + (i & 1) * C * Lp + k;
+                const int m = min(C, spc - i * C);
+#pragma unroll 8
+                for (int n = 0; n < m; n++) {
+                    p[n * Lp] = make_float2(cr, ci);
                     const float ncr = cr * dre - ci * dim, nci = cr * dim + ci * dre;
                     cr = ncr;
                     ci = nci;
                 }
             }
+        } else if (wave == 1) {
+            if (i >= 2 && k < L) {
+                const float2* q = qq + (i & 1) * C * Lp + k;
+                const int m = min(C, spc - (i - 2) * C);
+#pragma unroll 8
+                for (int n = 0; n < m; n++) {
+                    const float2 v = q[n * Lp];
+                    ar += v.x;
+                    ai += v.y;
+                }
+            }
+        } else {
+            const int t = tid - 128;
+            float2 nx[NI];
+            float nc[NI];
+            if (i < nch) {
+#pragma unroll
+                for (int u = 0; u < NI; u++) {
+                    const int e = min(t + NPT * u, C * L - 1);
+                    const int n = min(i * C + (e & (C - 1)), spc - 1), kk = e >> lc;
+                    nx[u] = load_sample(sig, ELT, (int64_t)kk * spc + n);
+                    nc[u] = (float)R.code[n];
+                }
+            }
+            if (i >= 1 && i <= nch) {
+                const int o = ((i - 1) & 1) * C * Lp;
+#pragma unroll
+                for (int u = 0; u < NI; u++) {
+                    const int e = t + NPT * u;
+                    if (e < C * L) {
+                        const int at = o + (e & (C - 1)) * Lp + (e >> lc);
+                        const float2 x = xs[u], w = ph[at];
+                        const float pr = x.x * w.x - x.y * w.y, pim = x.x * w.y + x.y * w.x;
+                        const float c = cs[u];
+                        qq[at] = make_float2(pr * c - pim * 0.0f, pr * 0.0f + pim * c);
+                    }
+                }
+            }
+            if (i < nch) {
+#pragma unroll
+                for (int u = 0; u < NI; u++) {
+                    xs[u] = nx[u];
+                    cs[u] = nc[u];
+                }
+            }
         }
+        __syncthreads();
+    }
+    if (wave == 1 && k < L) {
         zr[k] = ar;
         zi[k] = ai;
     }
     __syncthreads();
-    if (k == 0) {
+    if (tid < L) {  // rotation r = tid
+        float sr = 0.0f, si = 0.0f;
+        for (int q = 0; q < L; q++) {
+            int j = q + tid;
+            if (j >= L) j -= L;
+            const float sv = (float)R.sec[j];
+            sr += sv * zr[q];
+            si += sv * zi[q];
+        }
+        mags[tid] = sr * sr + si * si;
+    }
+    __syncthreads();
+    if (tid == 0) {
         int best_r = 0;
         float best = -1.0f;
-        for (int r = 0; r < R.L; r++) {
-            float sr = 0.0f, si = 0.0f;
-            for (int q = 0; q < R.L; q++) {
-                const float sv = (float)R.sec[(q + r) % R.L];
-                sr += sv * zr[q];
-                si += sv * zi[q];
-            }
-            const float mag = sr * sr + si * si;
-            if (mag > best) {
-                best = mag;
+        for (int r = 0; r < L; r++)
+            if (mags[r] > best) {
+                best = mags[r];
                 best_r = r;
             }
-        }
         out[blockIdx.x] = best_r;
     }
 }
