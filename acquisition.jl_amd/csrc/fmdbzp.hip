@@ -140,6 +140,8 @@ static int corr_nbuf(int v)
     }
 }
 constexpr size_t kLdsDefault = 64 * 1024;
+// bytes of one row's partial of a column-major reduction chunk (FP64 sum, key, value)
+constexpr size_t kRedPart = sizeof(double) + sizeof(uint64_t) + sizeof(float);
 
 struct TimedEvent {
     int cls;
@@ -193,7 +195,8 @@ struct fmdbzp_plan {
     float* d_rowbest_v = nullptr;
     uint64_t* d_rowbest_k = nullptr;
     // column-major accumulator (few columns per column-stage workgroup): the
-    // row reduction runs over column chunks of red_cw, partials per chunk
+    // row reduction runs over column chunks of red_cw, partials per chunk in
+    // the consumed tile
     bool acc_cm = false;
     int apc = 0;             // column pitch (ndop rounded up to 32)
     size_t acc_ps = 0;       // accumulator elements per PRN
@@ -798,8 +801,6 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         P->nsub = (P->chunk_cols + P->red_cw - 1) / P->red_cw;
         P->nparts = P->nchunks * R * P->nsub;
     }
-    P->red_cw = 4096;
-    P->red_nchunk = (spc_eff + P->red_cw - 1) / P->red_cw;
     P->col_lds = per_col * LB + fixed;
     if (P->col_static) P->col_lds = (size_t)LB * P->bstride * sizeof(float2);  // one column buffer
     if (P->rot2000)
@@ -929,7 +930,7 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
     const int tile_blocks = P->rotbig ? P->nrb_max : nb;
     {
         size_t per_prn = (size_t)tile_blocks * ndop * P->tp * sizeof(float2) * (P->col_pair ? 2 : 1) +
-                         P->acc_ps * sizeof(float) + (P->acc_cm ? (size_t)P->red_nchunk * ndop * 20 : 0);
+                         P->acc_ps * sizeof(float);
         if (P->rotbig)
             per_prn = (size_t)tile_blocks * ndop * P->tp * sizeof(float2) + P->acc_ps * sizeof(float) +
                       (size_t)P->nparts * ndop * (8 + 4 + 8 + 16) + (size_t)ndop * 16 +
@@ -942,6 +943,20 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         P->batch = (int)b;
         P->nlanes = P->batch >= lanes_requested() && !P->rotbig ? lanes_requested() : 1;
     }
+    if (P->acc_cm && !P->rotbig) {
+        // columns per workgroup of the column-major reduction: about 1024
+        // workgroups over the batch, 32 to 4096 columns each. With 4096
+        // columns always, 8 PRNs of 4000 columns (640 Doppler rows) ran on 8
+        // workgroups, 1430 us; a 2.5 M-column surface keeps 4096. The
+        // partials (20 bytes per row and chunk) live in the batch's tile,
+        // which is consumed by then: wider chunks where they would not fit.
+        const size_t rb4 = (ndop + 4 * FMDBZP_NTHR - 1) / (4 * FMDBZP_NTHR);
+        const size_t cw = (size_t)spc_eff * rb4 * P->batch / 1024;
+        P->red_cw = (int)std::min<size_t>(4096, std::max<size_t>(32, (cw + 31) / 32 * 32));
+        auto nchunk = [&]() { return (spc_eff + P->red_cw - 1) / P->red_cw; };
+        while ((size_t)nchunk() * kRedPart > (size_t)nb * P->tp * sizeof(float2)) P->red_cw *= 2;
+        P->red_nchunk = nchunk();
+    }
     if ((rc = dev_alloc(&P->d_tile, (size_t)P->batch * tile_blocks * ndop * P->tp)) ||
         (P->col_pair && (rc = dev_alloc(&P->d_tile2, (size_t)P->batch * tile_blocks * ndop * P->tp))) ||
         (rc = dev_alloc(&P->d_acc, (size_t)P->batch * P->acc_ps)) ||
@@ -949,14 +964,13 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         (rc = dev_alloc(&P->d_rowbest_v, (size_t)P->batch * ndop)) ||
         (rc = dev_alloc(&P->d_rowbest_k, (size_t)P->batch * ndop)))
         return fail(rc);
-    if (P->acc_cm) {
-        const size_t np = (size_t)P->batch * (P->rotbig ? P->nparts : P->red_nchunk) * ndop;
+    if (P->rotbig) {
+        const size_t np = (size_t)P->batch * P->nparts * ndop;
         if ((rc = dev_alloc(&P->d_psum, np)) || (rc = dev_alloc(&P->d_pbest_v, np)) ||
-            (rc = dev_alloc(&P->d_pbest_k, np)))
+            (rc = dev_alloc(&P->d_pbest_k, np)) || (rc = dev_alloc(&P->d_pnbr, np)) ||
+            (rc = dev_alloc(&P->d_rownbr, (size_t)P->batch * ndop)))
             return fail(rc);
-        if (P->rotbig && ((rc = dev_alloc(&P->d_pnbr, np)) || (rc = dev_alloc(&P->d_rownbr, (size_t)P->batch * ndop))))
-            return fail(rc);
-        if (P->rotbig && d.noise_estimator == FMDBZP_NOISE_GLOBAL_MEAN &&
+        if (d.noise_estimator == FMDBZP_NOISE_GLOBAL_MEAN &&
             (rc = dev_alloc(&P->d_colsum, (size_t)P->batch * spc_eff)))
             return fail(rc);
     }
@@ -1671,8 +1685,10 @@ int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t elt
             {
                 Timed t(P, FMDBZP_K_REDUCE, st, W.timing);
                 if (P->acc_cm) {
-                    const size_t po = (size_t)lo * P->red_nchunk * ndop;
-                    const int rb = (ndop + FMDBZP_NTHR - 1) / FMDBZP_NTHR;
+                    const size_t np = (size_t)cnt * P->red_nchunk * ndop;
+                    double* psum = (double*)tile;
+                    uint64_t* pbest_k = (uint64_t*)(psum + np);
+                    float* pbest_v = (float*)(pbest_k + np);
                     const int rb4 = (ndop + 4 * FMDBZP_NTHR - 1) / (4 * FMDBZP_NTHR);
                     k_reduce_cols<<<dim3(P->red_nchunk, rb4, cnt), FMDBZP_NTHR, 0, st>>>(
                         acc, P->acc_ps, P->apc, ndop, spc, spc_eff, d.num_secondary_rotations, streamed_rot,
@@ -2058,7 +2074,9 @@ extern "C" int fmdbzp_acquire_noalloc(fmdbzp_plan* plan, const void* signal, int
     const size_t b_stats = align256(sizeof(fmdbzp_prn_stats) * (size_t)nreq);
     const size_t t_prn = align256(sizeof(float2) * (size_t)d.num_blocks * ndop * P->tp);
     const size_t a_prn = align256(sizeof(float) * P->acc_ps);
-    const size_t np = P->acc_cm ? (size_t)P->red_nchunk * ndop : 0;
+    // the size limit counts a reduction partial per row and 4096 columns beside
+    // the tile (they are kept in the tile)
+    const size_t np = P->acc_cm ? (size_t)((d.samples_per_code_eff + 4095) / 4096) * ndop : 0;
     const size_t r_prn = align256(sizeof(double) * ndop) + align256(sizeof(float) * ndop) +
                          align256(sizeof(uint64_t) * ndop) + align256(sizeof(double) * np) +
                          align256(sizeof(float) * np) + align256(sizeof(uint64_t) * np);
@@ -2108,9 +2126,6 @@ extern "C" int fmdbzp_acquire_noalloc(fmdbzp_plan* plan, const void* signal, int
     W.rowsum = (double*)take(sizeof(double) * ndop * batch);
     W.rowbest_v = (float*)take(sizeof(float) * ndop * batch);
     W.rowbest_k = (uint64_t*)take(sizeof(uint64_t) * ndop * batch);
-    W.psum = (double*)take(sizeof(double) * np * batch);
-    W.pbest_v = (float*)take(sizeof(float) * np * batch);
-    W.pbest_k = (uint64_t*)take(sizeof(uint64_t) * np * batch);
     W.batch = batch;
     W.nlanes = 1;
     W.timing = false;

@@ -1295,26 +1295,47 @@ k_reduce_cols(const float* __restrict__ acc, size_t acc_ps, int ldc, int ndop, i
     }
 }
 
-// Column-major accumulator, pass 2. grid (ceil(ndop / NTHR), batch): per row,
-// the chunk partials in chunk order give the row sum and the row's best cell.
+// Column-major accumulator, pass 2. grid (ceil(ndop / MERGE_ROWS), batch): 32
+// rows per workgroup, eight threads per row, each over a contiguous eighth of
+// the chunks in order; the eighths are combined in order. One thread per row
+// walked 611 dependent chunks in 290 us (2000 rows, 2.5 M columns).
+#define FMDBZP_MERGE_ROWS 32
 __global__ void __launch_bounds__(FMDBZP_NTHR)
 k_merge_rows(const double* __restrict__ psum, const float* __restrict__ pbest_v,
              const uint64_t* __restrict__ pbest_k, int nchunk, int ndop, double* __restrict__ rowsum,
              float* __restrict__ rowbest_v, uint64_t* __restrict__ rowbest_k)
 {
-    const int row = blockIdx.x * FMDBZP_NTHR + threadIdx.x, p = blockIdx.y;
-    if (row >= ndop) return;
+    constexpr int G = FMDBZP_NTHR / FMDBZP_MERGE_ROWS;
+    __shared__ double ss[G][FMDBZP_MERGE_ROWS];
+    __shared__ float sv[G][FMDBZP_MERGE_ROWS];
+    __shared__ uint64_t sk[G][FMDBZP_MERGE_ROWS];
+    const int lr = threadIdx.x % FMDBZP_MERGE_ROWS, g = threadIdx.x / FMDBZP_MERGE_ROWS;
+    const int row = blockIdx.x * FMDBZP_MERGE_ROWS + lr, p = blockIdx.y;
+    const int per = (nchunk + G - 1) / G;
     double s = 0.0;
     float bv = -INFINITY;
     uint64_t bk = ~0ull;
-    for (int c = 0; c < nchunk; c++) {
-        const size_t o = ((size_t)p * nchunk + c) * ndop + row;
-        s += psum[o];
-        if (better(pbest_v[o], pbest_k[o], bv, bk)) { bv = pbest_v[o]; bk = pbest_k[o]; }
+    if (row < ndop) {
+#pragma unroll 4
+        for (int c = g * per; c < min(nchunk, (g + 1) * per); c++) {
+            const size_t o = ((size_t)p * nchunk + c) * ndop + row;
+            s += psum[o];
+            if (better(pbest_v[o], pbest_k[o], bv, bk)) { bv = pbest_v[o]; bk = pbest_k[o]; }
+        }
     }
-    rowsum[(size_t)p * ndop + row] = s;
-    rowbest_v[(size_t)p * ndop + row] = bv;
-    rowbest_k[(size_t)p * ndop + row] = bk;
+    ss[g][lr] = s;
+    sv[g][lr] = bv;
+    sk[g][lr] = bk;
+    __syncthreads();
+    if (g == 0 && row < ndop) {
+        for (int h = 1; h < G; h++) {
+            s += ss[h][lr];
+            if (better(sv[h][lr], sk[h][lr], bv, bk)) { bv = sv[h][lr]; bk = sk[h][lr]; }
+        }
+        rowsum[(size_t)p * ndop + row] = s;
+        rowbest_v[(size_t)p * ndop + row] = bv;
+        rowbest_k[(size_t)p * ndop + row] = bk;
+    }
 }
 
 // grid (batch): peak, noise estimate (src/acquire.jl:687-697,
