@@ -31,6 +31,7 @@ OPT_LITERAL_EDGES = 0x1  # FMDBZP_OPT_LITERAL_EDGES
 OPT_GRAPH = 0x2          # FMDBZP_OPT_GRAPH
 OPT_AUTOTUNE = 0x4       # FMDBZP_OPT_AUTOTUNE
 OPT_FP64_PHASE = 0x8     # FMDBZP_OPT_FP64_PHASE
+OPT_TILE_PATH = 0x10     # FMDBZP_OPT_TILE_PATH
 
 
 def nextprod(factors: Sequence[int], n: int) -> int:
@@ -404,7 +405,8 @@ def plan_desc_fields(plan: AcquisitionPlan) -> dict:
         options=(OPT_LITERAL_EDGES if getattr(plan, "literal_edges", False) else 0)
         | (OPT_GRAPH if getattr(plan, "graphs", False) else 0)
         | (OPT_AUTOTUNE if getattr(plan, "autotune", False) else 0)
-        | (OPT_FP64_PHASE if getattr(plan, "fp64_carrier_phase", False) else 0),
+        | (OPT_FP64_PHASE if getattr(plan, "fp64_carrier_phase", False) else 0)
+        | (OPT_TILE_PATH if getattr(plan, "tile_path", False) else 0),
         sampling_freq_hz=plan.sampling_freq,
     )
 

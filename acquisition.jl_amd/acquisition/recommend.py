@@ -340,19 +340,23 @@ class GpuCostModel:
     @staticmethod
     def measure(system: GNSSSystem, sampling_freq: float, num_coherently_integrated_code_periods: int,
                 nprn: int, *, min_doppler_coverage: float = 7000.0, repeats: int = 3, seed: int = 1) -> dict:
-        """Run the engine at one geometry on the device (noise input, N_nc 2,
-        `nprn` PRNs) and return the geometry with the mean correlation and
-        column kernel time per noncoherent step and PRN batch (seconds), from
-        the engine's HIP-event timing. One correlation launch runs per step
+        """Run the engine's tile kernels (the model's two stages) at one
+        geometry on the device (noise input, N_nc 2, `nprn` PRNs) and return
+        the geometry with the mean correlation and column kernel time per
+        noncoherent step and PRN batch (seconds), from the engine's HIP-event
+        timing. One correlation launch runs per step
         and batch; a column launch may carry two steps (k_column_c160_pair),
         so both totals are divided by the correlation launch count."""
+        from . import _native
         from .acquire import acquire_
-        from .plan import plan_acquire
+        from .plan import _plan_host
 
         N = num_coherently_integrated_code_periods
         prns = list(range(1, nprn + 1))
-        plan = plan_acquire(system, sampling_freq, prns, min_doppler_coverage=min_doppler_coverage,
-                            num_coherently_integrated_code_periods=N, num_noncoherent_accumulations=2)
+        plan = _plan_host(system, sampling_freq, prns, min_doppler_coverage=min_doppler_coverage,
+                          num_coherently_integrated_code_periods=N, num_noncoherent_accumulations=2)
+        plan.tile_path = True
+        plan.native = _native.NativePlan.create(plan)
         try:
             spc, nb, F, ndop = plan.samples_per_code, plan.num_blocks, plan.fft_size, plan.num_doppler_bins
             n = 2 * N * spc + spc

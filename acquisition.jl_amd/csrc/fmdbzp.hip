@@ -25,6 +25,7 @@
 
 #include "../../include/fmdbzp.h"
 #include "kernels.hpp"
+#include "full_corr.hpp"
 #include "synth.hpp"
 
 namespace {
@@ -120,6 +121,76 @@ int make_row_plan(int n, FftPlanDev* p)
 
 constexpr size_t kLdsMax = 160 * 1024;   // gfx950 LDS per workgroup
 
+// Radix sequence of the full-period transform (full_corr.hpp) of n points: the
+// cheapest ordered product of its radices under a per-point cost of the
+// butterflies and of each further pass (twiddle, addresses, LDS, barrier),
+// with a stage's cost scaled up to whole waves on the four SIMDs. The first
+// radix is odd unless n is a power of two (bank spread); with one noncoherent
+// step 25 may run first and 20 and 22 in the middle, else at most 16. false: n has a
+// prime factor above 13, more than FC_MAX_STAGES stages, or fewer than two.
+bool make_full_plan(int n, int nthr, bool multi, FullPlanDev* f, std::vector<float2>* tw)
+{
+    struct Radix {
+        int r;
+        double cost;
+    };
+    static const Radix kRadix[] = {{2, 2},     {3, 5.3},   {4, 4},     {5, 6.4},   {6, 7.3},   {7, 9},
+                                   {8, 6.5},   {9, 12.4},  {10, 8.4},  {11, 14},   {12, 9.3},  {13, 16},
+                                   {15, 11.7}, {16, 10.5}, {20, 10.4}, {22, 16},   {25, 15.4}};
+    const bool pow2 = (n & (n - 1)) == 0;
+    std::vector<int> best, cur;
+    double best_cost = 1e30;
+    auto search = [&](auto&& self, int left, double cost) -> void {
+        if (cost >= best_cost || (int)cur.size() > FC_MAX_STAGES) return;
+        if (left == 1) {
+            // the last stage: at most FC_CELLS outputs per thread
+            if (cur.size() >= 2 && cur.back() <= 16 && n / cur.back() <= FC_CELLS / cur.back() * nthr) {
+                best = cur;
+                best_cost = cost;
+            }
+            return;
+        }
+        if ((int)cur.size() == FC_MAX_STAGES) return;
+        for (const Radix& x : kRadix) {
+            if (left % x.r != 0) continue;
+            const bool first = cur.empty();
+            if (x.r > 16 && (multi || (first ? x.r != 25 : x.r > 22))) continue;
+            if (first && !pow2 && x.r % 2 == 0) continue;
+            const int waves = (n / x.r + 63) / 64;
+            const double fill = (double)((waves + 3) / 4 * 4 * 64) * x.r / n;
+            cur.push_back(x.r);
+            self(self, left / x.r, cost + (x.cost + 16.0) * std::min(fill, 4.0));
+            cur.pop_back();
+        }
+    };
+    if (n < 64) return false;
+    search(search, n, 0.0);
+    if (best.empty()) return false;
+    *f = FullPlanDev{};
+    f->n = n;
+    f->nst = (int)best.size();
+    f->pad_shift = 31;
+    if (best[0] % 2 == 0) f->pad_shift = __builtin_ctz((unsigned)best[0]);
+    int ns = 1;
+    tw->clear();
+    for (int t = 0; t < f->nst; t++) {
+        const int R = best[(size_t)t];
+        f->radix[t] = R;
+        f->ns[t] = ns;
+        f->inv_ns[t] = 1.0f / (float)ns;
+        f->twoff[t] = (int)tw->size();
+        if (t > 0)
+            for (int r = 1; r < R; r++)
+                for (int k = 0; k < ns; k++) {
+                    double s, c;
+                    sincospi_d(2.0 * (double)((int64_t)r * k) / ((double)ns * R), &s, &c);
+                    tw->push_back(make_float2((float)c, (float)(-s)));
+                }
+        ns *= R;
+    }
+    return true;
+}
+
 // k_corr_tile variants: transforms per pass and LDS transform buffers
 static int corr_nt(int v)
 {
@@ -139,6 +210,35 @@ static int corr_nbuf(int v)
     default: return 2;  // two transforms per pass, or the ping-pong pair
     }
 }
+
+// Axes of the 31 x rb x rc transform of n points (full_corr.hpp): pairwise
+// coprime, radices of its switches, the widest c axis (the fewest last-stage
+// butterflies). rc is odd but for 22 = 2 mod 4, which spreads its stride over
+// the banks; pk = 4 mod 8 does so for the four row groups that a
+// wave stores from the matrix products.
+bool make_full31_plan(int n, Full31Dev* f)
+{
+    if (n % 31 != 0 || (n / 31) % 31 == 0) return false;
+    const int m = n / 31;
+    bool found = false;
+    for (int rb = 2; rb <= 24; rb++) {
+        if (m % rb != 0 || !fc31_b_ok(rb) || !fc31_c_ok(m / rb)) continue;
+        const int rc = m / rb;
+        int a = rb, b = rc;
+        while (b) {
+            const int t = a % b;
+            a = b;
+            b = t;
+        }
+        if (a != 1) continue;
+        if (found && rc <= f->rc) continue;
+        *f = Full31Dev{n, m, rb, rc, rc, 0, 1.0f / (float)rb, 1.0f / (float)rc};
+        f->pk = m + 1 + ((4 - (m + 1) % 8) + 8) % 8;  // at least one spare slot per row
+        found = true;
+    }
+    return found;
+}
+
 constexpr size_t kLdsDefault = 64 * 1024;
 // bytes of one row's partial of a column-major reduction chunk (FP64 sum, key, value)
 constexpr size_t kRedPart = sizeof(double) + sizeof(uint64_t) + sizeof(float);
@@ -189,6 +289,7 @@ struct fmdbzp_plan {
     size_t signal_cap = 0;
     float2* d_sigfft = nullptr;
     float2* d_tile = nullptr;
+    size_t tile_elems = 0;
     float2* d_tile2 = nullptr;   // second step's tile of a two-step column launch (col_pair)
     float* d_acc = nullptr;
     double* d_rowsum = nullptr;
@@ -232,6 +333,16 @@ struct fmdbzp_plan {
     bool col_pair = false;
     std::vector<uint8_t> pair_ok;
     size_t col_lds2 = 0;
+    // full-period correlation (full_corr.hpp): statistics-only calls of simple
+    // plans; the tile, if other calls need it, is allocated by the first of them
+    bool full = false;
+    FullPlanDev fp{};
+    Full31Dev fp31{};                // the chip-rate multiples' form (fp31.n != 0)
+    int full_nthr = 0;
+    size_t full_lds = 0;
+    float2* d_full_tw = nullptr;
+    float2* d_full_code = nullptr;   // [nprn][ndop][spc] code spectra
+    uint16_t* d_full_map = nullptr;  // [spc] column of delay tau
     bool tile_half = false;      // FMDBZP_PREC_TILE_FP16: FP16 coherent tile
     bool tile_auto = false;      // FMDBZP_PREC_AUTO on a plan that admits the FP16 tile: per call, by sample type
     bool rot_direct = false;     // rotation kernel writes transform outputs straight to the accumulator
@@ -291,6 +402,7 @@ namespace {
 
 int acquire_finish(fmdbzp_plan* P);
 int autotune(fmdbzp_plan* P);
+size_t workspace_budget();
 
 size_t elsize(int eltype)
 {
@@ -467,6 +579,9 @@ void free_plan(fmdbzp_plan* P)
     hipFree(P->d_sigfft);
     hipFree(P->d_tile);
     hipFree(P->d_tile2);
+    hipFree(P->d_full_tw);
+    hipFree(P->d_full_code);
+    hipFree(P->d_full_map);
     hipFree(P->d_acc);
     hipFree(P->d_rowsum);
     hipFree(P->d_rowbest_v);
@@ -513,6 +628,93 @@ size_t workspace_budget()
         if (want > cap) want = cap;
     }
     return want;
+}
+
+// The coherent tile (and the second one of two-step column launches). Plans
+// whose calls normally run the full-period correlation allocate it with the
+// first call that needs it.
+int ensure_tile(fmdbzp_plan* P)
+{
+    int rc;
+    if (!P->d_tile && (rc = dev_alloc(&P->d_tile, P->tile_elems))) return rc;
+    if (P->col_pair && !P->d_tile2 && (rc = dev_alloc(&P->d_tile2, P->tile_elems))) return rc;
+    return FMDBZP_OK;
+}
+
+// Full-period correlation of a plan, where it admits it: simple column stage
+// (any E with one data bit included), the code period's transform in one LDS
+// buffer with the axes of make_full31_plan or the radices of make_full_plan,
+// and the code spectra, plan data like the code FFTs, within a quarter of the
+// free memory (else, or when their allocation fails, the plan keeps to the
+// tile path; not by the workspace budget, which must not change results).
+int full_create(fmdbzp_plan* P, const int8_t* d_codes)
+{
+    const fmdbzp_plan_desc& d = P->d;
+    const int n = d.samples_per_code, ndop = d.num_doppler_bins;
+    if (!P->simple_kernel || P->tile_half || n > 65535 || (d.options & FMDBZP_OPT_TILE_PATH)) return FMDBZP_OK;
+    if ((int64_t)d.num_coh * n > INT32_MAX || (size_t)P->ap * 4 > UINT32_MAX) return FMDBZP_OK;
+    // 32 elements behind the last spectrum: k_full31_corr's groups read past a row's end
+    const size_t spec = ((size_t)P->nprn * ndop * n + 32) * sizeof(float2);
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || spec > free_b / 4) return FMDBZP_OK;
+    const int nb = d.num_blocks, bs = d.block_size;
+    auto column = [&](int tau) { return (uint16_t)(((nb - tau / bs) % nb) * bs + tau % bs); };
+    std::vector<float2> tw;
+    std::vector<uint16_t> map((size_t)n);
+    int rc;
+    if (make_full31_plan(n, &P->fp31)) {
+        const Full31Dev& q = P->fp31;
+        map.assign((size_t)(q.rc + 1) / 2 * 2 * 31 * q.rb, 0);
+        P->full_lds = (size_t)fc31_lds_span(q) * sizeof(float2);
+        // one butterfly of the last stage per thread, 24 or 32 cells per thread
+        P->full_nthr = (31 * q.rb > 256 || n > 6144) ? 512 : 256;
+        if (31 * q.rb > P->full_nthr || n > 32 * P->full_nthr) {
+            P->fp31.n = 0;
+            return FMDBZP_OK;
+        }
+        for (int tau = 0; tau < n; tau++)
+            map[((size_t)(tau % q.rc / 2) * 31 * q.rb + (tau % 31) * q.rb + tau % q.rb) * 2 + (tau % q.rc) % 2] = column(tau);
+    } else {
+        P->fp31.n = 0;
+        P->full_nthr = n > 10240 ? 1024 : n > 5120 ? 512 : 256;  // at most FC_CELLS cells per thread
+        if (!make_full_plan(n, P->full_nthr, d.num_noncoherent > 1, &P->fp, &tw)) return FMDBZP_OK;
+        P->full_lds = (size_t)fc_lds_span(P->fp) * sizeof(float2);
+        for (int tau = 0; tau < n; tau++) map[(size_t)tau] = column(tau);
+    }
+    // the cell exchange reads whole groups of four cells per thread
+    const size_t group = (size_t)4 * P->full_nthr;
+    P->full_lds = std::max(P->full_lds, ((size_t)n + group - 1) / group * group * sizeof(float));
+    if (P->full_lds > kLdsMax) return FMDBZP_OK;
+    if ((rc = set_lds_attr((const void*)k_full_corr<256, true>, P->full_lds)) ||
+        (rc = set_lds_attr((const void*)k_full_corr<256, false>, P->full_lds)) ||
+        (rc = set_lds_attr((const void*)k_full_corr<512, true>, P->full_lds)) ||
+        (rc = set_lds_attr((const void*)k_full_corr<512, false>, P->full_lds)) ||
+        (rc = set_lds_attr((const void*)k_full_corr<1024, true>, P->full_lds)) ||
+        (rc = set_lds_attr((const void*)k_full_corr<1024, false>, P->full_lds)) ||
+        (rc = set_lds_attr((const void*)k_full31_corr<256>, P->full_lds)) ||
+        (rc = set_lds_attr((const void*)k_full31_corr<512>, P->full_lds)) ||
+        (rc = set_lds_attr((const void*)k_full_signal<512>, P->full_lds)) ||
+        (rc = set_lds_attr((const void*)k_full31_signal<512>, P->full_lds)) ||
+        (rc = set_lds_attr((const void*)k_full_code, P->full_lds)) ||
+        (rc = set_lds_attr((const void*)k_full31_code, P->full_lds)))
+        return rc;
+    if (hipMalloc((void**)&P->d_full_code, spec) != hipSuccess) {
+        (void)hipGetLastError();
+        P->d_full_code = nullptr;
+        return FMDBZP_OK;
+    }
+    if ((rc = dev_alloc(&P->d_full_tw, tw.size())) || (rc = dev_alloc(&P->d_full_map, map.size()))) return rc;
+    HIP_TRY(hipMemcpy(P->d_full_tw, tw.data(), sizeof(float2) * tw.size(), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemcpy(P->d_full_map, map.data(), sizeof(uint16_t) * map.size(), hipMemcpyHostToDevice));
+    if (P->fp31.n)
+        k_full31_code<<<dim3(ndop, P->nprn), FC_FWD_NTHR, P->full_lds, P->stream>>>(
+            d_codes, P->d_full_code, P->fp31, bs, d.num_coh, 1.0f / (float)n);
+    else
+        k_full_code<<<dim3(ndop, P->nprn), FC_FWD_NTHR, P->full_lds, P->stream>>>(
+            d_codes, P->d_full_code, P->fp, P->d_full_tw, bs, d.num_coh, 1.0f / (float)n);
+    HIP_TRY(hipGetLastError());
+    P->full = true;
+    return FMDBZP_OK;
 }
 
 // k_secondary_phase by sample type
@@ -920,6 +1122,11 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
                                                                               P->d_twF, spc, nb, bs, P->pscale);
             e = hipGetLastError();
         }
+        if (e == hipSuccess && (rc = full_create(P, d_codes))) {
+            hipStreamSynchronize(P->stream);
+            hipFree(d_codes);
+            return fail(rc);
+        }
         if (e == hipSuccess) e = hipStreamSynchronize(P->stream);
         hipFree(d_codes);
         if (e != hipSuccess) return fail(set_err(FMDBZP_EHIP, "code FFT failed: %s", hipGetErrorString(e)));
@@ -957,9 +1164,8 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         while ((size_t)nchunk() * kRedPart > (size_t)nb * P->tp * sizeof(float2)) P->red_cw *= 2;
         P->red_nchunk = nchunk();
     }
-    if ((rc = dev_alloc(&P->d_tile, (size_t)P->batch * tile_blocks * ndop * P->tp)) ||
-        (P->col_pair && (rc = dev_alloc(&P->d_tile2, (size_t)P->batch * tile_blocks * ndop * P->tp))) ||
-        (rc = dev_alloc(&P->d_acc, (size_t)P->batch * P->acc_ps)) ||
+    P->tile_elems = (size_t)P->batch * tile_blocks * ndop * P->tp;
+    if ((!P->full && (rc = ensure_tile(P))) || (rc = dev_alloc(&P->d_acc, (size_t)P->batch * P->acc_ps)) ||
         (rc = dev_alloc(&P->d_rowsum, (size_t)P->batch * ndop)) ||
         (rc = dev_alloc(&P->d_rowbest_v, (size_t)P->batch * ndop)) ||
         (rc = dev_alloc(&P->d_rowbest_k, (size_t)P->batch * ndop)))
@@ -1245,6 +1451,19 @@ struct Work {
 int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t eltype, double interm_freq_hz,
                    int32_t nreq, uint32_t flags, float* const* out_surfaces);
 
+bool int_samples(int32_t eltype)
+{
+    return eltype == FMDBZP_I16 || eltype == FMDBZP_CI8 || eltype == FMDBZP_CI16 || eltype == FMDBZP_C2BIT;
+}
+
+// Whether a call runs the full-period correlation: not with surfaces (their
+// time is the copy to the caller, and the tile path's column kernels stay the
+// ones that write them), nor where FMDBZP_PREC_AUTO takes the FP16 tile.
+bool full_call(const fmdbzp_plan* P, int32_t eltype, bool store)
+{
+    return P->full && !store && !(P->tile_auto && int_samples(eltype));
+}
+
 // Enqueue one search on the plan's stream; statistics land in the plan's
 // pinned staging buffer and are returned by acquire_finish. The caller holds
 // the plan's mutex.
@@ -1314,6 +1533,10 @@ int acquire_enqueue(fmdbzp_plan* P, const void* signal, int32_t eltype, int64_t 
     if (store && !P->d_export && !(flags & FMDBZP_FLAG_DEVICE_OUTPUT))
         HIP_TRY(hipMalloc((void**)&P->d_export, sizeof(float) * (size_t)ndop * surf_cols * kLanes));
 
+    if (!full_call(P, eltype, store)) {
+        const int rc = ensure_tile(P);
+        if (rc) return rc;
+    }
     Work W{P->d_sigfft, P->d_tile, P->d_acc, P->d_rowsum, P->d_rowbest_v, P->d_rowbest_k, P->d_psum,
            P->d_pbest_v, P->d_pbest_k, P->d_req, P->d_stats, P->batch, P->nlanes, true,
            P->col_pair ? P->d_tile2 : nullptr};
@@ -1525,6 +1748,72 @@ int launch_rotbig(fmdbzp_plan* P, const Work& W, ColumnArgs A, int32_t nreq, boo
     return FMDBZP_OK;
 }
 
+// Full-period correlation search (full_corr.hpp) on the plan's stream.
+int launch_full(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t eltype, double interm_freq_hz, int32_t nreq)
+{
+    const fmdbzp_plan_desc& d = P->d;
+    const int n = d.samples_per_code, ncoh = d.num_coh, nnc = d.num_noncoherent, ndop = d.num_doppler_bins;
+    const int do_if = interm_freq_hz == 0.0 ? 0 : (d.options & FMDBZP_OPT_FP64_PHASE) ? 2 : 1;
+    const double dstep = (-6.283185307179586 * interm_freq_hz) / d.sampling_freq_hz;  // Julia `2π`
+    hipStream_t st = P->stream;
+    {
+        Timed t(P, FMDBZP_K_SIGNAL_FFT, st, W.timing);
+        if (ncoh > 1) {
+            k_full_fold<<<dim3((n + 255) / 256, (ncoh + FC_FOLD_SB - 1) / FC_FOLD_SB, nnc), 256,
+                          sizeof(float2) * (size_t)ncoh, st>>>(d_sig, eltype, W.sigfft, n, ncoh, do_if, (float)dstep,
+                                                               dstep);
+            HIP_TRY(hipGetLastError());
+        }
+        if (P->fp31.n)
+            k_full31_signal<512><<<dim3(ncoh, nnc), 512, P->full_lds, st>>>(d_sig, eltype, W.sigfft, P->fp31, do_if,
+                                                                            (float)dstep, dstep);
+        else
+            k_full_signal<512><<<dim3(ncoh, nnc), 512, P->full_lds, st>>>(d_sig, eltype, W.sigfft, P->fp,
+                                                                          P->d_full_tw, do_if, (float)dstep, dstep);
+        HIP_TRY(hipGetLastError());
+    }
+    FullArgs A{P->fp, P->d_full_tw, W.sigfft, P->d_full_code, P->d_full_map, P->d_shifts, nullptr, W.acc, W.rowsum,
+               W.rowbest_v, W.rowbest_k, ncoh, ndop, nnc, 0, P->ap};
+    Full31Args B{P->fp31, W.sigfft, P->d_full_code, (const uint32_t*)P->d_full_map, P->d_shifts, nullptr, W.acc, W.rowsum,
+                 W.rowbest_v, W.rowbest_k, ncoh, ndop, nnc, 0, P->ap};
+    for (int b0 = 0; b0 < nreq; b0 += W.batch) {
+        const int cnt = std::min(W.batch, nreq - b0);
+        A.cnt = B.cnt = cnt;
+        A.req = B.req = W.req + b0;
+        {
+            Timed t(P, FMDBZP_K_COLUMN, st, W.timing);
+            const dim3 g((unsigned)(ndop * cnt));
+            if (P->fp31.n) {
+                switch (P->full_nthr) {
+                case 512: k_full31_corr<512><<<g, 512, P->full_lds, st>>>(B); break;
+                default: k_full31_corr<256><<<g, 256, P->full_lds, st>>>(B); break;
+                }
+            } else if (nnc > 1) {
+                switch (P->full_nthr) {
+                case 1024: k_full_corr<1024, true><<<g, 1024, P->full_lds, st>>>(A); break;
+                case 512: k_full_corr<512, true><<<g, 512, P->full_lds, st>>>(A); break;
+                default: k_full_corr<256, true><<<g, 256, P->full_lds, st>>>(A); break;
+                }
+            } else {
+                switch (P->full_nthr) {
+                case 1024: k_full_corr<1024, false><<<g, 1024, P->full_lds, st>>>(A); break;
+                case 512: k_full_corr<512, false><<<g, 512, P->full_lds, st>>>(A); break;
+                default: k_full_corr<256, false><<<g, 256, P->full_lds, st>>>(A); break;
+                }
+            }
+            HIP_TRY(hipGetLastError());
+        }
+        {
+            Timed t(P, FMDBZP_K_FINALIZE, st, W.timing);
+            k_finalize<<<dim3(cnt), FMDBZP_NTHR, 0, st>>>(W.acc, W.rowsum, W.rowbest_v, W.rowbest_k, ndop, n, n,
+                                                          P->acc_ps, P->ap, 1, 1, 0, d.noise_estimator,
+                                                          d.samples_per_chip, W.stats + b0);
+            HIP_TRY(hipGetLastError());
+        }
+    }
+    return FMDBZP_OK;
+}
+
 // Launch a search's kernels on the plan's stream (lanes joined back into it
 // before returning). Reads the device signal d_sig; writes W.stats.
 int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t eltype, double interm_freq_hz,
@@ -1536,6 +1825,7 @@ int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t elt
     const int spc = d.samples_per_code, spc_eff = d.samples_per_code_eff, nnc = d.num_noncoherent;
     const int64_t seglen = (int64_t)d.num_coh * spc;
     const size_t surf_cols = P->surf_bins > 0 ? (size_t)P->surf_bins : (size_t)spc_eff;
+    if (full_call(P, eltype, store)) return launch_full(P, W, d_sig, eltype, interm_freq_hz, nreq);
 
     // 1. downconvert + double-block FFTs of every segment
     {
@@ -1582,9 +1872,7 @@ int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t elt
     // FP16 tile: scale 2^-e with bs * max|sample| * 2^-e below the FP16 range
     // (every tile value is a sum of bs code-weighted samples of that modulus)
     float hscale = 0.f, hinv = 1.f;
-    const bool int_samples = eltype == FMDBZP_I16 || eltype == FMDBZP_CI8 || eltype == FMDBZP_CI16 ||
-                             eltype == FMDBZP_C2BIT;
-    const bool tile_half = P->tile_half || (P->tile_auto && int_samples);
+    const bool tile_half = P->tile_half || (P->tile_auto && int_samples(eltype));
     if (tile_half) {
         double maxabs = 0.0;
         switch (eltype) {
@@ -1804,6 +2092,7 @@ int autotune(fmdbzp_plan* P)
                 return FMDBZP_OK;
             }
     }
+    if (const int rc = ensure_tile(P)) return rc;
     std::vector<int> variants;
     if (P->corr_variant >= 3) variants.push_back(P->corr_variant);  // compile-time transform
     else {

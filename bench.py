@@ -65,7 +65,8 @@ def copy_calibration(nbytes: int):
 
 KERNEL_CLASS_OF = {"k_corr_tile": "corr_tile", "k_column_simple": "column", "k_column_sign": "column",
                    "k_column_rotation": "column", "k_column_c160": "column", "k_column_c160_pair": "column",
-                   "k_column_rot2000": "column",
+                   "k_column_rot2000": "column", "k_full_corr": "column", "k_full31_corr": "column",
+                   "k_full_fold": "signal_fft", "k_full_signal": "signal_fft", "k_full31_signal": "signal_fft",
                    "k_signal_fft": "signal_fft", "k_reduce_rows": "reduce", "k_reduce_cols": "reduce",
                    "k_merge_rows": "reduce", "k_finalize": "finalize", "k_code_fft": "code_fft",
                    "k_export": "export", "k_export_cm": "export", "k_export_chip": "export",
@@ -562,7 +563,21 @@ def main():
         # written, written only at the first step; mean over the steps
         acc = (8 * ndop * spc_eff * (nnc - 1) + 4 * ndop * spc_eff) / nnc
         bpl = len(prns) * nnc * (8 * ndop * spc + acc) / launches_per_step["column"]
+    full = "corr_tile" not in launches_per_step or not kt["corr_tile"][1]
     roofline = None
+    if full and dom == "column":
+        # full-period correlation: one circular correlation of the code period
+        # per PRN, Doppler row and step (product and inverse transform, 5 n log2 n
+        # + 6 n float operations, power and sum 4 n), bound by the vector unit;
+        # against the FP32 vector rate without packed instructions
+        fl = len(prns) * nnc * ndop * spc * (5 * math.log2(spc) + 10) / launches_per_step["column"]
+        tf = fl / (avg_ms * 1e-3) / 1e12
+        roofline = {"bound": "fp32", "achieved": round(tf, 2), "peak": 78.6, "unit": "TFLOP/s",
+                    "frac": round(tf / 78.6, 4), "traffic": None, "kernel": "full_corr",
+                    "avg_launch_ms": round(avg_ms, 4), "algorithmic_flops_per_launch": int(fl),
+                    "algorithmic_bytes_per_launch": int((8 + 4) * len(prns) * ndop * spc
+                                                        / launches_per_step["column"])}
+        bpl = None
     if bpl:
         ach = bpl / (avg_ms * 1e-3) / 1e9
         config_key = (f"{args.workload}-E{plan.bit_edge_search_steps}-"
@@ -576,7 +591,7 @@ def main():
     # dominant class above can be either); with code-column chunks (ndop above
     # 4000) the per-launch formulas above hold for the dominant class only
     roofline_by_class = {}
-    for k in ("corr_tile", "column"):
+    for k in () if full else ("corr_tile", "column"):
         b = bpl if k == dom else bytes_per_launch.get(k)
         if b and kt.get(k, (0, 0))[1] and not (plan.num_doppler_bins > 4000 and k != dom):
             ms = kt[k][0] / kt[k][1]

@@ -125,6 +125,13 @@ enum fmdbzp_precision {
  * the phase). The Float32 form stays the default, for parity with the
  * reference. No effect at IF = 0. No counterpart in the reference. */
 #define FMDBZP_OPT_FP64_PHASE 0x8
+/* Run every call of a simple-path plan on the coherent tile (block correlation,
+ * then the column stage). By default calls that return statistics only run the
+ * full-period correlation where the plan admits it (one circular correlation
+ * of the code period per Doppler row, no tile); calls with surfaces run on the
+ * tile either way. For measuring the tile kernels. Results agree to FP32
+ * rounding. No counterpart in the reference. */
+#define FMDBZP_OPT_TILE_PATH 0x10
 
 /* fmdbzp_acquire flags */
 #define FMDBZP_FLAG_STORE_SURFACES 0x1u  /* copy (ndop, spc_eff) power surfaces out */
@@ -304,7 +311,8 @@ enum fmdbzp_kernel_class {
     FMDBZP_K_CODE_FFT = 0,    /* plan-time conj code FFTs                 */
     FMDBZP_K_SIGNAL_FFT = 1,  /* downconvert + signal double-block FFTs   */
     FMDBZP_K_CORR_TILE = 2,   /* block correlation: multiply + inverse FFT */
-    FMDBZP_K_COLUMN = 3,      /* column Doppler FFT / sign search + accumulate */
+    FMDBZP_K_COLUMN = 3,      /* column Doppler FFT / sign search + accumulate, or
+                                 the whole full-period correlation of a call   */
     FMDBZP_K_REDUCE = 4,      /* per-row sums and peak candidates          */
     FMDBZP_K_FINALIZE = 5,    /* per-PRN peak, noise, neighbours           */
     FMDBZP_K_EXPORT = 6,      /* surface transpose for store_power_bins    */
@@ -316,8 +324,8 @@ int fmdbzp_plan_set_timing(fmdbzp_plan* plan, int32_t enable);
 int fmdbzp_plan_tuning(fmdbzp_plan* plan, char* buf, size_t buflen);
 /* Graphs captured and replayed by a FMDBZP_OPT_GRAPH plan so far. */
 int fmdbzp_plan_graph_counts(fmdbzp_plan* plan, int64_t* captures, int64_t* replays);
-/* Name of the kernel that runs the plan's column stage (the column Doppler
- * transforms, sign or rotation search and accumulation), e.g.
+/* Name of the kernel that runs the plan's column stage on the coherent tile
+ * (the column Doppler transforms, sign or rotation search and accumulation), e.g.
  * "k_column_rotmma<8,3,20>". No counterpart in the reference (which has one
  * CPU implementation); for tests and reports. */
 int fmdbzp_plan_column_kernel(fmdbzp_plan* plan, char* buf, size_t buflen);
