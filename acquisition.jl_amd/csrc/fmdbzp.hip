@@ -333,6 +333,11 @@ struct fmdbzp_plan {
     bool col_pair = false;
     std::vector<uint8_t> pair_ok;
     size_t col_lds2 = 0;
+    // block correlation on the in-place transforms of full_corr.hpp (corr_variant 10)
+    FullPlanDev fc{};
+    int fc_nthr = 0;
+    size_t fc_lds = 0;
+    float2* d_fc_tw = nullptr;
     // full-period correlation (full_corr.hpp): statistics-only calls of simple
     // plans; the tile, if other calls need it, is allocated by the first of them
     bool full = false;
@@ -365,7 +370,7 @@ struct fmdbzp_plan {
     float4* d_pnbr = nullptr;    // chunk partials: best cell's neighbours
     float4* d_rownbr = nullptr;
     double* d_colsum = nullptr;  // GlobalMean: FP64 sum over rows per effective column
-    int corr_variant = 0;        // k_corr_tile: 6-9 = compile-time F = 400, 800, 2000, 4000,
+    int corr_variant = 0;        // 10 = k_corr_fc; k_corr_tile: 6-9 = compile-time F = 400, 800, 2000, 4000,
                                  // 5 = compile-time F = 500, 4 = compile-time F = 2500,
                                  // 3 = compile-time F = 2048, 2 = two in-place transforms per
                                  // pass, 1 = one, 0 = ping-pong
@@ -403,6 +408,13 @@ namespace {
 int acquire_finish(fmdbzp_plan* P);
 int autotune(fmdbzp_plan* P);
 size_t workspace_budget();
+
+// LDS of the block-correlation variant v.
+size_t corr_lds_of(const fmdbzp_plan* P, int v)
+{
+    if (v == 10) return P->fc_lds;
+    return ((size_t)P->d.fft_size + (size_t)corr_nbuf(v) * fft_lds_span(P->d.fft_size)) * sizeof(float2);
+}
 
 size_t elsize(int eltype)
 {
@@ -584,6 +596,7 @@ void free_plan(fmdbzp_plan* P)
     hipFree(P->d_full_map);
     hipFree(P->d_acc);
     hipFree(P->d_rowsum);
+    hipFree(P->d_fc_tw);
     hipFree(P->d_rowbest_v);
     hipFree(P->d_rowbest_k);
     hipFree(P->d_psum);
@@ -836,7 +849,17 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
     else if (fft_inplace_ok(P->pf) && 2 * F <= FMDBZP_CORR_MAXV * FMDBZP_NTHR) P->corr_variant = 2;
     else if (fft_inplace_ok(P->pf) && F <= FMDBZP_CORR_MAXV * FMDBZP_NTHR) P->corr_variant = 1;
     else P->corr_variant = 0;
-    P->corr_lds = (size_t)F * sizeof(float2) + (size_t)corr_nbuf(P->corr_variant) * fft_lds_span(F) * sizeof(float2);
+    std::vector<float2> fc_tw;
+    if (P->corr_variant < 2) {  // one transform per pass, runtime radices: in place instead, where F factors
+        P->fc_nthr = F > 5120 ? 512 : 256;
+        if (make_full_plan(F, P->fc_nthr, false, &P->fc, &fc_tw)) {
+            P->corr_variant = 10;
+            P->fc_lds = (size_t)fc_lds_span(P->fc) * sizeof(float2);
+            P->pscale = P->inv_f;  // 1/F in the code spectra for every F
+            P->tile_scale = 1.0f;
+        }
+    }
+    P->corr_lds = corr_lds_of(P, P->corr_variant);
 
     // column-stage geometry: LB columns per workgroup, padded column stride
     // (odd, so lanes on consecutive columns spread over the LDS banks)
@@ -1095,6 +1118,19 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
             for (int i = 0; i < nprn; i++) {
                 if (pattern_set[i] < 0 || pattern_set[i] >= P->nsets)
                     return fail(set_err(FMDBZP_EINVAL, "pattern_set[%d] = %d out of range", i, pattern_set[i]));
+    if (P->corr_variant == 10) {
+        if ((rc = dev_alloc(&P->d_fc_tw, fc_tw.size()))) return fail(rc);
+        if (hipMemcpy(P->d_fc_tw, fc_tw.data(), sizeof(float2) * fc_tw.size(), hipMemcpyHostToDevice) != hipSuccess ||
+            (rc = set_lds_attr((const void*)k_fc_code<256>, P->fc_lds)) ||
+            (rc = set_lds_attr((const void*)k_fc_code<512>, P->fc_lds)) ||
+            (rc = set_lds_attr((const void*)k_fc_signal<256>, P->fc_lds)) ||
+            (rc = set_lds_attr((const void*)k_fc_signal<512>, P->fc_lds)) ||
+            (rc = set_lds_attr((const void*)k_corr_fc<256, float2>, P->fc_lds)) ||
+            (rc = set_lds_attr((const void*)k_corr_fc<512, float2>, P->fc_lds)) ||
+            (rc = set_lds_attr((const void*)k_corr_fc<256, __half2>, P->fc_lds)) ||
+            (rc = set_lds_attr((const void*)k_corr_fc<512, __half2>, P->fc_lds)))
+            return fail(rc ? rc : set_err(FMDBZP_EHIP, "transform twiddle upload failed"));
+    }
                 pset[(size_t)i] = pattern_set[i];
             }
         }
@@ -1118,8 +1154,15 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         hipError_t e = hipMemcpy(d_codes, code_samples, (size_t)nprn * spc, hipMemcpyHostToDevice);
         if (e == hipSuccess) {
             Timed t(P, FMDBZP_K_CODE_FFT, P->stream);
-            k_code_fft<<<dim3(nb, nprn), FMDBZP_NTHR, P->fft_lds, P->stream>>>(d_codes, P->d_prnconj, P->pf8,
-                                                                              P->d_twF, spc, nb, bs, P->pscale);
+            if (P->corr_variant != 10)
+                k_code_fft<<<dim3(nb, nprn), FMDBZP_NTHR, P->fft_lds, P->stream>>>(
+                    d_codes, P->d_prnconj, P->pf8, P->d_twF, spc, nb, bs, P->pscale);
+            else if (P->fc_nthr == 512)
+                k_fc_code<512><<<dim3(nb, nprn), 512, P->fc_lds, P->stream>>>(d_codes, P->d_prnconj, P->fc, P->d_fc_tw,
+                                                                             spc, nb, bs, P->pscale);
+            else
+                k_fc_code<256><<<dim3(nb, nprn), 256, P->fc_lds, P->stream>>>(d_codes, P->d_prnconj, P->fc, P->d_fc_tw,
+                                                                             spc, nb, bs, P->pscale);
             e = hipGetLastError();
         }
         if (e == hipSuccess && (rc = full_create(P, d_codes))) {
@@ -1396,7 +1439,13 @@ void launch_corr(fmdbzp_plan* P, dim3 g, hipStream_t st, const float2* sf, const
     const int npass = (nrb + nt - 1) / nt;
     const int wgs = (int)(g.x * g.y);
     g.z = (P->split_wgs <= 0 || wgs >= P->split_wgs) ? 1 : std::min(npass, (P->split_wgs + wgs - 1) / wgs);
-    if (P->corr_variant == 6)
+    if (P->corr_variant == 10 && P->fc_nthr == 512)
+        k_corr_fc<512, TileT><<<g, 512, P->fc_lds, st>>>(sf, P->d_prnconj, req, tile, P->fc, P->d_fc_tw, nb, bs, P->tp,
+                                                         ndop, hscale, rb0, nrb);
+    else if (P->corr_variant == 10)
+        k_corr_fc<256, TileT><<<g, 256, P->fc_lds, st>>>(sf, P->d_prnconj, req, tile, P->fc, P->d_fc_tw, nb, bs, P->tp,
+                                                         ndop, hscale, rb0, nrb);
+    else if (P->corr_variant == 6)
         k_corr_tile<10, true, 400, TileT><<<g, FMDBZP_NTHR, P->corr_lds, st>>>(
             sf, P->d_prnconj, req, tile, P->pf, P->d_twF, nb, bs, P->tp, ndop, P->tile_scale, hscale, rb0, nrb);
     else if (P->corr_variant == 7)
@@ -1835,8 +1884,15 @@ int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t elt
         const double dstep = (-twopi * interm_freq_hz) / d.sampling_freq_hz;
         const float step = (float)dstep;
         Timed t(P, FMDBZP_K_SIGNAL_FFT, P->stream, W.timing);
-        k_signal_fft<<<dim3(ndop, nnc), FMDBZP_NTHR, P->fft_lds, P->stream>>>(
-            d_sig, eltype, W.sigfft, P->pf8, P->d_twF, bs, seglen, ndop, do_if, step, dstep);
+        if (P->corr_variant != 10)
+            k_signal_fft<<<dim3(ndop, nnc), FMDBZP_NTHR, P->fft_lds, P->stream>>>(
+                d_sig, eltype, W.sigfft, P->pf8, P->d_twF, bs, seglen, ndop, do_if, step, dstep);
+        else if (P->fc_nthr == 512)
+            k_fc_signal<512><<<dim3(ndop, nnc), 512, P->fc_lds, P->stream>>>(
+                d_sig, eltype, W.sigfft, P->fc, P->d_fc_tw, bs, seglen, ndop, do_if, step, dstep);
+        else
+            k_fc_signal<256><<<dim3(ndop, nnc), 256, P->fc_lds, P->stream>>>(
+                d_sig, eltype, W.sigfft, P->fc, P->d_fc_tw, bs, seglen, ndop, do_if, step, dstep);
         HIP_TRY(hipGetLastError());
     }
 
@@ -2039,12 +2095,6 @@ int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t elt
     return FMDBZP_OK;
 }
 
-// LDS of the block-correlation variant v.
-size_t corr_lds_of(int v, int F)
-{
-    return (size_t)F * sizeof(float2) + (size_t)corr_nbuf(v) * fft_lds_span(F) * sizeof(float2);
-}
-
 struct TuneKey {
     int F, nb, bs, ndop, batch, ncol_kind, LB;
     bool operator==(const TuneKey& o) const
@@ -2083,7 +2133,7 @@ int autotune(fmdbzp_plan* P)
             if (e.first == key) {
                 P->corr_variant = e.second.corr_variant;
                 P->split_wgs = e.second.split_wgs;
-                P->corr_lds = corr_lds_of(P->corr_variant, F);
+                P->corr_lds = corr_lds_of(P, P->corr_variant);
                 if (col_generic && e.second.LB != P->LB) {
                     P->LB = e.second.LB;
                     P->col_lds = (size_t)P->bstride * (P->col_onebuf ? 1 : 2) * sizeof(float2) * P->LB;
@@ -2102,7 +2152,7 @@ int autotune(fmdbzp_plan* P)
     }
     int rc;
     for (int v : variants) {
-        const size_t lds = corr_lds_of(v, F);
+        const size_t lds = corr_lds_of(P, v);
         if (lds > kLdsMax) continue;
         if ((rc = set_lds_attr((const void*)k_corr_tile<2, true>, lds)) ||
             (rc = set_lds_attr((const void*)k_corr_tile<1, true>, lds)) ||
@@ -2147,11 +2197,11 @@ int autotune(fmdbzp_plan* P)
     int best_v = P->corr_variant, best_split = P->split_wgs;
     float best_ms = 1e30f;
     for (int v : variants) {
-        if (corr_lds_of(v, F) > kLdsMax) continue;
+        if (corr_lds_of(P, v) > kLdsMax) continue;
         for (int split : {0, 2048, 4096}) {
             P->corr_variant = v;
             P->split_wgs = split;
-            P->corr_lds = corr_lds_of(v, F);
+            P->corr_lds = corr_lds_of(P, v);
             const float ms = time_it([&]() {
                 launch_corr(P, dim3(ndop, cnt), st, P->d_sigfft, d_req, P->d_tile, nb, bs, ndop, 0.f, 0, nb);
             });
@@ -2166,7 +2216,7 @@ int autotune(fmdbzp_plan* P)
     }
     P->corr_variant = best_v;
     P->split_wgs = best_split;
-    P->corr_lds = corr_lds_of(best_v, F);
+    P->corr_lds = corr_lds_of(P, best_v);
     int best_lb = P->LB;
     if (col_generic) {
         // columns per workgroup of k_column_simple: the plan's choice and

@@ -465,6 +465,64 @@ k_full_signal(const void* __restrict__ sig, int eltype, float2* z, FullPlanDev f
 // in registers between the steps and are written once; the row's FP64 sum and
 // best cell come from the same registers.
 // ---------------------------------------------------------------------------
+// The product of two spectra and all but the last stage of its inverse
+// transform, ending with a barrier. WIDE: the radices of FC_RADIX_SWITCH_FIRST
+// and FC_RADIX_SWITCH_MID.
+template <int NTHR, bool WIDE>
+__device__ __forceinline__ void fc_inverse_head(float2* lds, const FullPlanDev& f, const float2* __restrict__ tw, int tid,
+                                                const float2* __restrict__ Z, const float2* __restrict__ G)
+{
+    {
+        const int m0 = f.n / f.radix[0], p1 = f.radix[0] + (f.pad_shift < 31 ? 1 : 0);
+        auto op = [&](auto rc) {
+            constexpr int R = decltype(rc)::value;
+            for (int j = fc_opaque(tid); j < m0; j += NTHR) {
+                float2 v[R], gv[R];
+                fc_ld_run(gv, G, j, m0);
+                fc_ld_run(v, Z, j, m0);
+                fc_issued();
+#pragma unroll
+                for (int r = 0; r < R; r++) v[r] = cmulf(v[r], gv[r]);
+                float2* dst = lds + j * p1;
+                dft_reg<R, true>(v);
+#pragma unroll
+                for (int r = 0; r < R; r++) dst[r] = v[r];
+            }
+        };
+        if constexpr (WIDE) {
+            FC_RADIX_SWITCH_FIRST(f.radix[0], op)
+        } else {
+            FC_RADIX_SWITCH(f.radix[0], op)
+        }
+    }
+    __syncthreads();
+    for (int t = 1; t + 1 < f.nst; t++) {
+        const float2* twt = tw + f.twoff[t];
+        const int ns = f.ns[t];
+        auto op = [&](auto rc) {
+            constexpr int R = decltype(rc)::value;
+            fc_butterflies<R, NTHR>(f, t, fc_opaque(tid), [&](int a, int pn, int k) {
+                float2 v[R], tv[R - 1];
+                fc_ld_run(tv, twt, k, ns);
+#pragma unroll
+                for (int r = 0; r < R; r++) v[r] = lds[a + r * pn];
+                fc_issued();
+#pragma unroll
+                for (int r = 1; r < R; r++) v[r] = cmulf(v[r], make_float2(tv[r - 1].x, -tv[r - 1].y));
+                dft_reg<R, true>(v);
+#pragma unroll
+                for (int r = 0; r < R; r++) lds[a + r * pn] = v[r];
+            });
+        };
+        if constexpr (WIDE) {
+            FC_RADIX_SWITCH_MID(f.radix[t], op)
+        } else {
+            FC_RADIX_SWITCH(f.radix[t], op)
+        }
+        __syncthreads();
+    }
+}
+
 // Row sum and best cell over the workgroup's threads (the lowest column on
 // ties: the visit order within a row). The LDS buffer is free.
 template <int NTHR>
@@ -558,6 +616,7 @@ struct FullArgs {
     int ncoh, ndop, nnc, cnt, ap;
 };
 
+// MULTI: several noncoherent steps.
 template <int NTHR, bool MULTI>
 __global__ void __launch_bounds__(NTHR)
 __attribute__((amdgpu_waves_per_eu(4))) k_full_corr(FullArgs A)
@@ -583,53 +642,7 @@ __attribute__((amdgpu_waves_per_eu(4))) k_full_corr(FullArgs A)
     for (int i = 0; i < (MULTI ? FC_CELLS : 1); i++) acc[i] = 0.f;
     for (int step = 0; step < A.nnc; step++) {
         const float2* Z = A.spec + ((size_t)step * A.ncoh + s) * n;
-        {
-            const int m0 = n / f.radix[0], p1 = f.radix[0] + (f.pad_shift < 31 ? 1 : 0);
-            auto op = [&](auto rc) {
-                constexpr int R = decltype(rc)::value;
-                for (int j = fc_opaque(tid); j < m0; j += NTHR) {
-                    float2 v[R], gv[R];
-                    fc_ld_run(gv, G, j, m0);
-                    fc_ld_run(v, Z, j, m0);
-                    fc_issued();
-#pragma unroll
-                    for (int r = 0; r < R; r++) v[r] = cmulf(v[r], gv[r]);
-                    float2* dst = lds + j * p1;
-                    dft_out<R, true>(v, [&](auto r, float2 x) { dst[r] = x; });
-                }
-            };
-            if constexpr (MULTI) {
-                FC_RADIX_SWITCH(f.radix[0], op)
-            } else {
-                FC_RADIX_SWITCH_FIRST(f.radix[0], op)
-            }
-        }
-        __syncthreads();
-        for (int t = 1; t + 1 < f.nst; t++) {
-            const float2* twt = A.tw + f.twoff[t];
-            const int ns = f.ns[t];
-            auto op = [&](auto rc) {
-                constexpr int R = decltype(rc)::value;
-                fc_butterflies<R, NTHR>(f, t, fc_opaque(tid), [&](int a, int pn, int k) {
-                    float2 v[R], tv[R - 1];
-                    fc_ld_run(tv, twt, k, ns);
-#pragma unroll
-                    for (int r = 0; r < R; r++) v[r] = lds[a + r * pn];
-                    fc_issued();
-#pragma unroll
-                    for (int r = 1; r < R; r++) v[r] = cmulf(v[r], make_float2(tv[r - 1].x, -tv[r - 1].y));
-                    dft_reg<R, true>(v);
-#pragma unroll
-                    for (int r = 0; r < R; r++) lds[a + r * pn] = v[r];
-                });
-            };
-            if constexpr (MULTI) {
-                FC_RADIX_SWITCH(f.radix[t], op)
-            } else {
-                FC_RADIX_SWITCH_MID(f.radix[t], op)
-            }
-            __syncthreads();
-        }
+        fc_inverse_head<NTHR, !MULTI>(lds, f, A.tw, tid, Z, G);
         const uint32_t shift = (uint32_t)A.shifts[(size_t)step * A.ndop + row];
         {
             const int t = f.nst - 1, ns = f.ns[t];
@@ -704,6 +717,90 @@ __attribute__((amdgpu_waves_per_eu(4))) k_full_corr(FullArgs A)
     }
     if constexpr (MULTI) fc_store_cells<NTHR, FC_CELLS>(acc, accp, n, sum, bv, bc);
     full_row_reduce<NTHR>(lds, sum, bv, bc, A.rowsum, A.rowbest_v, A.rowbest_k, (size_t)p * A.ndop, row, A.ndop);
+}
+
+// ---------------------------------------------------------------------------
+// The tile's block correlation (k_corr_tile: row k of column block r is signal
+// double block k times code sub-block (k mod nb + r) mod nb, lags < bs) on the
+// same in-place transforms, for the sizes that k_corr_tile runs with one
+// transform per pass and runtime radices: more than 2048 points, or a radix
+// above 5 in a middle stage, where it computes each output of a prime radix by
+// its own sum. F 5600 (L5-like 30.69 MHz, 110 rows, 11 blocks, 6 PRNs) took
+// 1.89 ms per launch there. grid (ndop, batch, split)
+// ---------------------------------------------------------------------------
+template <int NTHR, class TileT>
+__global__ void __launch_bounds__(NTHR)
+__attribute__((amdgpu_waves_per_eu(4)))
+k_corr_fc(const float2* __restrict__ sigfft_step, const float2* __restrict__ prnconj, const int32_t* __restrict__ req,
+          TileT* __restrict__ tile, FullPlanDev f, const float2* __restrict__ tw, int nb, int bs, int tp, int ndop,
+          float hscale, int rb0, int nrb)
+{
+    extern __shared__ float2 lds[];
+    const int tid = threadIdx.x;
+    const int lbk = xcd_logical_block();
+    const int k = __builtin_amdgcn_readfirstlane(lbk % gridDim.x);
+    const int rest = __builtin_amdgcn_readfirstlane(lbk / gridDim.x);
+    const int p = rest % gridDim.y, sp = rest / gridDim.y;
+    const int chunk = (nrb + gridDim.z - 1) / gridDim.z;
+    const int r_end = min(nrb, (sp + 1) * chunk);
+    const float2* S = sigfft_step + (size_t)k * f.n;
+    const float2* Pp = prnconj + (size_t)req[p] * nb * f.n;
+    for (int rr = sp * chunk; rr < r_end; rr++) {
+        const int b = (k % nb + rb0 + rr) % nb;
+        fc_inverse_head<NTHR, true>(lds, f, tw, tid, S, Pp + (size_t)b * f.n);
+        const LagOut<TileT, false> out{tile + (((size_t)p * nrb + rr) * ndop + k) * tp, 0, bs, 1.0f, 1, hscale};
+        const int t = f.nst - 1, ns = f.ns[t];
+        const float2* twt = tw + f.twoff[t];
+        const int pn = ns + (ns >> f.pad_shift);
+        auto op = [&](auto rc) {
+            constexpr int R = decltype(rc)::value;
+            for (int j = fc_opaque(tid); j < ns; j += NTHR) {
+                float2 v[R], tv[R - 1];
+                fc_ld_run(tv, twt, j, ns);
+                const float2* src = lds + fc_addr(j, f.pad_shift);
+#pragma unroll
+                for (int r = 0; r < R; r++) v[r] = src[r * pn];
+                fc_issued();
+#pragma unroll
+                for (int r = 1; r < R; r++) v[r] = cmulf(v[r], make_float2(tv[r - 1].x, -tv[r - 1].y));
+                dft_reg<R, true>(v);
+                // lags below bs <= F / 2: outputs r <= R / 2
+#pragma unroll
+                for (int r = 0; r <= R / 2; r++) out(0, j + r * ns, v[r]);
+            }
+        };
+        FC_RADIX_SWITCH(f.radix[t], op)
+        __syncthreads();
+    }
+}
+
+// Spectra for k_corr_fc: signal double blocks (grid (ndop, nnc)) and conj code
+// sub-blocks times 1 / F (grid (nb, nprn)).
+template <int NTHR>
+__global__ void __launch_bounds__(NTHR)
+k_fc_signal(const void* __restrict__ sig, int eltype, float2* __restrict__ sigfft, FullPlanDev f,
+            const float2* __restrict__ tw, int bs, int64_t seglen, int ndop, int do_if, float phase_step,
+            double phase_step64)
+{
+    extern __shared__ float2 lds[];
+    const int64_t seg0 = (int64_t)blockIdx.y * seglen;
+    const DownconvIn in{sig, eltype, seg0, seglen, (int64_t)blockIdx.x * bs, 2 * bs, do_if,
+                        __fmul_rn((float)seg0, phase_step), phase_step, phase_step64};
+    float2* out = sigfft + ((size_t)blockIdx.y * ndop + blockIdx.x) * f.n;
+    fc_forward<NTHR>(
+        lds, f, tw, threadIdx.x, [&](int i) { return in(0, i); }, [&](int i, float2 x) { out[i] = x; });
+}
+template <int NTHR>
+__global__ void __launch_bounds__(NTHR)
+k_fc_code(const int8_t* __restrict__ codes, float2* __restrict__ prnconj, FullPlanDev f, const float2* __restrict__ tw,
+          int spc, int nb, int bs, float scale)
+{
+    extern __shared__ float2 lds[];
+    const CodeIn in{codes + (size_t)blockIdx.y * spc + (size_t)blockIdx.x * bs, bs};
+    float2* out = prnconj + ((size_t)blockIdx.y * nb + blockIdx.x) * f.n;
+    fc_forward<NTHR>(
+        lds, f, tw, threadIdx.x, [&](int i) { return in(0, i); },
+        [&](int i, float2 x) { out[i] = make_float2(x.x * scale, -x.y * scale); });
 }
 
 // ---------------------------------------------------------------------------
