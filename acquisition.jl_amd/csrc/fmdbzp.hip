@@ -351,6 +351,10 @@ struct fmdbzp_plan {
     bool tile_half = false;      // FMDBZP_PREC_TILE_FP16: FP16 coherent tile
     bool tile_auto = false;      // FMDBZP_PREC_AUTO on a plan that admits the FP16 tile: per call, by sample type
     bool rot_direct = false;     // rotation kernel writes transform outputs straight to the accumulator
+    int rotsplit = 0;            // direct rotation, few Doppler rows: columns per workgroup of k_column_rotsplit
+    // accumulator layout and size that fmdbzp_acquire_noalloc's limit counts
+    bool lim_cm = false;
+    size_t lim_acc_ps = 0;
     bool rot2000 = false;        // direct rotation at ndop 2000: compile-time kernel, one column per workgroup
     // Direct rotation at large ndop (k_column_rotbig), accumulated in code-column
     // chunks: every chunk owns chunk_cols scrambled code columns (the last one
@@ -405,16 +409,16 @@ struct fmdbzp_plan {
 
 namespace {
 
-int acquire_finish(fmdbzp_plan* P);
-int autotune(fmdbzp_plan* P);
-size_t workspace_budget();
-
 // LDS of the block-correlation variant v.
 size_t corr_lds_of(const fmdbzp_plan* P, int v)
 {
     if (v == 10) return P->fc_lds;
     return ((size_t)P->d.fft_size + (size_t)corr_nbuf(v) * fft_lds_span(P->d.fft_size)) * sizeof(float2);
 }
+
+int acquire_finish(fmdbzp_plan* P);
+int autotune(fmdbzp_plan* P);
+size_t workspace_budget();
 
 size_t elsize(int eltype)
 {
@@ -592,11 +596,11 @@ void free_plan(fmdbzp_plan* P)
     hipFree(P->d_tile);
     hipFree(P->d_tile2);
     hipFree(P->d_full_tw);
+    hipFree(P->d_fc_tw);
     hipFree(P->d_full_code);
     hipFree(P->d_full_map);
     hipFree(P->d_acc);
     hipFree(P->d_rowsum);
-    hipFree(P->d_fc_tw);
     hipFree(P->d_rowbest_v);
     hipFree(P->d_rowbest_k);
     hipFree(P->d_psum);
@@ -967,6 +971,20 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
             LB = P->LB = 1;
         }
     }
+    P->lim_cm = P->acc_cm;
+    // direct rotation of 10 or 20 coherent periods and a row length with an
+    // in-register transform (the L5-like searches up to +-10 kHz): 32 columns
+    // per workgroup where both roles fit its threads, else 16
+    if (P->rot_direct && !P->rot2000 && !P->rotbig && d.num_secondary_rotations <= 64 &&
+        (size_t)ndop * P->ap * sizeof(float) < (1ull << 32)) {
+#define RS_OK(PP, NN) if (d.num_coh == PP && nb == NN) P->rotsplit = 32 * std::max(PP, NN) <= ROTSPLIT_NTHR ? 32 : 16;
+        ROTSPLIT_ALL(RS_OK)
+#undef RS_OK
+        if (P->rotsplit) {
+            P->acc_cm = false;
+            LB = P->LB = P->rotsplit;
+        }
+    }
     // the matrix-core form of the same search (nb = 25 n1, n1 = 2, 4, 10, 20);
     // FMDBZP_PREC_AUTO takes it where it is the faster kernel (n1 = 10, 20:
     // at n1 = 2 and 4 the FP32 kernel's transforms are short and both run at
@@ -981,6 +999,7 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
                                            "and ndop = 625 n1, n1 in {2, 4, 10, 20}"));
     P->apc = (ndop + 31) & ~31;
     P->acc_ps = P->acc_cm ? (size_t)spc_eff * P->apc : (size_t)ndop * P->ap;
+    P->lim_acc_ps = P->lim_cm ? (size_t)spc_eff * P->apc : (size_t)ndop * P->ap;
     if (P->rotbig) {
         const int R = d.num_secondary_rotations;
         int span = 0;
@@ -1028,6 +1047,7 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
     }
     P->col_lds = per_col * LB + fixed;
     if (P->col_static) P->col_lds = (size_t)LB * P->bstride * sizeof(float2);  // one column buffer
+    if (P->rotsplit) P->col_lds = (size_t)d.num_coh * rotsplit_pitch(nb, P->rotsplit) * sizeof(float2);
     if (P->rot2000)
         P->col_lds = (size_t)(2000 + 2 * fft_lds_span(2000)) * sizeof(float2) +
                      ((size_t)d.num_secondary_rotations * 4 + 7) / 8 * 8;
@@ -1098,6 +1118,19 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
             hipMemcpy(P->d_twD, twD.data(), sizeof(float2) * ndop, hipMemcpyHostToDevice) != hipSuccess)
             return fail(set_err(FMDBZP_EHIP, "twiddle upload failed"));
     }
+    if (P->corr_variant == 10) {
+        if ((rc = dev_alloc(&P->d_fc_tw, fc_tw.size()))) return fail(rc);
+        if (hipMemcpy(P->d_fc_tw, fc_tw.data(), sizeof(float2) * fc_tw.size(), hipMemcpyHostToDevice) != hipSuccess ||
+            (rc = set_lds_attr((const void*)k_fc_code<256>, P->fc_lds)) ||
+            (rc = set_lds_attr((const void*)k_fc_code<512>, P->fc_lds)) ||
+            (rc = set_lds_attr((const void*)k_fc_signal<256>, P->fc_lds)) ||
+            (rc = set_lds_attr((const void*)k_fc_signal<512>, P->fc_lds)) ||
+            (rc = set_lds_attr((const void*)k_corr_fc<256, float2>, P->fc_lds)) ||
+            (rc = set_lds_attr((const void*)k_corr_fc<512, float2>, P->fc_lds)) ||
+            (rc = set_lds_attr((const void*)k_corr_fc<256, __half2>, P->fc_lds)) ||
+            (rc = set_lds_attr((const void*)k_corr_fc<512, __half2>, P->fc_lds)))
+            return fail(rc ? rc : set_err(FMDBZP_EHIP, "transform twiddle upload failed"));
+    }
     if (P->rotbig) {
         std::vector<float2> twR = twiddles(nb);
         if ((rc = dev_alloc(&P->d_twR, (size_t)nb))) return fail(rc);
@@ -1118,19 +1151,6 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
             for (int i = 0; i < nprn; i++) {
                 if (pattern_set[i] < 0 || pattern_set[i] >= P->nsets)
                     return fail(set_err(FMDBZP_EINVAL, "pattern_set[%d] = %d out of range", i, pattern_set[i]));
-    if (P->corr_variant == 10) {
-        if ((rc = dev_alloc(&P->d_fc_tw, fc_tw.size()))) return fail(rc);
-        if (hipMemcpy(P->d_fc_tw, fc_tw.data(), sizeof(float2) * fc_tw.size(), hipMemcpyHostToDevice) != hipSuccess ||
-            (rc = set_lds_attr((const void*)k_fc_code<256>, P->fc_lds)) ||
-            (rc = set_lds_attr((const void*)k_fc_code<512>, P->fc_lds)) ||
-            (rc = set_lds_attr((const void*)k_fc_signal<256>, P->fc_lds)) ||
-            (rc = set_lds_attr((const void*)k_fc_signal<512>, P->fc_lds)) ||
-            (rc = set_lds_attr((const void*)k_corr_fc<256, float2>, P->fc_lds)) ||
-            (rc = set_lds_attr((const void*)k_corr_fc<512, float2>, P->fc_lds)) ||
-            (rc = set_lds_attr((const void*)k_corr_fc<256, __half2>, P->fc_lds)) ||
-            (rc = set_lds_attr((const void*)k_corr_fc<512, __half2>, P->fc_lds)))
-            return fail(rc ? rc : set_err(FMDBZP_EHIP, "transform twiddle upload failed"));
-    }
                 pset[(size_t)i] = pattern_set[i];
             }
         }
@@ -1394,6 +1414,7 @@ int fmdbzp_plan_column_kernel(fmdbzp_plan* plan, char* buf, size_t buflen)
     if (P->rotmma) name = rotmma[P->rotmma == 2 ? 0 : P->rotmma == 4 ? 1 : P->rotmma == 10 ? 2 : 3];
     else if (P->rotbig) snprintf(tmp, sizeof tmp, "k_column_rotbig<%d,25>", P->rotbig_nt);
     else if (P->rot2000) name = "k_column_rot2000";
+    else if (P->rotsplit) snprintf(tmp, sizeof tmp, "k_column_rotsplit<%d,%d>", P->d.num_coh, P->d.num_blocks);
     else if (P->col_pair) name = P->tile_half ? "k_column_c160_pair<32,512,fp16>" : "k_column_c160_pair<32,512>";
     else if (P->col_static) name = P->tile_half ? "k_column_c160<32,512,fp16>" : "k_column_c160<32,512>";
     else if (P->simple_kernel) name = P->col_onebuf ? "k_column_simple<onebuf>" : "k_column_simple";
@@ -2019,6 +2040,18 @@ int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t elt
                         k_column_sign<<<g, FMDBZP_NTHR, P->col_lds, st>>>(A);
                     } else if (P->rot2000) {
                         k_column_rot2000<512><<<dim3(bs, nb, cnt), 512, P->col_lds, st>>>(A);
+                    } else if (P->rotsplit) {
+                        const int C = P->rotsplit;
+                        const int nt = (C * std::max(d.num_coh, nb) + 63) & ~63;
+                        bool done = false;
+#define RS_LAUNCH(PP, NN)                                                          \
+    if (d.num_coh == PP && nb == NN) {                                             \
+        k_column_rotsplit<PP, NN><<<g, nt, P->col_lds, st>>>(A, C);                \
+        done = true;                                                               \
+    }
+                        ROTSPLIT_ALL(RS_LAUNCH)
+#undef RS_LAUNCH
+                        if (!done) return set_err(FMDBZP_EINVAL, "no rotation kernel for %d x %d", d.num_coh, nb);
                     } else {
                         k_column_rotation<<<g, FMDBZP_NTHR, P->col_lds, st>>>(A);
                     }
@@ -2412,10 +2445,10 @@ extern "C" int fmdbzp_acquire_noalloc(fmdbzp_plan* plan, const void* signal, int
     const size_t b_req = align256(sizeof(int32_t) * (size_t)nreq);
     const size_t b_stats = align256(sizeof(fmdbzp_prn_stats) * (size_t)nreq);
     const size_t t_prn = align256(sizeof(float2) * (size_t)d.num_blocks * ndop * P->tp);
-    const size_t a_prn = align256(sizeof(float) * P->acc_ps);
+    const size_t a_prn = align256(sizeof(float) * std::max(P->acc_ps, P->lim_acc_ps));
     // the size limit counts a reduction partial per row and 4096 columns beside
     // the tile (they are kept in the tile)
-    const size_t np = P->acc_cm ? (size_t)((d.samples_per_code_eff + 4095) / 4096) * ndop : 0;
+    const size_t np = P->lim_cm ? (size_t)((d.samples_per_code_eff + 4095) / 4096) * ndop : 0;
     const size_t r_prn = align256(sizeof(double) * ndop) + align256(sizeof(float) * ndop) +
                          align256(sizeof(uint64_t) * ndop) + align256(sizeof(double) * np) +
                          align256(sizeof(float) * np) + align256(sizeof(uint64_t) * np);
