@@ -355,6 +355,7 @@ struct fmdbzp_plan {
     // accumulator layout and size that fmdbzp_acquire_noalloc's limit counts
     bool lim_cm = false;
     size_t lim_acc_ps = 0;
+    bool rot25x80 = false;       // ... with 25 periods of 80 rows: k_column_rot25x80
     bool rot2000 = false;        // direct rotation at ndop 2000: compile-time kernel, one column per workgroup
     // Direct rotation at large ndop (k_column_rotbig), accumulated in code-column
     // chunks: every chunk owns chunk_cols scrambled code columns (the last one
@@ -944,6 +945,10 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
     P->rot2000 = P->rot_direct && ndop == 2000 && d.num_coh <= 32 && !(r2k && atoi(r2k) == 0) &&
                  (size_t)spc * ((ndop + 31) & ~31) * sizeof(float) < (1ull << 32);
     if (P->rot2000) {
+        // 25 periods of 80 rows, the E1-like search: 10.5 ms per PRN-step at 25 MHz
+        // against 15.1 ms of the 16 x 5 x 5 x 5 kernel, which serves other N_coh
+        // (the masks of a workgroup hold at most 64 rotations)
+        P->rot25x80 = d.num_coh == 25 && d.num_secondary_rotations <= 64;
         P->acc_cm = true;
         LB = P->LB = 1;
     }
@@ -1051,6 +1056,7 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
     if (P->rot2000)
         P->col_lds = (size_t)(2000 + 2 * fft_lds_span(2000)) * sizeof(float2) +
                      ((size_t)d.num_secondary_rotations * 4 + 7) / 8 * 8;
+    if (P->rot25x80) P->col_lds = kRot2000Lds;
     if (P->rotbig)
         P->col_lds = (size_t)(25 * fft_lds_span(nb) + nb) * sizeof(float2) +
                      ((size_t)ndop + d.num_secondary_rotations) * sizeof(uint32_t);
@@ -1094,6 +1100,7 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         (rc = set_lds_attr((const void*)k_column_sign, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rotation, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rot2000<512>, P->col_lds)) ||
+        (rc = set_lds_attr((const void*)k_column_rot25x80, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rotbig<64, 25>, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rotbig<128, 25>, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rotbig<256, 25>, P->col_lds)) ||
@@ -2038,6 +2045,8 @@ int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t elt
                             k_column_simple<false><<<g, FMDBZP_COL_NTHR, P->col_lds, st>>>(A);
                     } else if (d.path == FMDBZP_PATH_SIGN) {
                         k_column_sign<<<g, FMDBZP_NTHR, P->col_lds, st>>>(A);
+                    } else if (P->rot25x80) {
+                        k_column_rot25x80<<<dim3((bs + ROT2000_C - 1) / ROT2000_C, nb, cnt), ROT2000_NTHR, P->col_lds, st>>>(A);
                     } else if (P->rot2000) {
                         k_column_rot2000<512><<<dim3(bs, nb, cnt), 512, P->col_lds, st>>>(A);
                     } else if (P->rotsplit) {

@@ -1177,6 +1177,231 @@ k_column_rot2000(ColumnArgs A)
     }
 }
 
+// W_25^k = exp(-2 pi i k / 25), k = 0..16 (the in-register 5 x 5 DFT's twiddles)
+__constant__ float2 kW25[17] = {
+    {1.0f, -0.0f}, {0.9685831611286311f, -0.2486898871648548f}, {0.8763066800438636f, -0.4817536741017153f},
+    {0.7289686274214116f, -0.6845471059286886f}, {0.5358267949789965f, -0.8443279255020151f},
+    {0.30901699437494745f, -0.9510565162951535f}, {0.06279051952931353f, -0.9980267284282716f},
+    {-0.1873813145857246f, -0.9822872507286887f}, {-0.4257792915650727f, -0.9048270524660195f},
+    {-0.6374239897486897f, -0.7705132427757893f}, {-0.8090169943749473f, -0.5877852522924732f},
+    {-0.9297764858882513f, -0.36812455268467814f}, {-0.9921147013144778f, -0.12533323356430454f},
+    {-0.9921147013144779f, 0.12533323356430429f}, {-0.9297764858882515f, 0.3681245526846779f},
+    {-0.8090169943749478f, 0.5877852522924727f}, {-0.6374239897486895f, 0.7705132427757894f}};
+
+// Direct rotation path at ndop = 2000 = 25 nb, nb = 80 (the E1-like search at
+// 25 MHz and the default +-7 kHz): rows n = p nb + m, raw bins w = s + 25 k, as
+// k_column_rotbig below,
+//   X_q[s + 25 k] = sum_m W_80^(k m) W_2000^(s m) sum_p sigma_q[p] W_25^(s p) x[p nb + m].
+// A workgroup owns C = 3 code columns. Thread (column, m) keeps the 25 samples
+// of its lag in registers for all rotations; per rotation it applies the
+// signs (flips of the float sign bit), a 5 x 5 DFT over p and the twiddles,
+// and writes the 25 classes s to LDS. The 80-point transforms of the 3 x 25
+// rows follow as 8 x 10 in place, and the last stage adds the powers to the
+// cells straight from its registers: butterfly (s, i) of a column has rows
+// s + 25 i + 200 k2, so consecutive threads hold consecutive rows of the
+// column-major accumulator. Offsets of the cells stay in registers, and their
+// previous values are read ahead of the rotation's first stage.
+// grid (ceil(bs / 3), nb, batch), 256 threads, 49 KB of LDS.
+// Bound by vector instructions: 2130 per column and rotation against 2600 of
+// the 16 x 5 x 5 x 5 kernel above, 8.5 ms at 100000 columns and R 25 if
+// nothing waited, next to 41.9 GB of cells (8.5 ms at a copy's rate). Three
+// columns make four waves, one per SIMD, and two workgroups per CU leave the
+// 231 registers for all 30 offsets and values: four columns in five waves, two
+// and a half per SIMD with one butterfly's cells ahead, took 14.4 ms
+// and k_column_rot2000 15.1 ms; this takes 10.5 ms per PRN-step.
+#define ROT2000_C 3
+#define ROT2000_NTHR 256
+constexpr int kRot2000Pitch = 81;                 // row of 80 values (odd: lanes along rows spread over the banks)
+constexpr int kRot2000Col = 25 * kRot2000Pitch + 2;  // column: 11 mod 32, so three columns' lanes spread too
+constexpr size_t kRot2000Lds = (size_t)ROT2000_C * kRot2000Col * 8 + 80 * 8;
+
+__global__ void __launch_bounds__(ROT2000_NTHR)
+__attribute__((amdgpu_waves_per_eu(2, 2)))
+k_column_rot25x80(ColumnArgs A)
+{
+    constexpr int N = 2000, NB = 80, P = 25, RA = 8, RB = 10, C = ROT2000_C, NT = ROT2000_NTHR;
+    constexpr int RP = kRot2000Pitch, CP = kRot2000Col;
+    constexpr int ITA = (C * P * RB + NT - 1) / NT, ITB = (C * P * RA + NT - 1) / NT;
+    static_assert(C * NB <= NT && RP >= NB, "work split");
+    extern __shared__ float2 lds[];
+    float2* stw = lds + C * CP;                // W_80^(i j) at [j][i], i < 8, j < 10
+    __shared__ uint32_t smask[64];
+    const int tid = threadIdx.x;
+    const int lbk = xcd_logical_block();
+    const int lb = __builtin_amdgcn_readfirstlane(lbk % gridDim.x);
+    const int r = __builtin_amdgcn_readfirstlane((lbk / gridDim.x) % gridDim.y);
+    const int p = __builtin_amdgcn_readfirstlane(lbk / (gridDim.x * gridDim.y));
+    const int lag0 = lb * C, ncol = min(C, A.bs - lag0);
+    if (tid < NB) stw[tid] = A.twD[P * (tid % RA) * (tid / RA)];
+    if (tid < A.R) {
+        const float* pat = A.patterns + ((size_t)A.pset[A.req[p]] * A.Q + tid) * A.ncoh;
+        uint32_t msk = 0;
+        for (int q = 0; q < P; q++)
+            if (pat[q] < 0.f) msk |= 1u << q;
+        smask[tid] = msk;
+    }
+    // lag m of column c: 25 samples of the column rotated by its alignment
+    // (src/noncoherent_integration.jl:212-215), factors of W_N^(s m), s = s1 + 5 s2
+    const int c1 = tid % C, m = min(tid / C, NB - 1);
+    float2 x[P], tw1[5], tw5[5];
+    {
+        const int lag = lag0 + min(c1, ncol - 1), pc = r * A.bs + lag;
+        const int wrap = ((NB - pc / A.bs) % NB) * A.bs + (pc % A.bs);
+        const int eff = ((wrap + (A.bs >> 1)) / A.bs) % NB;
+        const float2* T = A.tile + (((size_t)p * NB + r) * N) * A.tp + lag;
+#pragma unroll
+        for (int q = 0; q < P; q++) {
+            int src = q * NB + m + eff;
+            if (src >= N) src -= N;
+            // neighbouring workgroups (the next lags) read the same tile lines: plain, cached loads
+            x[q] = T[(size_t)src * A.tp];
+        }
+#pragma unroll
+        for (int i = 1; i < 5; i++) {
+            tw1[i] = A.twD[i * m];
+            tw5[i] = A.twD[5 * i * m];
+        }
+    }
+    float* accp = A.acc + (size_t)p * A.acc_ps;
+    const size_t slice = (size_t)A.spc * A.acc_ldc * 4;  // bytes of a rotation slice (below 2^32)
+    const bool first = A.first_step != 0;
+    // The stages' butterflies (their index arithmetic is full of slow
+    // multiplications). Radix 8: LDS index | j << 16, all ones past the end.
+    // Radix 10: LDS index and the byte offsets of the cells in a slice; it takes
+    // the threads in reverse, so that the remainders of the two stages fall to
+    // different waves.
+    uint32_t pa[ITA], pb[ITB], off[ITB][RB];
+#pragma unroll
+    for (int it = 0; it < ITA; it++) {
+        const uint32_t idx = tid + it * NT, c = idx / (P * RB), b = idx % (P * RB), j = b / P, s = b % P;
+        pa[it] = idx < C * P * RB ? (c * CP + s * RP + j) | j << 16 : 0xffffffffu;
+    }
+#pragma unroll
+    for (int it = 0; it < ITB; it++) {
+        const uint32_t idx = NT - 1 - tid + it * NT, c = idx / (P * RA), b = idx % (P * RA), i = b / P, s = b % P;
+        const bool act = idx < C * P * RA && c < (uint32_t)ncol;
+        pb[it] = act ? c * CP + s * RP + RB * i : 0xffffffffu;
+#pragma unroll
+        for (int k2 = 0; k2 < RB; k2++) {
+            // raw bin b + 200 k2, sorted row (b + 200 k2 + 1000) mod 2000, column + its drift (mod spc)
+            const int row = b + P * RA * ((k2 + RB / 2) % RB);
+            int dc = r * A.bs + lag0 + (act ? (int)c : 0) + A.shifts[row];
+            if (dc >= A.spc) dc -= A.spc;
+            off[it][k2] = ((uint32_t)row + (uint32_t)dc * (uint32_t)A.acc_ldc) * 4u;
+        }
+    }
+    __syncthreads();  // tables and masks
+#pragma unroll 1
+    for (int q = 0; q < A.R; q++) {
+        // opaque copies: what follows from them is not hoisted into registers
+        uint32_t ia[ITA], ib[ITB];
+#pragma unroll
+        for (int it = 0; it < ITA; it++) {
+            ia[it] = pa[it];
+            asm volatile("" : "+v"(ia[it]));
+        }
+#pragma unroll
+        for (int it = 0; it < ITB; it++) {
+            ib[it] = pb[it];
+            asm volatile("" : "+v"(ib[it]));
+        }
+        const uint32_t mq = __builtin_amdgcn_readfirstlane(smask[q]);
+        char* base = (char*)accp + (size_t)q * slice;
+        // opaque copies of the offsets: loads and stores take the form of a
+        // scalar base and a 32-bit offset
+        uint32_t po[ITB][RB];
+#pragma unroll
+        for (int it = 0; it < ITB; it++)
+#pragma unroll
+            for (int k2 = 0; k2 < RB; k2++) {
+                po[it][k2] = off[it][k2];
+                asm volatile("" : "+v"(po[it][k2]));
+            }
+        // previous values of the cells
+        float prev[ITB][RB];
+#pragma unroll
+        for (int it = 0; it < ITB; it++)
+#pragma unroll
+            for (int k2 = 0; k2 < RB; k2++) prev[it][k2] = 0.f;
+        if (!first) {
+#pragma unroll
+            for (int it = 0; it < ITB; it++)
+#pragma unroll
+                for (int k2 = 0; k2 < RB; k2++) prev[it][k2] = *(const float*)(base + po[it][k2]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        {
+            float2 u[5][5];
+#pragma unroll
+            for (int p2 = 0; p2 < 5; p2++) {
+#pragma unroll
+                for (int p1 = 0; p1 < 5; p1++) {
+                    const int pp = p2 + 5 * p1;
+                    const uint32_t sg = ((mq >> pp) & 1u) << 31;
+                    u[p2][p1] = make_float2(__uint_as_float(__float_as_uint(x[pp].x) ^ sg),
+                                            __uint_as_float(__float_as_uint(x[pp].y) ^ sg));
+                }
+                bfly5<false>(u[p2]);
+#pragma unroll
+                for (int s1 = 1; s1 < 5; s1++)
+                    if (p2) u[p2][s1] = cmulf(u[p2][s1], kW25[s1 * p2]);
+            }
+            float2* dst = lds + c1 * CP + m;
+            if (tid < C * NB) {
+#pragma unroll
+                for (int s1 = 0; s1 < 5; s1++) {
+                    float2 w5[5];
+#pragma unroll
+                    for (int p2 = 0; p2 < 5; p2++) w5[p2] = s1 ? cmulf(u[p2][s1], tw1[s1]) : u[p2][s1];
+                    bfly5<false>(w5);
+#pragma unroll
+                    for (int s2 = 0; s2 < 5; s2++) dst[(s1 + 5 * s2) * RP] = s2 ? cmulf(w5[s2], tw5[s2]) : w5[s2];
+                }
+            }
+        }
+        __syncthreads();
+        // radix 8 over m = j + 10 i: output i at slot 10 i + j, times W_80^(i j)
+#pragma unroll
+        for (int it = 0; it < ITA; it++) {
+            if (ia[it] != 0xffffffffu) {
+                float2* a = lds + (ia[it] & 0xffffu);
+                const float2* w = stw + RA * (ia[it] >> 16);
+                float2 v[RA], tw[RA];
+#pragma unroll
+                for (int i = 0; i < RA; i++) v[i] = a[RB * i];
+#pragma unroll
+                for (int i = 1; i < RA; i++) tw[i] = w[i];
+                __builtin_amdgcn_sched_barrier(0);
+                bfly8<false>(v);
+                a[0] = v[0];
+#pragma unroll
+                for (int i = 1; i < RA; i++) a[RB * i] = cmulf(v[i], tw[i]);
+            }
+        }
+        __syncthreads();
+        // radix 10 over j of (s, i): raw bins s + 25 (i + 8 k2)
+#pragma unroll
+        for (int it = 0; it < ITB; it++) {
+            const bool act = ib[it] != 0xffffffffu;
+            float2 v[RB];
+            const float2* a = lds + (act ? ib[it] : 0u);
+#pragma unroll
+            for (int j = 0; j < RB; j++) v[j] = a[j];
+            __builtin_amdgcn_sched_barrier(0);
+            bfly10<false>(v);
+            if (act) {
+#pragma unroll
+                for (int k2 = 0; k2 < RB; k2++) {
+                    // muladd(re, re, im * im), the reference's rotation power
+                    const float pw = fmaf(v[k2].x, v[k2].x, __fmul_rn(v[k2].y, v[k2].y));
+                    *(float*)(base + po[it][k2]) = prev[it][k2] + pw;
+                }
+            }
+        }
+        __syncthreads();  // the rows are consumed
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Reductions: peak with the reference's tie-break order, FP64 row sums.
 // ---------------------------------------------------------------------------
@@ -1472,17 +1697,6 @@ k_finalize(const float* __restrict__ acc, const double* __restrict__ rowsum,
 // grid (bs, nrb, batch); dynamic LDS: 25 padded rows of nb float2, nb row
 // twiddles, ndop cell offsets, R masks.
 // ---------------------------------------------------------------------------
-// W_25^k = exp(-2 pi i k / 25), k = 0..16 (the in-register 5 x 5 DFT's twiddles)
-__constant__ float2 kW25[17] = {
-    {1.0f, -0.0f}, {0.9685831611286311f, -0.2486898871648548f}, {0.8763066800438636f, -0.4817536741017153f},
-    {0.7289686274214116f, -0.6845471059286886f}, {0.5358267949789965f, -0.8443279255020151f},
-    {0.30901699437494745f, -0.9510565162951535f}, {0.06279051952931353f, -0.9980267284282716f},
-    {-0.1873813145857246f, -0.9822872507286887f}, {-0.4257792915650727f, -0.9048270524660195f},
-    {-0.6374239897486897f, -0.7705132427757893f}, {-0.8090169943749473f, -0.5877852522924732f},
-    {-0.9297764858882513f, -0.36812455268467814f}, {-0.9921147013144778f, -0.12533323356430454f},
-    {-0.9921147013144779f, 0.12533323356430429f}, {-0.9297764858882515f, 0.3681245526846779f},
-    {-0.8090169943749478f, 0.5877852522924727f}, {-0.6374239897486895f, 0.7705132427757894f}};
-
 // LDS accesses of one wave stay in program order across this point (the
 // wave's own LDS operations complete in order; this keeps the compiler from
 // moving them across it).
