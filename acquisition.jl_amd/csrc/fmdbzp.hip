@@ -351,6 +351,7 @@ struct fmdbzp_plan {
     bool tile_half = false;      // FMDBZP_PREC_TILE_FP16: FP16 coherent tile
     bool tile_auto = false;      // FMDBZP_PREC_AUTO on a plan that admits the FP16 tile: per call, by sample type
     bool rot_direct = false;     // rotation kernel writes transform outputs straight to the accumulator
+    bool bitsplit = false;       // data-bit search of two 20-period bits: k_column_bitsplit
     int rotsplit = 0;            // direct rotation, few Doppler rows: columns per workgroup of k_column_rotsplit
     // accumulator layout and size that fmdbzp_acquire_noalloc's limit counts
     bool lim_cm = false;
@@ -990,7 +991,20 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
             LB = P->LB = P->rotsplit;
         }
     }
-    // the matrix-core form of the same search (nb = 25 n1, n1 = 2, 4, 10, 20);
+    // two bits of 20 periods, edge offsets of whole periods, a row length with an
+    // in-register transform and 16 columns: 781 -> 210 us (see the kernel)
+    if (d.path == FMDBZP_PATH_SIGN && d.num_data_bits == 2 && d.num_coh == 40 && 20 % d.bit_edge_search_steps == 0 &&
+        bs >= BITSPLIT_C && (size_t)ndop * P->ap * sizeof(float) < (1ull << 32) &&
+        (size_t)ndop * P->tp * sizeof(float2) < (1ull << 31)) {
+#define BS_OK(NN) if (nb == NN) P->bitsplit = true;
+        BITSPLIT_ALL(BS_OK)
+#undef BS_OK
+        if (P->bitsplit) {
+            P->acc_cm = false;
+            LB = P->LB = BITSPLIT_C;
+        }
+    }
+    // the matrix-core form of the E1-like search (nb = 25 n1, n1 = 2, 4, 10, 20);
     // FMDBZP_PREC_AUTO takes it where it is the faster kernel (n1 = 10, 20:
     // at n1 = 2 and 4 the FP32 kernel's transforms are short and both run at
     // the same speed)
@@ -1056,6 +1070,7 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
     if (P->rot2000)
         P->col_lds = (size_t)(2000 + 2 * fft_lds_span(2000)) * sizeof(float2) +
                      ((size_t)d.num_secondary_rotations * 4 + 7) / 8 * 8;
+    if (P->bitsplit) P->col_lds = bitsplit_lds(nb);
     if (P->rot25x80) P->col_lds = kRot2000Lds;
     if (P->rotbig)
         P->col_lds = (size_t)(25 * fft_lds_span(nb) + nb) * sizeof(float2) +
@@ -1101,6 +1116,9 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         (rc = set_lds_attr((const void*)k_column_rotation, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rot2000<512>, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rot25x80, P->col_lds)) ||
+#define BS_ATTR(NN) (rc = set_lds_attr((const void*)k_column_bitsplit<NN>, bitsplit_lds(NN))) ||
+        BITSPLIT_ALL(BS_ATTR)
+#undef BS_ATTR
         (rc = set_lds_attr((const void*)k_column_rotbig<64, 25>, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rotbig<128, 25>, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rotbig<256, 25>, P->col_lds)) ||
@@ -1426,6 +1444,7 @@ int fmdbzp_plan_column_kernel(fmdbzp_plan* plan, char* buf, size_t buflen)
     else if (P->col_static) name = P->tile_half ? "k_column_c160<32,512,fp16>" : "k_column_c160<32,512>";
     else if (P->simple_kernel) name = P->col_onebuf ? "k_column_simple<onebuf>" : "k_column_simple";
     else if (P->d.path == FMDBZP_PATH_ROTATION) name = "k_column_rotation";
+    else if (P->bitsplit) snprintf(tmp, sizeof tmp, "k_column_bitsplit<%d>", P->d.num_blocks);
     else name = "k_column_sign";
     snprintf(buf, buflen, "%s", name);
     return FMDBZP_OK;
@@ -2043,6 +2062,11 @@ int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t elt
                             k_column_simple<true><<<g, FMDBZP_COL_NTHR, P->col_lds, st>>>(A);
                         else
                             k_column_simple<false><<<g, FMDBZP_COL_NTHR, P->col_lds, st>>>(A);
+                    } else if (P->bitsplit) {
+                        const int nt = (BITSPLIT_C * std::max(20, nb) + 63) & ~63;
+#define BS_LAUNCH(NN) if (nb == NN) k_column_bitsplit<NN><<<g, nt, P->col_lds, st>>>(A);
+                        BITSPLIT_ALL(BS_LAUNCH)
+#undef BS_LAUNCH
                     } else if (d.path == FMDBZP_PATH_SIGN) {
                         k_column_sign<<<g, FMDBZP_NTHR, P->col_lds, st>>>(A);
                     } else if (P->rot25x80) {

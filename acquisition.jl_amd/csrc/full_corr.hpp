@@ -927,6 +927,164 @@ k_column_rotsplit(ColumnArgs A, int C)
 #define ROTSPLIT_ALL(OP) ROTSPLIT_NB(10, OP) ROTSPLIT_NB(20, OP)
 
 // ---------------------------------------------------------------------------
+// Data-bit search (k_column_sign) of two 20-period bits, ndop = 40 nb: for
+// every edge offset and sign combination the window's two bits are added onto
+// each other, x_e[i] +- x_e[i + 20] at period i < 20, and transformed with
+// 20 periods of zeros behind them; a cell is the largest power of the set.
+//   X[w] = sum_m W_nb^(k m) W_N^(w' m) DFT20_s(W_40^(o i) y[i nb + m]),
+// w' = 2 s + o, w = w' + 40 k: the zeros cost nothing, both parities o are
+// 20-point transforms of the same y. A workgroup owns C = 16 lags; thread
+// (lag, m) adds the bits and transforms over the periods in registers, thread
+// (lag, s) takes the nb-point rows after one LDS transpose and keeps the
+// maxima of its 2 nb cells in registers, lanes along lags throughout. The tile
+// is read again for each edge and combination, from L2 mostly: 80 registers of
+// samples, or as much LDS, would leave one workgroup per CU.
+// k_column_sign runs the padded transforms with runtime radices in LDS, and
+// its maxima too: 781 us at ndop 640, 4000 columns, 8 PRNs, two edges and two
+// combinations; this takes 210 us. grid (ceil(bs / 16), nb, batch)
+// ---------------------------------------------------------------------------
+#define BITSPLIT_C 16
+#define BITSPLIT_NTHR 384
+// W_40^i = exp(-2 pi i / 40)
+__constant__ float2 kW40[20] = {
+    {1.0f, 0.0f}, {0.98768834059513777f, -0.15643446504023087f},
+    {0.95105651629515353f, -0.3090169943749474f}, {0.8910065241883679f, -0.45399049973954675f},
+    {0.80901699437494745f, -0.58778525229247314f}, {0.70710678118654757f, -0.70710678118654746f},
+    {0.58778525229247314f, -0.80901699437494745f}, {0.4539904997395468f, -0.89100652418836779f},
+    {0.30901699437494745f, -0.95105651629515353f}, {0.15643446504023092f, -0.98768834059513777f},
+    {0.0f, -1.0f}, {-0.15643446504023059f, -0.98768834059513777f},
+    {-0.30901699437494734f, -0.95105651629515364f}, {-0.45399049973954669f, -0.8910065241883679f},
+    {-0.58778525229247303f, -0.80901699437494745f}, {-0.70710678118654746f, -0.70710678118654757f},
+    {-0.80901699437494734f, -0.58778525229247325f}, {-0.89100652418836779f, -0.45399049973954686f},
+    {-0.95105651629515353f, -0.30901699437494751f}, {-0.98768834059513766f, -0.15643446504023098f}};
+constexpr size_t bitsplit_lds(int nb)
+{
+    return ((size_t)20 * rotsplit_pitch(nb, BITSPLIT_C) + (size_t)40 * nb) * sizeof(float2);
+}
+template <int NB>
+__global__ void __launch_bounds__(BITSPLIT_NTHR)
+__attribute__((amdgpu_waves_per_eu(3)))
+k_column_bitsplit(ColumnArgs A)
+{
+    extern __shared__ float2 lds[];
+    constexpr int PB = 20, P = 2 * PB, N = P * NB, C = BITSPLIT_C, pitch = rotsplit_pitch(NB, C);
+    float2* stw = lds + PB * pitch;  // W_N^(s m) at [s][m]
+    const int tid = threadIdx.x;
+    const int lbk = xcd_logical_block();
+    const int lb = __builtin_amdgcn_readfirstlane(lbk % gridDim.x);
+    const int r = __builtin_amdgcn_readfirstlane((lbk / gridDim.x) % gridDim.y);
+    const int p = __builtin_amdgcn_readfirstlane(lbk / (gridDim.x * gridDim.y));
+    const int lag0 = lb * C, ncol = min(C, A.bs - lag0);
+    const int c = tid % C, m = tid / C;  // m: lag within the period, and the bin class s
+    const bool act1 = m < NB && c < ncol, act2 = m < PB && c < ncol;
+    for (int i = tid; i < N; i += blockDim.x) stw[i] = A.twD[(i / NB) * (i % NB)];
+    const float* pat = A.patterns + (size_t)A.pset[A.req[p]] * A.ncoh * A.Q;
+    const float2* T = A.tile + (((size_t)p * NB + r) * N) * A.tp + lag0;
+    const uint32_t voff = (uint32_t)(min(m, NB - 1) * A.tp + min(c, ncol - 1)) * (uint32_t)sizeof(float2);
+    const int es = __builtin_amdgcn_readfirstlane(PB / A.E);
+    const uint32_t bit = (uint32_t)(PB * NB * A.tp) * (uint32_t)sizeof(float2);
+    const uint32_t period = bit / PB;  // bytes of a period's rows; the 40 below 2^31
+    float* accp = A.acc + (size_t)p * A.acc_ps;
+    const int pc = r * A.bs + lag0 + min(c, ncol - 1);
+    __syncthreads();  // twiddles
+    // both parities per read of the tile where their maxima fit the registers
+    // with the transforms, else one after the other
+    constexpr int NO = NB <= 16 ? 2 : 1;
+#pragma unroll
+    for (int o0 = 0; o0 < 2; o0 += NO) {
+        float mx[NO][NB];
+#pragma unroll
+        for (int k = 0; k < NB; k++) mx[0][k] = mx[NO - 1][k] = 0.f;
+#pragma unroll 1
+        for (int e = 0; e < A.E; e++) {
+#pragma unroll 1
+            for (int d = 0; d < A.Q; d++) {
+                // the power does not see a common sign: the second bit relative to the first
+                const uint32_t sg = __builtin_amdgcn_readfirstlane(
+                    (__float_as_uint(pat[(size_t)d * P]) ^ __float_as_uint(pat[(size_t)d * P + PB])) & 0x80000000u);
+                float2 y[PB];
+                {
+                    float2 b1[PB];
+                    uint32_t vo = voff, q0 = e * es * period;
+                    asm volatile("" : "+v"(vo), "+s"(q0));  // opaque: no addresses kept across combinations
+#pragma unroll
+                    for (int i = 0; i < PB; i++) {
+                        const uint32_t q1 = q0 >= bit ? q0 - bit : q0 + bit;
+                        y[i] = *(const float2*)((const char*)T + (q0 + vo));
+                        b1[i] = *(const float2*)((const char*)T + (q1 + vo));
+                        q0 += period;
+                    }
+                    fc_issued();
+#pragma unroll
+                    for (int i = 0; i < PB; i++) {
+                        y[i].x += __uint_as_float(__float_as_uint(b1[i].x) ^ sg);
+                        y[i].y += __uint_as_float(__float_as_uint(b1[i].y) ^ sg);
+                    }
+                }
+#pragma unroll
+                for (int o1 = 0; o1 < NO; o1++) {
+                    const int o = o0 + o1;
+                    if (act1) {
+                        float2 u[PB];
+#pragma unroll
+                        for (int i = 0; i < PB; i++) u[i] = o && i ? cmulf(y[i], kW40[i]) : y[i];
+                        dft_reg<PB, false>(u);
+                        float2* dst = lds + m * C + c;
+                        const float2* w = stw + o * NB + m;
+#pragma unroll
+                        for (int s = 0; s < PB; s++) dst[s * pitch] = s + o ? cmulf(u[s], w[2 * s * NB]) : u[s];
+                    }
+                    __syncthreads();
+                    __builtin_amdgcn_sched_barrier(0);
+                    float2 v[NB];
+                    if (act2) {
+                        const float2* src = lds + m * pitch + c;
+#pragma unroll
+                        for (int i = 0; i < NB; i++) v[i] = src[i * C];
+                    }
+                    __syncthreads();  // the transpose is consumed
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (act2) {
+                        dft_reg<NB, false>(v);
+#pragma unroll
+                        for (int k = 0; k < NB; k++) {
+                            const float pw = abs2_exact(v[k]);
+                            mx[o1][k] = pw > mx[o1][k] ? pw : mx[o1][k];
+                        }
+                    }
+                }
+            }
+        }
+        if (act2) {
+            // raw bin w = 2 s + o + 40 k -> row (w + N / 2) mod N, drifted column
+#pragma unroll
+            for (int o1 = 0; o1 < NO; o1++) {
+                uint32_t off[NB];
+#pragma unroll
+                for (int k = 0; k < NB; k++) {
+                    int row = 2 * m + o0 + o1 + P * k + N / 2;
+                    if (row >= N) row -= N;
+                    int dc = pc + A.shifts[row];
+                    if (dc >= A.spc) dc -= A.spc;
+                    off[k] = (uint32_t)(row * A.ap + dc) * (uint32_t)sizeof(float);
+                }
+                if (!A.first_step) {
+                    float prev[NB];
+#pragma unroll
+                    for (int k = 0; k < NB; k++) prev[k] = *(const float*)((const char*)accp + off[k]);
+#pragma unroll
+                    for (int k = 0; k < NB; k++) mx[o1][k] = prev[k] + mx[o1][k];
+                }
+#pragma unroll
+                for (int k = 0; k < NB; k++) *(float*)((char*)accp + off[k]) = mx[o1][k];
+            }
+        }
+    }
+}
+// OP(NB) for the compiled row lengths
+#define BITSPLIT_ALL(OP) OP(10) OP(11) OP(12) OP(15) OP(16) OP(20) OP(22)
+
+// ---------------------------------------------------------------------------
 // Code periods of 31 RB RC samples with 31, RB and RC pairwise coprime: every
 // multiple of the 1.023 MHz chip rate up to 20.46 MHz (1023 = 3 11 31). By
 // Good-Thomas the transform is three independent DFTs along the axes of a
