@@ -351,6 +351,7 @@ struct fmdbzp_plan {
     bool tile_half = false;      // FMDBZP_PREC_TILE_FP16: FP16 coherent tile
     bool tile_auto = false;      // FMDBZP_PREC_AUTO on a plan that admits the FP16 tile: per call, by sample type
     bool rot_direct = false;     // rotation kernel writes transform outputs straight to the accumulator
+    bool col_reg = false;        // simple path, few Doppler rows: k_column_reg
     bool bitsplit = false;       // data-bit search of two 20-period bits: k_column_bitsplit
     int rotsplit = 0;            // direct rotation, few Doppler rows: columns per workgroup of k_column_rotsplit
     // accumulator layout and size that fmdbzp_acquire_noalloc's limit counts
@@ -910,6 +911,14 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
     P->col_static = P->simple_kernel && ndop == 160 && bs >= 32 &&
                     (size_t)ndop * P->ap * sizeof(float) < (1ull << 31);
     if (P->col_static) LB = 32;
+    // up to 32 rows with an in-register transform (32-bit byte offsets in a PRN's
+    // accumulator and a tile block): 46 -> 15.7 us (see the kernel)
+    if (P->simple_kernel && !P->col_static && (size_t)ndop * P->ap * sizeof(float) < (1ull << 32) &&
+        (size_t)ndop * P->tp * sizeof(float2) < (1ull << 32)) {
+#define CR_OK(NN) if (ndop == NN) P->col_reg = true;
+        COLREG_ALL(CR_OK)
+#undef CR_OK
+    }
     P->use_graph = (d.options & FMDBZP_OPT_GRAPH) != 0;
     P->tile_half = d.precision == FMDBZP_PREC_TILE_FP16;
     P->tile_auto = d.precision == FMDBZP_PREC_AUTO && P->col_static;
@@ -1442,6 +1451,7 @@ int fmdbzp_plan_column_kernel(fmdbzp_plan* plan, char* buf, size_t buflen)
     else if (P->rotsplit) snprintf(tmp, sizeof tmp, "k_column_rotsplit<%d,%d>", P->d.num_coh, P->d.num_blocks);
     else if (P->col_pair) name = P->tile_half ? "k_column_c160_pair<32,512,fp16>" : "k_column_c160_pair<32,512>";
     else if (P->col_static) name = P->tile_half ? "k_column_c160<32,512,fp16>" : "k_column_c160<32,512>";
+    else if (P->col_reg) snprintf(tmp, sizeof tmp, "k_column_reg<%d>", P->d.num_doppler_bins);
     else if (P->simple_kernel) name = P->col_onebuf ? "k_column_simple<onebuf>" : "k_column_simple";
     else if (P->d.path == FMDBZP_PATH_ROTATION) name = "k_column_rotation";
     else if (P->bitsplit) snprintf(tmp, sizeof tmp, "k_column_bitsplit<%d>", P->d.num_blocks);
@@ -2053,6 +2063,11 @@ int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t elt
                             k_column_c160_pair<32, 512, true><<<g, 512, P->col_lds2, st>>>(A, hinv);
                         else
                             k_column_c160_pair<32, 512><<<g, 512, P->col_lds2, st>>>(A, 1.f);
+                    } else if (P->col_reg) {
+                        const dim3 gr((bs + COLREG_NTHR - 1) / COLREG_NTHR, nb, cnt);
+#define CR_LAUNCH(NN) if (ndop == NN) k_column_reg<NN><<<gr, COLREG_NTHR, 0, st>>>(A);
+                        COLREG_ALL(CR_LAUNCH)
+#undef CR_LAUNCH
                     } else if (P->simple_kernel) {
                         if (P->col_static && tile_half)
                             k_column_c160<32, 512, true><<<g, 512, P->col_lds, st>>>(A, hinv);
@@ -2191,7 +2206,7 @@ int autotune(fmdbzp_plan* P)
     const fmdbzp_plan_desc& d = P->d;
     const int F = d.fft_size, ndop = d.num_doppler_bins, nb = d.num_blocks, bs = d.block_size;
     const int cnt = std::min(P->batch, P->nprn);
-    const bool col_generic = P->simple_kernel && !P->col_static;
+    const bool col_generic = P->simple_kernel && !P->col_static && !P->col_reg;
     const TuneKey key{F, nb, bs, ndop, cnt, col_generic ? 1 : 0, P->LB};
     {
         std::lock_guard<std::mutex> g(g_tune_mu);

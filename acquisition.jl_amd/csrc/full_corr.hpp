@@ -190,6 +190,34 @@ __device__ __forceinline__ void dft_square(float2* v)
     static_assert(R == 9 || R == 25, "square radices");
 }
 
+// 32 = 2 x 16: even and odd samples, twiddles W_32^k on the odd half
+template <bool INV>
+__device__ __forceinline__ void dft_32(float2* v)
+{
+    constexpr float c32[16] = {1.f, 0.98078528040323043f, 0.92387953251128674f, 0.83146961230254524f,
+                               0.70710678118654757f, 0.55557023301960229f, 0.38268343236508984f, 0.19509032201612833f,
+                               0.f, -0.19509032201612819f, -0.38268343236508973f, -0.55557023301960196f,
+                               -0.70710678118654746f, -0.83146961230254535f, -0.92387953251128674f, -0.98078528040323043f};
+    constexpr float s32[16] = {0.f, 0.19509032201612825f, 0.38268343236508978f, 0.55557023301960218f,
+                               0.70710678118654746f, 0.83146961230254524f, 0.92387953251128674f, 0.98078528040323043f,
+                               1.f, 0.98078528040323043f, 0.92387953251128674f, 0.83146961230254546f,
+                               0.70710678118654757f, 0.55557023301960218f, 0.38268343236508989f, 0.19509032201612861f};
+    float2 a[16], b[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        a[i] = v[2 * i];
+        b[i] = v[2 * i + 1];
+    }
+    dft_reg<16, INV>(a);
+    dft_reg<16, INV>(b);
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+        const float2 u = k ? cmul_const<INV>(b[k], c32[k], -s32[k]) : b[k];
+        v[k] = make_float2(a[k].x + u.x, a[k].y + u.y);
+        v[k + 16] = make_float2(a[k].x - u.x, a[k].y - u.y);
+    }
+}
+
 template <int R, bool INV>
 __device__ __forceinline__ void dft_reg(float2* v)
 {
@@ -200,6 +228,10 @@ __device__ __forceinline__ void dft_reg(float2* v)
     else if constexpr (R == 22) dft_pfa<2, 11, INV>(v);
     else if constexpr (R == 24) dft_pfa<3, 8, INV>(v);
     else if constexpr (R == 33) dft_pfa<3, 11, INV>(v);
+    else if constexpr (R == 18) dft_pfa<2, 9, INV>(v);
+    else if constexpr (R == 21) dft_pfa<3, 7, INV>(v);
+    else if constexpr (R == 30) dft_pfa<2, 15, INV>(v);
+    else if constexpr (R == 32) dft_32<INV>(v);
     else if constexpr (R == 9) dft_square<3, INV>(v);
     else if constexpr (R == 25) dft_square<5, INV>(v);
     else if constexpr (R == 7 || R == 11 || R == 13 || R == 31) {
@@ -802,6 +834,58 @@ k_fc_code(const int8_t* __restrict__ codes, float2* __restrict__ prnconj, FullPl
         lds, f, tw, threadIdx.x, [&](int i) { return in(0, i); },
         [&](int i, float2 x) { out[i] = make_float2(x.x * scale, -x.y * scale); });
 }
+
+// ---------------------------------------------------------------------------
+// Column stage of the simple path (k_column_simple) with few Doppler rows: a
+// thread owns a code column, reads its N tile values (consecutive lanes,
+// consecutive lags), transforms them in registers and adds the powers to its
+// N cells. No LDS and one round trip to memory: bound by the tile and the
+// accumulator's read-modify-write, 8 N + 8 N bytes per column. k_column_simple
+// gathers blocks of columns into LDS for transforms of any length: 46 us per
+// step at N 15, 30690 columns, 12 PRNs (88 MB), this 15.7 us (5.6 TB/s).
+// grid (ceil(bs / 256), nb, batch)
+// ---------------------------------------------------------------------------
+#define COLREG_NTHR 256
+template <int N>
+__global__ void __launch_bounds__(COLREG_NTHR)
+k_column_reg(ColumnArgs A)
+{
+    const int lbk = xcd_logical_block();
+    const int lb = __builtin_amdgcn_readfirstlane(lbk % gridDim.x);
+    const int r = __builtin_amdgcn_readfirstlane((lbk / gridDim.x) % gridDim.y);
+    const int p = __builtin_amdgcn_readfirstlane(lbk / (gridDim.x * gridDim.y));
+    const int lag = lb * COLREG_NTHR + threadIdx.x;
+    if (lag >= A.bs) return;
+    const char* T = (const char*)(A.tile + ((size_t)p * A.nb + r) * N * A.tp);
+    char* acc = (char*)(A.acc + (size_t)p * A.acc_ps);
+    const int pc = r * A.bs + lag;
+    float2 v[N];
+    float prev[N];
+    uint32_t off[N];
+#pragma unroll
+    for (int n = 0; n < N; n++) v[n] = *(const float2*)(T + (uint32_t)(n * A.tp + lag) * (uint32_t)sizeof(float2));
+    // raw bin k -> row (k + N / 2) mod N (src/plan.jl:528), drifted column
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        const int row = (k + N / 2) % N;
+        int dc = pc + A.shifts[row];
+        if (dc >= A.spc) dc -= A.spc;
+        off[k] = (uint32_t)(row * A.ap + dc) * (uint32_t)sizeof(float);
+        prev[k] = 0.f;
+    }
+    if (!A.first_step) {
+#pragma unroll
+        for (int k = 0; k < N; k++) prev[k] = *(const float*)(acc + off[k]);
+    }
+    fc_issued();
+    dft_reg<N, false>(v);
+#pragma unroll
+    for (int k = 0; k < N; k++) *(float*)(acc + off[k]) = prev[k] + abs2_exact(v[k]);
+}
+// OP(N) for the compiled row counts
+#define COLREG_ALL(OP)                                                                                           \
+    OP(4) OP(5) OP(6) OP(7) OP(8) OP(9) OP(10) OP(11) OP(12) OP(13) OP(15) OP(16) OP(18) OP(20) OP(21) OP(22) \
+    OP(24) OP(25) OP(30) OP(32)
 
 // ---------------------------------------------------------------------------
 // Direct rotation search (k_column_rotation with one pattern per rotation
