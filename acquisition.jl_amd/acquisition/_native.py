@@ -64,6 +64,16 @@ class PrnStats(ctypes.Structure):
     ]
 
 
+class PrnResult(ctypes.Structure):
+    _fields_ = [
+        ("cn0_dbhz", ctypes.c_double),
+        ("code_phase", ctypes.c_double),
+        ("doppler_offset", ctypes.c_double),
+        ("peak_to_noise", ctypes.c_float),
+        ("reserved", ctypes.c_int32),
+    ]
+
+
 class Request(ctypes.Structure):
     _fields_ = [
         ("plan", ctypes.c_void_p),
@@ -128,6 +138,7 @@ EXPORTED_SYMBOLS = (
     "fmdbzp_plan_create",
     "fmdbzp_acquire",
     "fmdbzp_acquire_batch",
+    "fmdbzp_prn_results",
     "fmdbzp_acquire_noalloc",
     "fmdbzp_plan_destroy",
     "fmdbzp_last_error",
@@ -155,6 +166,9 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.fmdbzp_acquire.argtypes = [P, P, ctypes.c_int32, ctypes.c_int64, ctypes.c_double, P, ctypes.c_int32,
                                    ctypes.c_uint32, P, P]
     lib.fmdbzp_acquire.restype = ctypes.c_int
+    D, I = ctypes.c_double, ctypes.c_int32
+    lib.fmdbzp_prn_results.argtypes = [P, I, I, I, I, D, D, D, D, D, I, P]
+    lib.fmdbzp_prn_results.restype = ctypes.c_int
     lib.fmdbzp_acquire_batch.argtypes = [P, ctypes.c_int32]
     lib.fmdbzp_acquire_batch.restype = ctypes.c_int
     lib.fmdbzp_plan_destroy.argtypes = [P]
@@ -197,6 +211,13 @@ def lib() -> ctypes.CDLL:
     if _lib is None:
         _lib = load_library()
     return _lib
+
+
+def prn_results(stats, n: int, spc: int, nb: int, bs: int, fs: float, fc: float, code_length: float, tcoh: float,
+                spacing: float, interpolate: int, out_ptr: int):
+    """`fmdbzp_prn_results` over a ctypes array of `PrnStats`."""
+    _check(lib().fmdbzp_prn_results(stats, n, spc, nb, bs, fs, fc, code_length, tcoh, spacing, interpolate, out_ptr),
+           "fmdbzp_prn_results")
 
 
 def acquire_batch(reqs):

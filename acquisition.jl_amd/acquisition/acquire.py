@@ -220,27 +220,6 @@ class _SignalView:
 # ---------------------------------------------------------------------------
 # acquire_
 # ---------------------------------------------------------------------------
-def _interpolate(plan: AcquisitionPlan, peak, noise, code_nbrs, dop_nbrs, delay: int, code_phase: float,
-                 doppler: float):
-    """Subsample interpolation of one peak (src/acquire.jl:593-619, :714-748): a parabola
-    through the code (Doppler) neighbours when the larger one exceeds sqrt(noise)."""
-    fs = plan.sampling_freq
-    fc = plan.system.get_code_frequency()
-    code_length = plan.system.get_code_length()
-    pl, pr = f32(code_nbrs[0]), f32(code_nbrs[1])
-    dl, dr = f32(dop_nbrs[0]), f32(dop_nbrs[1])
-    sq = np.sqrt(noise)
-    if max(pl, pr) > sq:
-        frac = parabolic_interp(pl, peak, pr)
-        if isinstance(frac, np.float32):
-            di = f32(f32(delay) + frac)
-            code_phase = jl_mod(float(-di) * fc / fs, code_length)
-    if max(dl, dr) > sq:
-        frac = parabolic_interp(dl, peak, dr)
-        doppler = doppler + float(frac) * plan.doppler_spacing_hz
-    return code_phase, doppler
-
-
 def _get_result_buffer(plan: AcquisitionPlan, prn_idx: int) -> np.ndarray:
     """Plan-owned (ndop, spc_eff) Float32 surface, allocated on first use and
     reused (src/acquire.jl:221-228)."""
@@ -279,7 +258,11 @@ def acquire_(plan: AcquisitionPlan, signal, prns: Union[int, Sequence[int]], *, 
 def _prepare(plan: AcquisitionPlan, signal, prns, interm_freq, store_power_bins):
     """Validation shared by `acquire_` and `acquire_batch` (src/acquire.jl:62-72)."""
     prns = [int(p) for p in prns]
-    if not all(p in plan.avail_prns for p in prns):
+    pos = {}
+    for i, p in enumerate(plan.avail_prns):
+        pos.setdefault(p, i)
+    idx = [pos.get(p) for p in prns]
+    if None in idx:
         raise ArgumentError(f"All requested PRNs must be in plan.avail_prns. Got: {prns}, "
                             f"available: {plan.avail_prns}")
     if plan.native is None:
@@ -292,7 +275,6 @@ def _prepare(plan: AcquisitionPlan, signal, prns, interm_freq, store_power_bins)
             f"Signal has {sv.n} samples → {num_segments} full segments of {segment_length}, "
             f"but plan.num_noncoherent_accumulations={plan.num_noncoherent_accumulations}. "
             "Provide a longer signal.")
-    idx = [plan.avail_prns.index(p) for p in prns]
     flags = _native.FLAG_DEVICE_SIGNAL if sv.device else 0
     bufs = surfaces = None
     if store_power_bins and prns:
@@ -302,19 +284,23 @@ def _prepare(plan: AcquisitionPlan, signal, prns, interm_freq, store_power_bins)
     return prns, sv, idx, flags, bufs, surfaces
 
 
-# numpy view of fmdbzp_prn_stats (the ctypes PrnStats layout), built once
-_STATS_DTYPE = np.dtype({"names": [f[0] for f in _native.PrnStats._fields_],
-                         "formats": [np.dtype(f[1]) for f in _native.PrnStats._fields_],
-                         "offsets": [getattr(_native.PrnStats, f[0]).offset for f in _native.PrnStats._fields_],
-                         "itemsize": ctypes.sizeof(_native.PrnStats)})
+def _view(struct):
+    """numpy dtype of a ctypes structure."""
+    return np.dtype({"names": [f[0] for f in struct._fields_], "formats": [np.dtype(f[1]) for f in struct._fields_],
+                     "offsets": [getattr(struct, f[0]).offset for f in struct._fields_],
+                     "itemsize": ctypes.sizeof(struct)})
+
+
+# numpy views of fmdbzp_prn_stats and fmdbzp_prn_result, built once
+_STATS_DTYPE = _view(_native.PrnStats)
+_RESULT_DTYPE = _view(_native.PrnResult)
 
 
 def _results_from_stats(plan, stats, prns, sv, interm_freq, subsample_interpolation, bufs):
     """Result extraction (src/acquire.jl:544-671 and :681-781) from the
-    engine's per-PRN statistics, all PRNs of the call at once. The Float32
-    steps (signal power, peak-to-noise ratio, the CN0 ratio) are numpy float32
-    array operations, each rounded to Float32 as the reference's scalar code
-    does; the code phase and Doppler follow in Float64 per PRN."""
+    engine's per-PRN statistics. The scalar formulas (power ratios in Float32,
+    code phase and Doppler in Float64, the subsample parabola) are evaluated by
+    `fmdbzp_prn_results` for all PRNs of the call."""
     n = len(prns)
     a = np.frombuffer(stats, dtype=_STATS_DTYPE, count=n)
     system = plan.system
@@ -322,18 +308,12 @@ def _results_from_stats(plan, stats, prns, sv, interm_freq, subsample_interpolat
     fc = system.get_code_frequency()
     code_length = system.get_code_length()
     spc, nb, bsz = plan.samples_per_code, plan.num_blocks, plan.block_size
-    peak = np.ascontiguousarray(a["peak_power"], dtype=np.float32)
-    noise = np.ascontiguousarray(a["noise_power"], dtype=np.float32)
-    with np.errstate(divide="ignore", invalid="ignore"):
-        signal_power = peak - noise
-        ptn = (signal_power + noise) / noise
-        ratio = (signal_power / noise).tolist()
-    code_period = code_length / fc
-    tcoh = plan.num_coherently_integrated_code_periods * code_period
-    rows, cols = a["peak_row"].tolist(), a["peak_col"].tolist()
-    peaks, noises = peak.tolist(), noise.tolist()
-    nbrs = np.stack([a["code_left"], a["code_right"], a["dop_left"], a["dop_right"]], axis=1).tolist()
-    nsums, ncells = a["noise_sum"].tolist(), a["noise_cells"].tolist()
+    tcoh = plan.num_coherently_integrated_code_periods * (code_length / fc)
+    vals = np.empty(n, dtype=_RESULT_DTYPE)
+    _native.prn_results(stats, n, spc, nb, bsz, fs, fc, code_length, tcoh, plan.doppler_spacing_hz,
+                        1 if subsample_interpolation else 0, vals.ctypes.data)
+    # float32 scalars of the two fields that the results hold as such
+    noise, ptn = list(a["noise_power"]), list(vals["peak_to_noise"])
     # the secondary-code phase of a detected PRN (src/acquire.jl:646-652) is
     # estimated for all such PRNs in one device call below
     R = plan.num_secondary_rotations
@@ -343,20 +323,15 @@ def _results_from_stats(plan, stats, prns, sv, interm_freq, subsample_interpolat
                              num_noncoherent_integrations=plan.num_noncoherent_accumulations)
     nnc, dfreqs = plan.num_noncoherent_accumulations, plan.doppler_freqs
     results, pending = [], []
-    for j, p in enumerate(prns):
-        rj = ratio[j]
-        cn0 = 10 * math.log10(rj / tcoh / 1.0) if rj > 0 else (-math.inf if rj == 0 else math.nan)
-        row, col = rows[j], cols[j]
-        delay = fmdbzp_column_to_tau(col % spc, nb, bsz)
-        code_phase = jl_mod(-delay * fc / fs, code_length)
-        doppler = float(plan.doppler_freqs[row])
+    for j, (q, v) in enumerate(zip(a.tolist(), vals.tolist())):
+        pk, row, col, nz, cl, cr, dl, dr, nsum, ncell = q
+        doppler = float(dfreqs[row])
         if subsample_interpolation:
-            code_phase, doppler = _interpolate(plan, peak[j], noise[j], nbrs[j][0:2], nbrs[j][2:4], delay, code_phase,
-                                               doppler)
+            doppler += v[2]
         # positional: the field order of AcquisitionResults
-        r = AcquisitionResults(system, p, fs, doppler, code_phase, None, cn0, noise[j], ptn[j], nnc,
+        r = AcquisitionResults(system, prns[j], fs, doppler, v[1], None, v[0], noise[j], ptn[j], nnc,
                                bufs[j] if bufs is not None else None, dfreqs, nb, bsz, R,
-                               (peaks[j], row, col, noises[j], nbrs[j], nsums[j], ncells[j]))
+                               (pk, row, col, nz, [cl, cr, dl, dr], nsum, ncell))
         if thr is not None and float(ptn[j]) > thr:
             pending.append(r)
         results.append(r)

@@ -1427,6 +1427,55 @@ int fmdbzp_secondary_phase(fmdbzp_plan* plan, const void* signal, int32_t eltype
     return FMDBZP_OK;
 }
 
+// Host arithmetic of the results: 44 results of four requests took 210 us in
+// numpy and Python, a numpy scalar operation at a time.
+int fmdbzp_prn_results(const fmdbzp_prn_stats* stats, int32_t n, int32_t samples_per_code, int32_t num_blocks,
+                       int32_t block_size, double sampling_freq_hz, double code_freq_hz, double code_length,
+                       double coherent_time_s, double doppler_spacing_hz, int32_t interpolate, fmdbzp_prn_result* out)
+{
+#pragma clang fp contract(off)
+    if (n < 0 || (n > 0 && (!stats || !out))) return set_err(FMDBZP_EINVAL, "fmdbzp_prn_results: null argument");
+    if (samples_per_code <= 0 || num_blocks <= 0 || block_size <= 0)
+        return set_err(FMDBZP_EINVAL, "fmdbzp_prn_results: sizes must be positive");
+    // Julia `mod`: fmod, shifted into the sign of y
+    auto jl_mod = [](double x, double y) {
+        const double r = fmod(x, y);
+        if (r == 0.0) return copysign(0.0, y);
+        return (r > 0) != (y > 0) ? r + y : r;
+    };
+    // `_parabolic_interp` in Float32; false where the denominator is zero
+    auto parabola = [](float left, float peak, float right, float* frac) {
+        const float denom = 2.f * ((2.f * peak - left) - right);
+        if (denom == 0.f) return false;
+        *frac = (right - left) / denom;
+        return true;
+    };
+    for (int i = 0; i < n; i++) {
+        const fmdbzp_prn_stats& q = stats[i];
+        fmdbzp_prn_result& o = out[i];
+        const float signal = q.peak_power - q.noise_power;
+        o.peak_to_noise = (signal + q.noise_power) / q.noise_power;
+        const double ratio = (double)(signal / q.noise_power);
+        o.cn0_dbhz = ratio > 0 ? 10 * log10(ratio / coherent_time_s) : ratio == 0 ? -INFINITY : NAN;
+        const int col = q.peak_col % samples_per_code, br = col / block_size;
+        const int delay = ((num_blocks - br) % num_blocks) * block_size + col % block_size;
+        o.code_phase = jl_mod((double)-delay * code_freq_hz / sampling_freq_hz, code_length);
+        o.doppler_offset = 0.0;
+        o.reserved = 0;
+        if (interpolate) {
+            const float sq = sqrtf(q.noise_power);
+            float frac;
+            if ((q.code_right > q.code_left ? q.code_right : q.code_left) > sq &&
+                parabola(q.code_left, q.peak_power, q.code_right, &frac))
+                o.code_phase = jl_mod((double)-((float)delay + frac) * code_freq_hz / sampling_freq_hz, code_length);
+            if ((q.dop_right > q.dop_left ? q.dop_right : q.dop_left) > sq &&
+                parabola(q.dop_left, q.peak_power, q.dop_right, &frac))
+                o.doppler_offset = (double)frac * doppler_spacing_hz;
+        }
+    }
+    return FMDBZP_OK;
+}
+
 int fmdbzp_plan_tuning(fmdbzp_plan* plan, char* buf, size_t buflen)
 {
     if (!plan) return set_err(FMDBZP_EHANDLE, "null plan");

@@ -235,6 +235,29 @@ int fmdbzp_acquire(fmdbzp_plan* plan,
                    float* const* out_surfaces);
 
 /*
+ * Result formulas of one PRN (src/acquire.jl:9-13, :544-671): Float32 power
+ * ratios, code phase and Doppler in Float64.
+ */
+typedef struct fmdbzp_prn_result {
+    double cn0_dbhz;        /* 10 log10(signal / noise / coherent time); -inf, NaN as the ratio is 0, below */
+    double code_phase;      /* chips, in [0, code length)                             */
+    double doppler_offset;  /* Hz from the peak row's bin (0 without interpolation)   */
+    float peak_to_noise;
+    int32_t reserved;
+} fmdbzp_prn_result;
+
+/*
+ * Evaluate the result formulas over the statistics of a call, on the host.
+ * `interpolate` != 0: a parabola through the code (Doppler) neighbours where
+ * the larger one exceeds sqrt(noise). FMDBZP_EINVAL on a null pointer or
+ * non-positive sizes.
+ */
+int fmdbzp_prn_results(const fmdbzp_prn_stats* stats, int32_t n, int32_t samples_per_code, int32_t num_blocks,
+                       int32_t block_size, double sampling_freq_hz, double code_freq_hz, double code_length,
+                       double coherent_time_s, double doppler_spacing_hz, int32_t interpolate,
+                       fmdbzp_prn_result* out);
+
+/*
  * One request of a batch: the arguments of fmdbzp_acquire. `nprn` PRN
  * indices of `plan` searched over `signal`.
  */
