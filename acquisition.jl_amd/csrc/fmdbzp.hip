@@ -357,7 +357,7 @@ struct fmdbzp_plan {
     // accumulator layout and size that fmdbzp_acquire_noalloc's limit counts
     bool lim_cm = false;
     size_t lim_acc_ps = 0;
-    bool rot25x80 = false;       // ... with 25 periods of 80 rows: k_column_rot25x80
+    bool rot25 = false;          // 25 periods of 50, 80, 100, 250 or 500 rows: k_column_rot25
     bool rot2000 = false;        // direct rotation at ndop 2000: compile-time kernel, one column per workgroup
     // Direct rotation at large ndop (k_column_rotbig), accumulated in code-column
     // chunks: every chunk owns chunk_cols scrambled code columns (the last one
@@ -958,7 +958,7 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         // 25 periods of 80 rows, the E1-like search: 10.5 ms per PRN-step at 25 MHz
         // against 15.1 ms of the 16 x 5 x 5 x 5 kernel, which serves other N_coh
         // (the masks of a workgroup hold at most 64 rotations)
-        P->rot25x80 = d.num_coh == 25 && d.num_secondary_rotations <= 64;
+        P->rot25 = d.num_coh == 25 && d.num_secondary_rotations <= 64;
         P->acc_cm = true;
         LB = P->LB = 1;
     }
@@ -982,6 +982,9 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         if (ok && lds <= kLdsMax) {
             P->rotbig = nt;
             P->rotbig_nt = nt;
+            // 25 MHz, per PRN-step against k_column_rotbig: 6.3 / 8.9 ms at 50 rows, 12.9 / 17.6 at
+            // 100, 32.3 / 55.6 at 250, 72 / 132 at 500 (the masks of a workgroup hold at most 64 rotations)
+            P->rot25 = (nb == 50 || nb == 100 || nb == 250 || nb == 500) && d.num_secondary_rotations <= 64;
             P->acc_cm = true;
             LB = P->LB = 1;
         }
@@ -1080,7 +1083,7 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         P->col_lds = (size_t)(2000 + 2 * fft_lds_span(2000)) * sizeof(float2) +
                      ((size_t)d.num_secondary_rotations * 4 + 7) / 8 * 8;
     if (P->bitsplit) P->col_lds = bitsplit_lds(nb);
-    if (P->rot25x80) P->col_lds = kRot2000Lds;
+    if (P->rot25 && P->rot2000) P->col_lds = rot25_lds<80>();
     if (P->rotbig)
         P->col_lds = (size_t)(25 * fft_lds_span(nb) + nb) * sizeof(float2) +
                      ((size_t)ndop + d.num_secondary_rotations) * sizeof(uint32_t);
@@ -1124,7 +1127,11 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         (rc = set_lds_attr((const void*)k_column_sign, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rotation, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rot2000<512>, P->col_lds)) ||
-        (rc = set_lds_attr((const void*)k_column_rot25x80, P->col_lds)) ||
+        (rc = set_lds_attr((const void*)k_column_rot25<80, false>, rot25_lds<80>())) ||
+        (rc = set_lds_attr((const void*)k_column_rot25<50, true>, rot25_lds<50>())) ||
+        (rc = set_lds_attr((const void*)k_column_rot25<100, true>, rot25_lds<100>())) ||
+        (rc = set_lds_attr((const void*)k_column_rot25<250, true>, rot25_lds<250>())) ||
+        (rc = set_lds_attr((const void*)k_column_rot25<500, true>, rot25_lds<500>())) ||
 #define BS_ATTR(NN) (rc = set_lds_attr((const void*)k_column_bitsplit<NN>, bitsplit_lds(NN))) ||
         BITSPLIT_ALL(BS_ATTR)
 #undef BS_ATTR
@@ -1133,10 +1140,6 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         (rc = set_lds_attr((const void*)k_column_rotbig<256, 25>, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rotbig<320, 25>, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rotbig<512, 25>, P->col_lds)) ||
-        (rc = set_lds_attr((const void*)k_column_rotbig<64, 25, 50>, P->col_lds)) ||
-        (rc = set_lds_attr((const void*)k_column_rotbig<128, 25, 100>, P->col_lds)) ||
-        (rc = set_lds_attr((const void*)k_column_rotbig<256, 25, 250>, P->col_lds)) ||
-        (rc = set_lds_attr((const void*)k_column_rotbig<512, 25, 500>, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rotmma<8, 3, 20>, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rotmma<4, 3, 10>, P->col_lds)) ||
         (rc = set_lds_attr((const void*)k_column_rotmma<4, 1, 4>, P->col_lds)) ||
@@ -1811,34 +1814,24 @@ int launch_rotbig(fmdbzp_plan* P, const Work& W, ColumnArgs A, int32_t nreq, boo
                         case 2: k_column_rotmma<2, 1, 2><<<g, 128, P->col_lds, st>>>(A); break;
                         default: return set_err(FMDBZP_EINVAL, "no matrix-core rotation kernel for n1 = %d", P->rotmma);
                         }
+                    } else if (P->rot25) {
+                        switch (nb) {
+#define R25_LAUNCH(NN)                                                                                     \
+    case NN:                                                                                               \
+        k_column_rot25<NN, true><<<dim3((bs + Rot25<NN>::C - 1) / Rot25<NN>::C, nrb, cnt), Rot25<NN>::NT, \
+                                   rot25_lds<NN>(), st>>>(A);                                              \
+        break;
+                            R25_LAUNCH(50) R25_LAUNCH(100) R25_LAUNCH(250) R25_LAUNCH(500)
+#undef R25_LAUNCH
+                        default: return set_err(FMDBZP_EINVAL, "no rotation kernel for %d rows", nb);
+                        }
                     } else {
                         switch (nt) {
-                        // the E1-like row lengths (nb = 50, 100, 250, 500) with a compile-time row plan
-                        case 64:
-                            if (nb == 50)
-                                k_column_rotbig<64, 25, 50><<<g, 64, P->col_lds, st>>>(A, P->prow, P->d_twR, P->rgrp);
-                            else
-                                k_column_rotbig<64, 25><<<g, 64, P->col_lds, st>>>(A, P->prow, P->d_twR, P->rgrp);
-                            break;
-                        case 128:
-                            if (nb == 100)
-                                k_column_rotbig<128, 25, 100><<<g, 128, P->col_lds, st>>>(A, P->prow, P->d_twR, P->rgrp);
-                            else
-                                k_column_rotbig<128, 25><<<g, 128, P->col_lds, st>>>(A, P->prow, P->d_twR, P->rgrp);
-                            break;
-                        case 256:
-                            if (nb == 250)
-                                k_column_rotbig<256, 25, 250><<<g, 256, P->col_lds, st>>>(A, P->prow, P->d_twR, P->rgrp);
-                            else
-                                k_column_rotbig<256, 25><<<g, 256, P->col_lds, st>>>(A, P->prow, P->d_twR, P->rgrp);
-                            break;
+                        case 64: k_column_rotbig<64, 25><<<g, 64, P->col_lds, st>>>(A, P->prow, P->d_twR, P->rgrp); break;
+                        case 128: k_column_rotbig<128, 25><<<g, 128, P->col_lds, st>>>(A, P->prow, P->d_twR, P->rgrp); break;
+                        case 256: k_column_rotbig<256, 25><<<g, 256, P->col_lds, st>>>(A, P->prow, P->d_twR, P->rgrp); break;
                         case 320: k_column_rotbig<320, 25><<<g, 320, P->col_lds, st>>>(A, P->prow, P->d_twR, P->rgrp); break;
-                        case 512:
-                            if (nb == 500)
-                                k_column_rotbig<512, 25, 500><<<g, 512, P->col_lds, st>>>(A, P->prow, P->d_twR, P->rgrp);
-                            else
-                                k_column_rotbig<512, 25><<<g, 512, P->col_lds, st>>>(A, P->prow, P->d_twR, P->rgrp);
-                            break;
+                        case 512: k_column_rotbig<512, 25><<<g, 512, P->col_lds, st>>>(A, P->prow, P->d_twR, P->rgrp); break;
                         default: return set_err(FMDBZP_EINVAL, "no rotation kernel for %d threads", nt);
                         }
                     }
@@ -2136,8 +2129,8 @@ int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t elt
 #undef BS_LAUNCH
                     } else if (d.path == FMDBZP_PATH_SIGN) {
                         k_column_sign<<<g, FMDBZP_NTHR, P->col_lds, st>>>(A);
-                    } else if (P->rot25x80) {
-                        k_column_rot25x80<<<dim3((bs + ROT2000_C - 1) / ROT2000_C, nb, cnt), ROT2000_NTHR, P->col_lds, st>>>(A);
+                    } else if (P->rot25) {
+                        k_column_rot25<80, false><<<dim3((bs + Rot25<80>::C - 1) / Rot25<80>::C, nb, cnt), Rot25<80>::NT, P->col_lds, st>>>(A);
                     } else if (P->rot2000) {
                         k_column_rot2000<512><<<dim3(bs, nb, cnt), 512, P->col_lds, st>>>(A);
                     } else if (P->rotsplit) {

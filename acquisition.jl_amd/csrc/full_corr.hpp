@@ -1011,6 +1011,256 @@ k_column_rotsplit(ColumnArgs A, int C)
 #define ROTSPLIT_ALL(OP) ROTSPLIT_NB(10, OP) ROTSPLIT_NB(20, OP)
 
 // ---------------------------------------------------------------------------
+// Direct rotation search of 25 coherent periods, ndop = 25 NB (the E1-like
+// searches): rows n = p NB + m, raw bins w = s + 25 k, as k_column_rotbig,
+//   X_q[s + 25 k] = sum_m W_NB^(k m) W_N^(s m) sum_p sigma_q[p] W_25^(s p) x[p NB + m].
+// A workgroup owns C code columns. Thread (column, m) keeps the 25 samples
+// of its lag in registers for all rotations; per rotation it applies the
+// signs (flips of the float sign bit), a 5 x 5 DFT over p and the twiddles,
+// and writes the 25 classes s to LDS. The NB-point transforms of the 25 C
+// rows follow as RA x RB in place, and the last stage adds the powers to the
+// cells straight from its registers: butterfly (s, i) of a column has rows
+// s + 25 i + 25 RA k2, so consecutive threads hold consecutive rows of the
+// column-major accumulator. Offsets of the cells stay in registers, and their
+// previous values are read ahead of the rotation's first stage.
+// CHUNK: cells outside a code-column window are dropped and the tile holds
+// blocks rb0 .. rb0 + nrb (launch_rotbig); else the whole code period.
+// grid (ceil(bs / C), column blocks, batch)
+// Bound by vector instructions. At NB 80: 2130 per column and rotation against
+// 2600 of k_column_rot2000, 8.5 ms at 100000 columns and R 25 if
+// nothing waited, next to 41.9 GB of cells (8.5 ms at a copy's rate). Three
+// columns make four waves, one per SIMD, and two workgroups per CU leave the
+// 231 registers for all 30 offsets and values: four columns in five waves, two
+// and a half per SIMD with one butterfly's cells ahead, took 14.4 ms
+// and k_column_rot2000 15.1 ms; this takes 10.5 ms per PRN-step. The other row
+// lengths take C and RA x RB that keep 200 to 250 of 256 threads (500 of 512)
+// busy in the 25-point stage with at most 30 cells each; against
+// k_column_rotbig with compile-time rows, per PRN-step at 25 MHz: 8.9 -> 6.3 ms
+// at NB 50, 17.6 -> 12.9 at 100, 55.6 -> 32.3 at 250, 132 -> 72 at 500 (windows
+// of a PRN added up, one step).
+template <int NB>
+struct Rot25;
+template <> struct Rot25<50> { static constexpr int RA = 10, RB = 5, C = 5, NT = 256; };
+template <> struct Rot25<80> { static constexpr int RA = 8, RB = 10, C = 3, NT = 256; };
+template <> struct Rot25<100> { static constexpr int RA = 10, RB = 10, C = 2, NT = 256; };
+template <> struct Rot25<250> { static constexpr int RA = 10, RB = 25, C = 1, NT = 256; };
+template <> struct Rot25<500> { static constexpr int RA = 20, RB = 25, C = 1, NT = 512; };
+// pitches of a row and of a column: odd, and about 32 / C mod 32, so that lanes
+// along rows and along columns spread over the banks
+template <int NB>
+constexpr int rot25_row() { return NB | 1; }
+template <int NB>
+constexpr int rot25_col()
+{
+    constexpr int C = Rot25<NB>::C, n = 25 * rot25_row<NB>();
+    return n + (((32 + C - 1) / C - n) % 32 + 32) % 32;
+}
+template <int NB>
+constexpr size_t rot25_lds() { return (size_t)(Rot25<NB>::C * rot25_col<NB>() + NB) * sizeof(float2); }
+
+template <int NB, bool CHUNK>
+__global__ void __launch_bounds__(Rot25<NB>::NT)
+__attribute__((amdgpu_waves_per_eu(2, 2)))
+k_column_rot25(ColumnArgs A)
+{
+    constexpr int P = 25, N = P * NB, RA = Rot25<NB>::RA, RB = Rot25<NB>::RB, C = Rot25<NB>::C, NT = Rot25<NB>::NT;
+    constexpr int RP = rot25_row<NB>(), CP = rot25_col<NB>();
+    constexpr int ITA = (C * P * RB + NT - 1) / NT, ITB = (C * P * RA + NT - 1) / NT;
+    static_assert(C * NB <= NT && RA * RB == NB && N % 2 == 0 && C * CP < 65536 && NT >= 64, "work split");
+    extern __shared__ float2 lds[];
+    float2* stw = lds + C * CP;                // W_NB^(i j) at [j][i], i < RA, j < RB
+    __shared__ uint32_t smask[64];
+    const int tid = threadIdx.x;
+    const int lbk = xcd_logical_block();
+    const int lb = __builtin_amdgcn_readfirstlane(lbk % gridDim.x);
+    const int rr = __builtin_amdgcn_readfirstlane((lbk / gridDim.x) % gridDim.y);  // tile block
+    const int p = __builtin_amdgcn_readfirstlane(lbk / (gridDim.x * gridDim.y));
+    const int nrb = CHUNK ? A.nrb : NB;
+    int r = CHUNK ? A.rb0 + rr : rr;
+    if (CHUNK && r >= NB) r -= NB;
+    const int lag0 = lb * C, ncol = min(C, A.bs - lag0);
+    for (int j = tid; j < NB; j += NT) stw[j] = A.twD[P * (j % RA) * (j / RA)];
+    if (tid < A.R) {
+        const float* pat = A.patterns + ((size_t)A.pset[A.req[p]] * A.Q + tid) * A.ncoh;
+        uint32_t msk = 0;
+        for (int q = 0; q < P; q++)
+            if (pat[q] < 0.f) msk |= 1u << q;
+        smask[tid] = msk;
+    }
+    // lag m of column c: 25 samples of the column rotated by its alignment
+    // (src/noncoherent_integration.jl:212-215), factors of W_N^(s m), s = s1 + 5 s2
+    const int c1 = tid % C, m = min(tid / C, NB - 1);
+    float2 x[P], tw1[5], tw5[5];
+    {
+        const int lag = lag0 + min(c1, ncol - 1), pc = r * A.bs + lag;
+        const int wrap = ((NB - pc / A.bs) % NB) * A.bs + (pc % A.bs);
+        const int eff = ((wrap + (A.bs >> 1)) / A.bs) % NB;
+        const float2* T = A.tile + (((size_t)p * nrb + rr) * N) * A.tp + lag;
+#pragma unroll
+        for (int q = 0; q < P; q++) {
+            int src = q * NB + m + eff;
+            if (src >= N) src -= N;
+            // neighbouring workgroups (the next lags) read the same tile lines: plain, cached loads
+            x[q] = T[(size_t)src * A.tp];
+        }
+#pragma unroll
+        for (int i = 1; i < 5; i++) {
+            tw1[i] = A.twD[i * m];
+            tw5[i] = A.twD[5 * i * m];
+        }
+    }
+    float* accp = A.acc + (size_t)p * A.acc_ps;
+    const size_t slice = (size_t)(CHUNK ? A.slice_cols : A.spc) * A.acc_ldc * 4;  // bytes of a rotation slice (below 2^32)
+    const bool first = A.first_step != 0;
+    const bool whole = !CHUNK || A.winlen >= A.spc;  // no cell falls outside the window
+    // The stages' butterflies (their index arithmetic is full of slow
+    // multiplications). Radix RA: LDS index | j << 16, all ones past the end.
+    // Radix RB: LDS index and the byte offsets of the cells in a slice; it takes
+    // the threads in reverse, so that the remainders of the two stages fall to
+    // different waves.
+    uint32_t pa[ITA], pb[ITB], off[ITB][RB];
+#pragma unroll
+    for (int it = 0; it < ITA; it++) {
+        const uint32_t idx = tid + it * NT, c = idx / (P * RB), b = idx % (P * RB), j = b / P, s = b % P;
+        pa[it] = idx < C * P * RB ? (c * CP + s * RP + j) | j << 16 : 0xffffffffu;
+    }
+#pragma unroll
+    for (int it = 0; it < ITB; it++) {
+        const uint32_t idx = NT - 1 - tid + it * NT, c = idx / (P * RA), b = idx % (P * RA), i = b / P, s = b % P;
+        const bool act = idx < C * P * RA && c < (uint32_t)ncol;
+        pb[it] = act ? c * CP + s * RP + RB * i : 0xffffffffu;
+#pragma unroll
+        for (int k2 = 0; k2 < RB; k2++) {
+            // raw bin b + 25 RA k2, its sorted row (N / 2 further), column + its drift (mod spc)
+            int row = (int)b + P * RA * k2 + N / 2;
+            if (row >= N) row -= N;
+            int dc = r * A.bs + lag0 + (act ? (int)c : 0) + A.shifts[row];
+            if (dc >= A.spc) dc -= A.spc;
+            if (CHUNK) {
+                dc -= A.win0;
+                if (dc < 0) dc += A.spc;
+            }
+            off[it][k2] = ((uint32_t)row + (uint32_t)dc * (uint32_t)A.acc_ldc) * 4u;
+            if (CHUNK && dc >= A.winlen) off[it][k2] = ~0u;
+        }
+    }
+    __syncthreads();  // tables and masks
+#pragma unroll 1
+    for (int q = 0; q < A.R; q++) {
+        // opaque copies: what follows from them is not hoisted into registers
+        uint32_t ia[ITA], ib[ITB];
+#pragma unroll
+        for (int it = 0; it < ITA; it++) {
+            ia[it] = pa[it];
+            asm volatile("" : "+v"(ia[it]));
+        }
+#pragma unroll
+        for (int it = 0; it < ITB; it++) {
+            ib[it] = pb[it];
+            asm volatile("" : "+v"(ib[it]));
+        }
+        const uint32_t mq = __builtin_amdgcn_readfirstlane(smask[q]);
+        char* base = (char*)accp + (size_t)q * slice;
+        // opaque copies of the offsets: loads and stores take the form of a
+        // scalar base and a 32-bit offset
+        uint32_t po[ITB][RB];
+#pragma unroll
+        for (int it = 0; it < ITB; it++)
+#pragma unroll
+            for (int k2 = 0; k2 < RB; k2++) {
+                po[it][k2] = off[it][k2];
+                asm volatile("" : "+v"(po[it][k2]));
+            }
+        // previous values of the cells
+        float prev[ITB][RB];
+#pragma unroll
+        for (int it = 0; it < ITB; it++)
+#pragma unroll
+            for (int k2 = 0; k2 < RB; k2++) prev[it][k2] = 0.f;
+        if (!first) {
+#pragma unroll
+            for (int it = 0; it < ITB; it++)
+#pragma unroll
+                for (int k2 = 0; k2 < RB; k2++) {
+                    // outside the window: the slice's first cell instead, no branch
+                    const uint32_t o = CHUNK && po[it][k2] == ~0u ? 0u : po[it][k2];
+                    prev[it][k2] = *(const float*)(base + o);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        {
+            float2 u[5][5];
+#pragma unroll
+            for (int p2 = 0; p2 < 5; p2++) {
+#pragma unroll
+                for (int p1 = 0; p1 < 5; p1++) {
+                    const int pp = p2 + 5 * p1;
+                    const uint32_t sg = ((mq >> pp) & 1u) << 31;
+                    u[p2][p1] = make_float2(__uint_as_float(__float_as_uint(x[pp].x) ^ sg),
+                                            __uint_as_float(__float_as_uint(x[pp].y) ^ sg));
+                }
+                bfly5<false>(u[p2]);
+#pragma unroll
+                for (int s1 = 1; s1 < 5; s1++)
+                    if (p2) u[p2][s1] = cmulf(u[p2][s1], kW25[s1 * p2]);
+            }
+            float2* dst = lds + c1 * CP + m;
+            if (tid < C * NB) {
+#pragma unroll
+                for (int s1 = 0; s1 < 5; s1++) {
+                    float2 w5[5];
+#pragma unroll
+                    for (int p2 = 0; p2 < 5; p2++) w5[p2] = s1 ? cmulf(u[p2][s1], tw1[s1]) : u[p2][s1];
+                    bfly5<false>(w5);
+#pragma unroll
+                    for (int s2 = 0; s2 < 5; s2++) dst[(s1 + 5 * s2) * RP] = s2 ? cmulf(w5[s2], tw5[s2]) : w5[s2];
+                }
+            }
+        }
+        __syncthreads();
+        // radix RA over m = j + RB i: output i at slot RB i + j, times W_NB^(i j)
+#pragma unroll
+        for (int it = 0; it < ITA; it++) {
+            if (ia[it] != 0xffffffffu) {
+                float2* a = lds + (ia[it] & 0xffffu);
+                const float2* w = stw + RA * (ia[it] >> 16);
+                float2 v[RA], tw[RA];
+#pragma unroll
+                for (int i = 0; i < RA; i++) v[i] = a[RB * i];
+#pragma unroll
+                for (int i = 1; i < RA; i++) tw[i] = w[i];
+                __builtin_amdgcn_sched_barrier(0);
+                dft_reg<RA, false>(v);
+                a[0] = v[0];
+#pragma unroll
+                for (int i = 1; i < RA; i++) a[RB * i] = cmulf(v[i], tw[i]);
+            }
+        }
+        __syncthreads();
+        // radix RB over j of (s, i): raw bins s + 25 (i + RA k2)
+#pragma unroll
+        for (int it = 0; it < ITB; it++) {
+            const bool act = ib[it] != 0xffffffffu;
+            float2 v[RB];
+            const float2* a = lds + (act ? ib[it] : 0u);
+#pragma unroll
+            for (int j = 0; j < RB; j++) v[j] = a[j];
+            __builtin_amdgcn_sched_barrier(0);
+            dft_reg<RB, false>(v);
+            if (act) {
+#pragma unroll
+                for (int k2 = 0; k2 < RB; k2++) {
+                    // muladd(re, re, im * im), the reference's rotation power
+                    const float pw = fmaf(v[k2].x, v[k2].x, __fmul_rn(v[k2].y, v[k2].y));
+                    if (whole || po[it][k2] != ~0u) *(float*)(base + po[it][k2]) = prev[it][k2] + pw;
+                }
+            }
+        }
+        __syncthreads();  // the rows are consumed
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Data-bit search (k_column_sign) of two 20-period bits, ndop = 40 nb: for
 // every edge offset and sign combination the window's two bits are added onto
 // each other, x_e[i] +- x_e[i + 20] at period i < 20, and transformed with

@@ -1188,220 +1188,6 @@ __constant__ float2 kW25[17] = {
     {-0.9921147013144779f, 0.12533323356430429f}, {-0.9297764858882515f, 0.3681245526846779f},
     {-0.8090169943749478f, 0.5877852522924727f}, {-0.6374239897486895f, 0.7705132427757894f}};
 
-// Direct rotation path at ndop = 2000 = 25 nb, nb = 80 (the E1-like search at
-// 25 MHz and the default +-7 kHz): rows n = p nb + m, raw bins w = s + 25 k, as
-// k_column_rotbig below,
-//   X_q[s + 25 k] = sum_m W_80^(k m) W_2000^(s m) sum_p sigma_q[p] W_25^(s p) x[p nb + m].
-// A workgroup owns C = 3 code columns. Thread (column, m) keeps the 25 samples
-// of its lag in registers for all rotations; per rotation it applies the
-// signs (flips of the float sign bit), a 5 x 5 DFT over p and the twiddles,
-// and writes the 25 classes s to LDS. The 80-point transforms of the 3 x 25
-// rows follow as 8 x 10 in place, and the last stage adds the powers to the
-// cells straight from its registers: butterfly (s, i) of a column has rows
-// s + 25 i + 200 k2, so consecutive threads hold consecutive rows of the
-// column-major accumulator. Offsets of the cells stay in registers, and their
-// previous values are read ahead of the rotation's first stage.
-// grid (ceil(bs / 3), nb, batch), 256 threads, 49 KB of LDS.
-// Bound by vector instructions: 2130 per column and rotation against 2600 of
-// the 16 x 5 x 5 x 5 kernel above, 8.5 ms at 100000 columns and R 25 if
-// nothing waited, next to 41.9 GB of cells (8.5 ms at a copy's rate). Three
-// columns make four waves, one per SIMD, and two workgroups per CU leave the
-// 231 registers for all 30 offsets and values: four columns in five waves, two
-// and a half per SIMD with one butterfly's cells ahead, took 14.4 ms
-// and k_column_rot2000 15.1 ms; this takes 10.5 ms per PRN-step.
-#define ROT2000_C 3
-#define ROT2000_NTHR 256
-constexpr int kRot2000Pitch = 81;                 // row of 80 values (odd: lanes along rows spread over the banks)
-constexpr int kRot2000Col = 25 * kRot2000Pitch + 2;  // column: 11 mod 32, so three columns' lanes spread too
-constexpr size_t kRot2000Lds = (size_t)ROT2000_C * kRot2000Col * 8 + 80 * 8;
-
-__global__ void __launch_bounds__(ROT2000_NTHR)
-__attribute__((amdgpu_waves_per_eu(2, 2)))
-k_column_rot25x80(ColumnArgs A)
-{
-    constexpr int N = 2000, NB = 80, P = 25, RA = 8, RB = 10, C = ROT2000_C, NT = ROT2000_NTHR;
-    constexpr int RP = kRot2000Pitch, CP = kRot2000Col;
-    constexpr int ITA = (C * P * RB + NT - 1) / NT, ITB = (C * P * RA + NT - 1) / NT;
-    static_assert(C * NB <= NT && RP >= NB, "work split");
-    extern __shared__ float2 lds[];
-    float2* stw = lds + C * CP;                // W_80^(i j) at [j][i], i < 8, j < 10
-    __shared__ uint32_t smask[64];
-    const int tid = threadIdx.x;
-    const int lbk = xcd_logical_block();
-    const int lb = __builtin_amdgcn_readfirstlane(lbk % gridDim.x);
-    const int r = __builtin_amdgcn_readfirstlane((lbk / gridDim.x) % gridDim.y);
-    const int p = __builtin_amdgcn_readfirstlane(lbk / (gridDim.x * gridDim.y));
-    const int lag0 = lb * C, ncol = min(C, A.bs - lag0);
-    if (tid < NB) stw[tid] = A.twD[P * (tid % RA) * (tid / RA)];
-    if (tid < A.R) {
-        const float* pat = A.patterns + ((size_t)A.pset[A.req[p]] * A.Q + tid) * A.ncoh;
-        uint32_t msk = 0;
-        for (int q = 0; q < P; q++)
-            if (pat[q] < 0.f) msk |= 1u << q;
-        smask[tid] = msk;
-    }
-    // lag m of column c: 25 samples of the column rotated by its alignment
-    // (src/noncoherent_integration.jl:212-215), factors of W_N^(s m), s = s1 + 5 s2
-    const int c1 = tid % C, m = min(tid / C, NB - 1);
-    float2 x[P], tw1[5], tw5[5];
-    {
-        const int lag = lag0 + min(c1, ncol - 1), pc = r * A.bs + lag;
-        const int wrap = ((NB - pc / A.bs) % NB) * A.bs + (pc % A.bs);
-        const int eff = ((wrap + (A.bs >> 1)) / A.bs) % NB;
-        const float2* T = A.tile + (((size_t)p * NB + r) * N) * A.tp + lag;
-#pragma unroll
-        for (int q = 0; q < P; q++) {
-            int src = q * NB + m + eff;
-            if (src >= N) src -= N;
-            // neighbouring workgroups (the next lags) read the same tile lines: plain, cached loads
-            x[q] = T[(size_t)src * A.tp];
-        }
-#pragma unroll
-        for (int i = 1; i < 5; i++) {
-            tw1[i] = A.twD[i * m];
-            tw5[i] = A.twD[5 * i * m];
-        }
-    }
-    float* accp = A.acc + (size_t)p * A.acc_ps;
-    const size_t slice = (size_t)A.spc * A.acc_ldc * 4;  // bytes of a rotation slice (below 2^32)
-    const bool first = A.first_step != 0;
-    // The stages' butterflies (their index arithmetic is full of slow
-    // multiplications). Radix 8: LDS index | j << 16, all ones past the end.
-    // Radix 10: LDS index and the byte offsets of the cells in a slice; it takes
-    // the threads in reverse, so that the remainders of the two stages fall to
-    // different waves.
-    uint32_t pa[ITA], pb[ITB], off[ITB][RB];
-#pragma unroll
-    for (int it = 0; it < ITA; it++) {
-        const uint32_t idx = tid + it * NT, c = idx / (P * RB), b = idx % (P * RB), j = b / P, s = b % P;
-        pa[it] = idx < C * P * RB ? (c * CP + s * RP + j) | j << 16 : 0xffffffffu;
-    }
-#pragma unroll
-    for (int it = 0; it < ITB; it++) {
-        const uint32_t idx = NT - 1 - tid + it * NT, c = idx / (P * RA), b = idx % (P * RA), i = b / P, s = b % P;
-        const bool act = idx < C * P * RA && c < (uint32_t)ncol;
-        pb[it] = act ? c * CP + s * RP + RB * i : 0xffffffffu;
-#pragma unroll
-        for (int k2 = 0; k2 < RB; k2++) {
-            // raw bin b + 200 k2, sorted row (b + 200 k2 + 1000) mod 2000, column + its drift (mod spc)
-            const int row = b + P * RA * ((k2 + RB / 2) % RB);
-            int dc = r * A.bs + lag0 + (act ? (int)c : 0) + A.shifts[row];
-            if (dc >= A.spc) dc -= A.spc;
-            off[it][k2] = ((uint32_t)row + (uint32_t)dc * (uint32_t)A.acc_ldc) * 4u;
-        }
-    }
-    __syncthreads();  // tables and masks
-#pragma unroll 1
-    for (int q = 0; q < A.R; q++) {
-        // opaque copies: what follows from them is not hoisted into registers
-        uint32_t ia[ITA], ib[ITB];
-#pragma unroll
-        for (int it = 0; it < ITA; it++) {
-            ia[it] = pa[it];
-            asm volatile("" : "+v"(ia[it]));
-        }
-#pragma unroll
-        for (int it = 0; it < ITB; it++) {
-            ib[it] = pb[it];
-            asm volatile("" : "+v"(ib[it]));
-        }
-        const uint32_t mq = __builtin_amdgcn_readfirstlane(smask[q]);
-        char* base = (char*)accp + (size_t)q * slice;
-        // opaque copies of the offsets: loads and stores take the form of a
-        // scalar base and a 32-bit offset
-        uint32_t po[ITB][RB];
-#pragma unroll
-        for (int it = 0; it < ITB; it++)
-#pragma unroll
-            for (int k2 = 0; k2 < RB; k2++) {
-                po[it][k2] = off[it][k2];
-                asm volatile("" : "+v"(po[it][k2]));
-            }
-        // previous values of the cells
-        float prev[ITB][RB];
-#pragma unroll
-        for (int it = 0; it < ITB; it++)
-#pragma unroll
-            for (int k2 = 0; k2 < RB; k2++) prev[it][k2] = 0.f;
-        if (!first) {
-#pragma unroll
-            for (int it = 0; it < ITB; it++)
-#pragma unroll
-                for (int k2 = 0; k2 < RB; k2++) prev[it][k2] = *(const float*)(base + po[it][k2]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        {
-            float2 u[5][5];
-#pragma unroll
-            for (int p2 = 0; p2 < 5; p2++) {
-#pragma unroll
-                for (int p1 = 0; p1 < 5; p1++) {
-                    const int pp = p2 + 5 * p1;
-                    const uint32_t sg = ((mq >> pp) & 1u) << 31;
-                    u[p2][p1] = make_float2(__uint_as_float(__float_as_uint(x[pp].x) ^ sg),
-                                            __uint_as_float(__float_as_uint(x[pp].y) ^ sg));
-                }
-                bfly5<false>(u[p2]);
-#pragma unroll
-                for (int s1 = 1; s1 < 5; s1++)
-                    if (p2) u[p2][s1] = cmulf(u[p2][s1], kW25[s1 * p2]);
-            }
-            float2* dst = lds + c1 * CP + m;
-            if (tid < C * NB) {
-#pragma unroll
-                for (int s1 = 0; s1 < 5; s1++) {
-                    float2 w5[5];
-#pragma unroll
-                    for (int p2 = 0; p2 < 5; p2++) w5[p2] = s1 ? cmulf(u[p2][s1], tw1[s1]) : u[p2][s1];
-                    bfly5<false>(w5);
-#pragma unroll
-                    for (int s2 = 0; s2 < 5; s2++) dst[(s1 + 5 * s2) * RP] = s2 ? cmulf(w5[s2], tw5[s2]) : w5[s2];
-                }
-            }
-        }
-        __syncthreads();
-        // radix 8 over m = j + 10 i: output i at slot 10 i + j, times W_80^(i j)
-#pragma unroll
-        for (int it = 0; it < ITA; it++) {
-            if (ia[it] != 0xffffffffu) {
-                float2* a = lds + (ia[it] & 0xffffu);
-                const float2* w = stw + RA * (ia[it] >> 16);
-                float2 v[RA], tw[RA];
-#pragma unroll
-                for (int i = 0; i < RA; i++) v[i] = a[RB * i];
-#pragma unroll
-                for (int i = 1; i < RA; i++) tw[i] = w[i];
-                __builtin_amdgcn_sched_barrier(0);
-                bfly8<false>(v);
-                a[0] = v[0];
-#pragma unroll
-                for (int i = 1; i < RA; i++) a[RB * i] = cmulf(v[i], tw[i]);
-            }
-        }
-        __syncthreads();
-        // radix 10 over j of (s, i): raw bins s + 25 (i + 8 k2)
-#pragma unroll
-        for (int it = 0; it < ITB; it++) {
-            const bool act = ib[it] != 0xffffffffu;
-            float2 v[RB];
-            const float2* a = lds + (act ? ib[it] : 0u);
-#pragma unroll
-            for (int j = 0; j < RB; j++) v[j] = a[j];
-            __builtin_amdgcn_sched_barrier(0);
-            bfly10<false>(v);
-            if (act) {
-#pragma unroll
-                for (int k2 = 0; k2 < RB; k2++) {
-                    // muladd(re, re, im * im), the reference's rotation power
-                    const float pw = fmaf(v[k2].x, v[k2].x, __fmul_rn(v[k2].y, v[k2].y));
-                    *(float*)(base + po[it][k2]) = prev[it][k2] + pw;
-                }
-            }
-        }
-        __syncthreads();  // the rows are consumed
-    }
-}
-
 // ---------------------------------------------------------------------------
 // Reductions: peak with the reference's tie-break order, FP64 row sums.
 // ---------------------------------------------------------------------------
@@ -1772,94 +1558,18 @@ __device__ __forceinline__ void rows_stage_any(int R, float2* rows, int rp, int 
     else rows_stage<5, 2, LAST>(rows, rp, s0, sstep, nr, n, Ns, twR, lane);
 }
 
-// rows_stage with the row length and stage stride as template constants (the
-// row lengths of the E1-like searches, below): the divisions, the twiddle
-// stride and the LDS offsets fold to shifts, multiplies and immediates. The
-// same butterflies on the same data as rows_stage.
-template <int R, int MB, bool LAST, int NB, int NS>
-__device__ __forceinline__ void rows_stage_c(float2* rows, int rp, int s0, int sstep, int nr,
-                                             const float2* __restrict__ twR, int lane)
-{
-    constexpr int m = NB / R;
-    constexpr int tstride = NB / (NS * R);
-    const int total = nr * m;
-    float2 v[MB][R];
-    int orow[MB], obase[MB];
-#pragma unroll
-    for (int b = 0; b < MB; b++) {
-        const int idx = lane + 64 * b;
-        orow[b] = -1;
-        obase[b] = 0;
-        if (idx < total) {
-            const int i = idx / m, j = idx - i * m;
-            const int g = j / NS, k = j - g * NS;
-            const int rb = (s0 + sstep * i) * rp;
-            const float2* a = rows + rb;
-#pragma unroll
-            for (int r = 0; r < R; r++) v[b][r] = a[lds_pad(j + r * m)];
-            if constexpr (NS > 1) {
-#pragma unroll
-                for (int r = 1; r < R; r++) v[b][r] = cmulf(v[b][r], twR[r * tstride * k]);
-            }
-            bfly<R, false>(v[b]);
-            orow[b] = rb;
-            obase[b] = g * NS * R + k;
-        }
-    }
-    wave_lds_sync();
-#pragma unroll
-    for (int b = 0; b < MB; b++) {
-        if (orow[b] >= 0) {
-            if constexpr (LAST) {
-                float* pw = (float*)(rows + orow[b]);
-#pragma unroll
-                for (int r = 0; r < R; r++)
-                    pw[obase[b] + r * NS] = fmaf(v[b][r].x, v[b][r].x, __fmul_rn(v[b][r].y, v[b][r].y));
-            } else {
-#pragma unroll
-                for (int r = 0; r < R; r++) rows[orow[b] + lds_pad(obase[b] + r * NS)] = v[b][r];
-            }
-        }
-    }
-    wave_lds_sync();
-}
-
-// The nb-point row transform at nb = 50, 100, 250, 500 in the runtime plan's
-// radix order (make_row_plan: radix 10 as often as it divides, then 5).
-template <int NB>
-__device__ __forceinline__ void rows_fft_c(float2* rows, int rp, int s0, int sstep, int nr,
-                                           const float2* __restrict__ twR, int lane)
-{
-    static_assert(NB == 50 || NB == 100 || NB == 250 || NB == 500, "compile-time row lengths");
-    if constexpr (NB == 500) {
-        rows_stage_c<10, 1, false, 500, 1>(rows, rp, s0, sstep, nr, twR, lane);
-        rows_stage_c<10, 1, false, 500, 10>(rows, rp, s0, sstep, nr, twR, lane);
-        rows_stage_c<5, 2, true, 500, 100>(rows, rp, s0, sstep, nr, twR, lane);
-    } else if constexpr (NB == 250) {
-        rows_stage_c<10, 1, false, 250, 1>(rows, rp, s0, sstep, nr, twR, lane);
-        rows_stage_c<5, 2, false, 250, 10>(rows, rp, s0, sstep, nr, twR, lane);
-        rows_stage_c<5, 2, true, 250, 50>(rows, rp, s0, sstep, nr, twR, lane);
-    } else if constexpr (NB == 100) {
-        rows_stage_c<10, 1, false, 100, 1>(rows, rp, s0, sstep, nr, twR, lane);
-        rows_stage_c<10, 1, true, 100, 10>(rows, rp, s0, sstep, nr, twR, lane);
-    } else {
-        rows_stage_c<10, 1, false, 50, 1>(rows, rp, s0, sstep, nr, twR, lane);
-        rows_stage_c<5, 2, true, 50, 10>(rows, rp, s0, sstep, nr, twR, lane);
-    }
-}
-
 // CPT: accumulator cells (sorted rows) per thread, ceil(ndop / NT); rgrp:
-// rows a wave transforms together (both checked on the host). NB > 0: the
-// row length nb as a compile-time constant (rows_fft_c); 0: any nb, through
-// the runtime plan prow.
-template <int NT, int CPT, int NB = 0>
+// rows a wave transforms together (both checked on the host). Serves the row
+// lengths that k_column_rot25 has no instance of (10, 25, 125) and more than 64
+// rotations.
+template <int NT, int CPT>
 __global__ void __launch_bounds__(NT)
 k_column_rotbig(ColumnArgs A, FftPlanDev prow, const float2* __restrict__ twR, int rgrp)
 {
     constexpr int NC = 25;
     extern __shared__ float2 lds[];
-    const int N = NB > 0 ? NC * NB : A.ndop, nb = NB > 0 ? NB : A.nb;
-    const int rp = NB > 0 ? NB + (NB >> 4) + 1 : fft_lds_span(nb);  // row pitch
+    const int N = A.ndop, nb = A.nb;
+    const int rp = fft_lds_span(nb);  // row pitch
     float2* rows = lds;
     float2* stw = lds + (size_t)NC * rp;  // row twiddles W_nb^j
     uint32_t* soff = (uint32_t*)(stw + nb);  // cell offset of each sorted row
@@ -1979,16 +1689,12 @@ k_column_rotbig(ColumnArgs A, FftPlanDev prow, const float2* __restrict__ twR, i
         for (int i0 = 0; i0 < nr; i0 += rgrp) {
             const int g = min(rgrp, nr - i0);
             const int s0 = wave + nw * i0;
-            if constexpr (NB > 0) {
-                rows_fft_c<NB>(rows, rp, s0, nw, g, stw, lane);
-            } else {
-                int Ns = 1;
-                for (int st = 0; st + 1 < prow.nst; st++) {
-                    rows_stage_any<false>(prow.radix[st], rows, rp, s0, nw, g, nb, Ns, stw, lane);
-                    Ns *= prow.radix[st];
-                }
-                rows_stage_any<true>(prow.radix[prow.nst - 1], rows, rp, s0, nw, g, nb, Ns, stw, lane);
+            int Ns = 1;
+            for (int st = 0; st + 1 < prow.nst; st++) {
+                rows_stage_any<false>(prow.radix[st], rows, rp, s0, nw, g, nb, Ns, stw, lane);
+                Ns *= prow.radix[st];
             }
+            rows_stage_any<true>(prow.radix[prow.nst - 1], rows, rp, s0, nw, g, nb, Ns, stw, lane);
         }
         __syncthreads();  // every row's powers are ready
         // accumulate the powers of this thread's cells: all sums first, then

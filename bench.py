@@ -65,7 +65,7 @@ def copy_calibration(nbytes: int):
 
 KERNEL_CLASS_OF = {"k_corr_tile": "corr_tile", "k_column_simple": "column", "k_column_sign": "column",
                    "k_column_rotation": "column", "k_column_c160": "column", "k_column_c160_pair": "column",
-                   "k_column_rot2000": "column", "k_column_rot25x80": "column", "k_column_bitsplit": "column",
+                   "k_column_rot2000": "column", "k_column_rot25": "column", "k_column_bitsplit": "column",
                    "k_column_reg": "column",
                    "k_full_corr": "column", "k_full31_corr": "column",
                    "k_column_rotsplit": "column", "k_corr_fc": "corr_tile", "k_fc_signal": "signal_fft",

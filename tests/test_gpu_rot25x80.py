@@ -1,4 +1,4 @@
-"""Direct rotation search at 25 periods of 80 rows (k_column_rot25x80).
+"""Direct rotation search at 25 periods of 80 rows (k_column_rot25 at 80 rows).
 
 E1-like pilots (25-chip secondary code, 4 ms codes) with 80 blocks of 49 to 52
 samples, so that the last workgroup of three code columns holds one to three of
