@@ -737,19 +737,20 @@ int full_create(fmdbzp_plan* P, const int8_t* d_codes)
     return FMDBZP_OK;
 }
 
-// k_secondary_phase by sample type
+// k_secondary_phase by sample type, for requests of up to LP - 1 rotations
 using SecKernel = void (*)(const void*, int, const SecReqDev*, int32_t*);
+template <int LP>
 SecKernel secondary_kernel(int eltype)
 {
     switch (eltype) {
-    case FMDBZP_CF32: return k_secondary_phase<FMDBZP_CF32>;
-    case FMDBZP_CF64: return k_secondary_phase<FMDBZP_CF64>;
-    case FMDBZP_I16: return k_secondary_phase<FMDBZP_I16>;
-    case FMDBZP_CI8: return k_secondary_phase<FMDBZP_CI8>;
-    case FMDBZP_CI16: return k_secondary_phase<FMDBZP_CI16>;
-    case FMDBZP_F32: return k_secondary_phase<FMDBZP_F32>;
-    case FMDBZP_F64: return k_secondary_phase<FMDBZP_F64>;
-    default: return k_secondary_phase<FMDBZP_C2BIT>;
+    case FMDBZP_CF32: return k_secondary_phase<FMDBZP_CF32, LP>;
+    case FMDBZP_CF64: return k_secondary_phase<FMDBZP_CF64, LP>;
+    case FMDBZP_I16: return k_secondary_phase<FMDBZP_I16, LP>;
+    case FMDBZP_CI8: return k_secondary_phase<FMDBZP_CI8, LP>;
+    case FMDBZP_CI16: return k_secondary_phase<FMDBZP_CI16, LP>;
+    case FMDBZP_F32: return k_secondary_phase<FMDBZP_F32, LP>;
+    case FMDBZP_F64: return k_secondary_phase<FMDBZP_F64, LP>;
+    default: return k_secondary_phase<FMDBZP_C2BIT, LP>;
     }
 }
 
@@ -1407,10 +1408,12 @@ int fmdbzp_secondary_phase(fmdbzp_plan* plan, const void* signal, int32_t eltype
         rq[(size_t)i].L = reqs[i].num_rotations;
         rq[(size_t)i].pad = 0;
     }
-    size_t lds_bytes = 0;
-    for (int i = 0; i < nreq; i++) lds_bytes = std::max(lds_bytes, sec_lds(reqs[i].num_rotations));
+    const SecKernel kernel = Lmax <= 16   ? secondary_kernel<17>(eltype)
+                             : Lmax <= 32 ? secondary_kernel<33>(eltype)
+                                          : secondary_kernel<65>(eltype);
+    const size_t lds_bytes = Lmax <= 16 ? sec_lds(17) : Lmax <= 32 ? sec_lds(33) : sec_lds(65);
     {
-        const int rc = set_lds_attr((const void*)secondary_kernel(eltype), lds_bytes);
+        const int rc = set_lds_attr((const void*)kernel, lds_bytes);
         if (rc) return rc;
     }
     hipError_t e = hipSuccess;
@@ -1419,7 +1422,7 @@ int fmdbzp_secondary_phase(fmdbzp_plan* plan, const void* signal, int32_t eltype
     if (e == hipSuccess) e = hipMemcpy(d_secs, secs.data(), secs.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(d_reqs, rq.data(), sizeof(SecReqDev) * (size_t)nreq, hipMemcpyHostToDevice);
     if (e == hipSuccess) {
-        secondary_kernel(eltype)<<<nreq, FMDBZP_SEC_NTHR, lds_bytes, plan->stream>>>(
+        kernel<<<nreq, FMDBZP_SEC_NTHR, lds_bytes, plan->stream>>>(
             dev_sig ? signal : plan->d_signal, spc, d_reqs, d_out);
         e = hipGetLastError();
     }

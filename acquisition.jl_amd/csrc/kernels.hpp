@@ -2358,12 +2358,18 @@ k_export_cm(const float* __restrict__ acc, float* __restrict__ out, int ndop, in
 //
 // Two chains are serial by that definition: the phasor of a period (two
 // dependent operations per sample) and its sum (one add). Everything else is
-// not, so the workgroup is a pipeline over chunks of C samples, all periods at
+// not, so the workgroup is a pipeline over chunks of 64 samples, all periods at
 // once, one barrier per chunk: wave 0 writes the phasors of chunk i to LDS
 // (lane = period), waves 2-7 form the despread products of chunk i - 1 and
-// load the samples of chunk i (lanes along samples: coalesced), wave 1 sums
-// chunk i - 2 (lane = period). The phasor chain bounds it. C is 64 up to 32
-// periods and 32 above, so the four LDS buffers stay within 66 KB.
+// load the samples of chunk i (lane = sample, wave 2 + g has the periods g,
+// g + 6, ...), wave 1 sums chunk i - 2 (lane = period). The loop runs two chunks
+// per turn with the samples in two register sets: moving them from one to the
+// other waited for the loads of the chunk just begun. The LDS pitch LP, odd and
+// above the largest L of the launch, is a constant, so that the chains' LDS
+// accesses carry their offsets; the four buffers take 35 to 133 KB. Bound by the
+// phasor chain (20 ns a sample on one wave): 10 periods of 30690 samples take
+// 684 us, 25 of 100000 2.06 ms (842 us and 2.37 ms with the samples moved and a
+// pitch of the request's L; chunks of 4096 products took 762 us and 3.77 ms).
 struct SecReqDev {
     const int8_t* code;  // spc samples at the estimated code phase
     const int8_t* sec;   // L secondary chips
@@ -2372,27 +2378,24 @@ struct SecReqDev {
     int pad;
 };
 #define FMDBZP_SEC_NTHR 512
-__host__ __device__ __forceinline__ int sec_chunk(int L) { return L <= 32 ? 64 : 32; }
-__host__ __device__ __forceinline__ int sec_pitch(int L) { return L | 1; }  // odd: lanes along samples spread over the banks
-__host__ __device__ __forceinline__ size_t sec_lds(int L)
-{
-    return (size_t)4 * sec_chunk(L) * sec_pitch(L) * sizeof(float2);
-}
-template <int ELT>
+#define FMDBZP_SEC_C 64
+__host__ __device__ constexpr size_t sec_lds(int LP) { return (size_t)4 * FMDBZP_SEC_C * LP * sizeof(float2); }
+// LP: 17, 33 or 65, L < LP
+template <int ELT, int LP>
 __global__ void __launch_bounds__(FMDBZP_SEC_NTHR)
 k_secondary_phase(const void* __restrict__ sig, int spc, const SecReqDev* __restrict__ reqs,
                   int32_t* __restrict__ out)
 {
 #pragma clang fp contract(off)
-    constexpr int NPT = FMDBZP_SEC_NTHR - 128;        // product threads
-    constexpr int NI = (64 * 32 + NPT - 1) / NPT;     // products per thread and chunk (C L <= 2048)
+    constexpr int C = FMDBZP_SEC_C, G = FMDBZP_SEC_NTHR / 64 - 2, NI = (LP - 1 + G - 1) / G;
     const SecReqDev R = reqs[blockIdx.x];
     extern __shared__ float2 lds[];
     __shared__ float zr[64], zi[64], mags[64];
-    const int tid = threadIdx.x, wave = tid >> 6, k = tid & 63;
-    const int L = R.L, C = sec_chunk(L), Lp = sec_pitch(L), lc = C == 64 ? 6 : 5;
-    float2* ph = lds;              // [2][C][Lp] phasors
-    float2* qq = lds + 2 * C * Lp; // [2][C][Lp] despread products
+    const int tid = threadIdx.x, k = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int L = R.L;
+    float2* ph = lds;              // [2][C][LP] phasors
+    float2* qq = lds + 2 * C * LP; // [2][C][LP] despread products
     const int nch = (spc + C - 1) / C;
     // wave 0: phasor of period k
     float cr = 1.0f, ci = 0.0f, dre = 1.0f, dim = 0.0f;
@@ -2404,68 +2407,72 @@ k_secondary_phase(const void* __restrict__ sig, int spc, const SecReqDev* __rest
         dim = (float)sin(R.phase_step);
     }
     float ar = 0.0f, ai = 0.0f;  // wave 1: sum of period k
-    float2 xs[NI];
-    float cs[NI];
-    for (int i = 0; i < nch + 2; i++) {
+    // product waves: samples of periods g + G u and the code, one set per chunk parity
+    float2 x0[NI], x1[NI];
+    int8_t c0 = 0, c1 = 0;
+    auto step = [&](int i, float2(&xn)[NI], int8_t& cn, const float2(&xs)[NI], const int8_t& cs) {
         if (wave == 0) {
             if (i < nch && k < L) {
-                float2* p = ph + (i & 1) * C * Lp + k;
-                const int m = min(C, spc - i * C);
-#pragma unroll 8
-                for (int n = 0; n < m; n++) {
-                    p[n * Lp] = make_float2(cr, ci);
+                float2* p = ph + (i & 1) * C * LP + k;
+                auto next = [&](int n) {
+                    p[n * LP] = make_float2(cr, ci);
                     const float ncr = cr * dre - ci * dim, nci = cr * dim + ci * dre;
                     cr = ncr;
                     ci = nci;
-                }
+                };
+                const int m = min(C, spc - i * C);
+                if (m == C) {
+#pragma unroll 16
+                    for (int n = 0; n < C; n++) next(n);
+                } else
+                    for (int n = 0; n < m; n++) next(n);
             }
         } else if (wave == 1) {
             if (i >= 2 && k < L) {
-                const float2* q = qq + (i & 1) * C * Lp + k;
+                const float2* q = qq + (i & 1) * C * LP + k;
                 const int m = min(C, spc - (i - 2) * C);
-#pragma unroll 8
-                for (int n = 0; n < m; n++) {
-                    const float2 v = q[n * Lp];
-                    ar += v.x;
-                    ai += v.y;
-                }
+                if (m == C) {
+#pragma unroll 16
+                    for (int n = 0; n < C; n++) {
+                        const float2 v = q[n * LP];
+                        ar += v.x;
+                        ai += v.y;
+                    }
+                } else
+                    for (int n = 0; n < m; n++) {
+                        const float2 v = q[n * LP];
+                        ar += v.x;
+                        ai += v.y;
+                    }
             }
         } else {
-            const int t = tid - 128;
-            float2 nx[NI];
-            float nc[NI];
+            const int g = wave - 2;
             if (i < nch) {
+                const int n = min(i * C + k, spc - 1);
+                cn = R.code[n];
 #pragma unroll
-                for (int u = 0; u < NI; u++) {
-                    const int e = min(t + NPT * u, C * L - 1);
-                    const int n = min(i * C + (e & (C - 1)), spc - 1), kk = e >> lc;
-                    nx[u] = load_sample(sig, ELT, (int64_t)kk * spc + n);
-                    nc[u] = (float)R.code[n];
-                }
+                for (int u = 0; u < NI; u++)
+                    if (g + G * u < L) xn[u] = load_sample(sig, ELT, (int64_t)(g + G * u) * spc + n);
             }
             if (i >= 1 && i <= nch) {
-                const int o = ((i - 1) & 1) * C * Lp;
+                const int at = ((i - 1) & 1) * C * LP + k * LP + g;
+                const float c = (float)cs;
 #pragma unroll
-                for (int u = 0; u < NI; u++) {
-                    const int e = t + NPT * u;
-                    if (e < C * L) {
-                        const int at = o + (e & (C - 1)) * Lp + (e >> lc);
-                        const float2 x = xs[u], w = ph[at];
+                for (int u = 0; u < NI; u++)
+                    if (g + G * u < L) {
+                        const float2 x = xs[u], w = ph[at + G * u];
                         const float pr = x.x * w.x - x.y * w.y, pim = x.x * w.y + x.y * w.x;
-                        const float c = cs[u];
-                        qq[at] = make_float2(pr * c - pim * 0.0f, pr * 0.0f + pim * c);
+                        qq[at + G * u] = make_float2(pr * c - pim * 0.0f, pr * 0.0f + pim * c);
                     }
-                }
-            }
-            if (i < nch) {
-#pragma unroll
-                for (int u = 0; u < NI; u++) {
-                    xs[u] = nx[u];
-                    cs[u] = nc[u];
-                }
             }
         }
         __syncthreads();
+    };
+#pragma unroll
+    for (int u = 0; u < NI; u++) x0[u] = x1[u] = make_float2(0.f, 0.f);
+    for (int i = 0; i < nch + 2; i += 2) {
+        step(i, x0, c0, x1, c1);
+        step(i + 1, x1, c1, x0, c0);  // past the last chunk: nothing but the barrier
     }
     if (wave == 1 && k < L) {
         zr[k] = ar;

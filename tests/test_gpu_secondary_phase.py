@@ -1,8 +1,8 @@
 """Secondary-code phase kernel (fmdbzp_secondary_phase) at the edges of its chunks.
 
-The kernel runs the periods of a request in chunks of 64 samples (32 above 32
-periods), so its edges are chunk remainders (spc = 2046, 2048, 2500), one
-period, 32, 33 and 64 periods, and requests of different length in one launch.
+The kernel runs the periods of a request in chunks of 64 samples, with instances
+for up to 16, 32 and 64 periods, so its edges are chunk remainders (spc = 2046,
+2048, 2500), one period, 32, 33 and 64 periods, and requests of different length in one launch.
 On white noise the rotations' scores lie close together, so a wrong or missing
 sample moves the best one. The bar: the oracle's rotation
 (src/acquire.jl:503-538), exactly: the kernel keeps the order of operations.
