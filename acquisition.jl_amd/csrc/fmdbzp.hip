@@ -1018,9 +1018,9 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         }
     }
     // the matrix-core form of the E1-like search (nb = 25 n1, n1 = 2, 4, 10, 20);
-    // FMDBZP_PREC_AUTO takes it where it is the faster kernel (n1 = 10, 20:
-    // at n1 = 2 and 4 the FP32 kernel's transforms are short and both run at
-    // the same speed)
+    // FMDBZP_PREC_AUTO takes it at n1 = 10 and 20, its documented choice (47.7
+    // and 109 ms per PRN-step at 25 MHz; k_column_rotbig took 55.6 and 132
+    // there, k_column_rot25 takes 32.3 and 72 in FP32)
     if ((d.precision == FMDBZP_PREC_MFMA || d.precision == FMDBZP_PREC_AUTO) && P->rotbig && nb % 25 == 0 &&
         ndop == 25 * nb &&
         (nb / 25 == 2 || nb / 25 == 4 || nb / 25 == 10 || nb / 25 == 20) && d.num_secondary_rotations <= 32 &&

@@ -84,7 +84,7 @@ enum fmdbzp_precision {
     FMDBZP_PREC_TILE_FP16 = 1,
     /* Per call: FMDBZP_PREC_TILE_FP16 when the plan admits it and the samples
      * are integers, FMDBZP_PREC_MFMA on the plans that admit it with n1 = 10
-     * or 20 (where it is the faster form), else FP32; never rejected. For
+     * or 20, else FP32; never rejected. For
      * batches of requests whose plans and sample types differ. */
     FMDBZP_PREC_AUTO = 2,
     /* Mixed, on matrix cores: the column Doppler transforms of the secondary-
