@@ -147,6 +147,7 @@ EXPORTED_SYMBOLS = (
     "fmdbzp_plan_graph_counts",
     "fmdbzp_plan_tuning",
     "fmdbzp_plan_column_kernel",
+    "fmdbzp_plan_call_kernels",
     "fmdbzp_plan_kernel_times",
     "fmdbzp_synthesize",
     "fmdbzp_plan_set_surface_layout",
@@ -200,6 +201,10 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
     if hasattr(lib, "fmdbzp_plan_column_kernel"):
         lib.fmdbzp_plan_column_kernel.argtypes = [P, ctypes.c_char_p, ctypes.c_size_t]
         lib.fmdbzp_plan_column_kernel.restype = ctypes.c_int
+    if hasattr(lib, "fmdbzp_plan_call_kernels"):
+        lib.fmdbzp_plan_call_kernels.argtypes = [P, ctypes.c_int32, ctypes.c_int32, ctypes.c_uint32, ctypes.c_char_p,
+                                                 ctypes.c_size_t]
+        lib.fmdbzp_plan_call_kernels.restype = ctypes.c_int
     return lib
 
 
@@ -343,9 +348,17 @@ class NativePlan:
         return buf.value.decode()
 
     def column_kernel(self) -> str:
-        """Name of the kernel running this plan's column stage."""
+        """Form of this plan's column stage on the tile."""
         buf = ctypes.create_string_buffer(128)
         _check(lib().fmdbzp_plan_column_kernel(self.handle, buf, len(buf)), "fmdbzp_plan_column_kernel")
+        return buf.value.decode()
+
+    def call_kernels(self, eltype: int, nreq: int, flags: int = 0) -> str:
+        """Kernels that a call over `nreq` PRNs launches for the search: the
+        full-period correlation, or block correlation and column kernel."""
+        buf = ctypes.create_string_buffer(160)
+        _check(lib().fmdbzp_plan_call_kernels(self.handle, eltype, int(nreq), flags, buf, len(buf)),
+               "fmdbzp_plan_call_kernels")
         return buf.value.decode()
 
     def graph_counts(self):

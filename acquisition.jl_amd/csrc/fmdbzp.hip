@@ -737,6 +737,40 @@ int full_create(fmdbzp_plan* P, const int8_t* d_codes)
     return FMDBZP_OK;
 }
 
+bool int_samples(int32_t eltype)
+{
+    return eltype == FMDBZP_I16 || eltype == FMDBZP_CI8 || eltype == FMDBZP_CI16 || eltype == FMDBZP_C2BIT;
+}
+
+// Whether a call runs the full-period correlation: not with surfaces (their
+// time is the copy to the caller, and the tile path's column kernels stay the
+// ones that write them), nor where FMDBZP_PREC_AUTO takes the FP16 tile.
+bool full_call(const fmdbzp_plan* P, int32_t eltype, bool store)
+{
+    return P->full && !store && !(P->tile_auto && int_samples(eltype));
+}
+
+// Column-stage form of the plan on the tile (fmdbzp_plan_column_kernel).
+void column_name(const fmdbzp_plan* P, char* buf, size_t buflen)
+{
+    static const char* const rotmma[] = {"k_column_rotmma<2,1,2>", "k_column_rotmma<4,1,4>",
+                                         "k_column_rotmma<4,3,10>", "k_column_rotmma<8,3,20>"};
+    char tmp[64];
+    const char* name = tmp;
+    if (P->rotmma) name = rotmma[P->rotmma == 2 ? 0 : P->rotmma == 4 ? 1 : P->rotmma == 10 ? 2 : 3];
+    else if (P->rotbig) snprintf(tmp, sizeof tmp, "k_column_rotbig<%d,25>", P->rotbig_nt);
+    else if (P->rot2000) name = "k_column_rot2000";
+    else if (P->rotsplit) snprintf(tmp, sizeof tmp, "k_column_rotsplit<%d,%d>", P->d.num_coh, P->d.num_blocks);
+    else if (P->col_pair) name = P->tile_half ? "k_column_c160_pair<32,512,fp16>" : "k_column_c160_pair<32,512>";
+    else if (P->col_static) name = P->tile_half ? "k_column_c160<32,512,fp16>" : "k_column_c160<32,512>";
+    else if (P->col_reg) snprintf(tmp, sizeof tmp, "k_column_reg<%d>", P->d.num_doppler_bins);
+    else if (P->simple_kernel) name = P->col_onebuf ? "k_column_simple<onebuf>" : "k_column_simple";
+    else if (P->d.path == FMDBZP_PATH_ROTATION) name = "k_column_rotation";
+    else if (P->bitsplit) snprintf(tmp, sizeof tmp, "k_column_bitsplit<%d>", P->d.num_blocks);
+    else name = "k_column_sign";
+    snprintf(buf, buflen, "%s", name);
+}
+
 // k_secondary_phase by sample type, for requests of up to LP - 1 rotations
 using SecKernel = void (*)(const void*, int, const SecReqDev*, int32_t*);
 template <int LP>
@@ -1495,23 +1529,34 @@ int fmdbzp_plan_column_kernel(fmdbzp_plan* plan, char* buf, size_t buflen)
 {
     if (!plan) return set_err(FMDBZP_EHANDLE, "null plan");
     if (!buf || buflen == 0) return set_err(FMDBZP_EINVAL, "null buffer");
+    column_name(plan, buf, buflen);
+    return FMDBZP_OK;
+}
+
+int fmdbzp_plan_call_kernels(fmdbzp_plan* plan, int32_t eltype, int32_t nreq, uint32_t flags, char* buf, size_t buflen)
+{
+    g_err.clear();
+    if (!plan) return set_err(FMDBZP_EHANDLE, "null plan");
+    if (!buf || buflen == 0) return set_err(FMDBZP_EINVAL, "null buffer");
+    if (nreq <= 0) return set_err(FMDBZP_EINVAL, "nreq must be positive");
+    if (!elsize(eltype) && eltype != FMDBZP_C2BIT) return set_err(FMDBZP_EINVAL, "unknown eltype %d", eltype);
+    std::lock_guard<std::mutex> lk(plan->mu);
     const fmdbzp_plan* P = plan;
-    static const char* const rotmma[] = {"k_column_rotmma<2,1,2>", "k_column_rotmma<4,1,4>",
-                                         "k_column_rotmma<4,3,10>", "k_column_rotmma<8,3,20>"};
-    char tmp[64];
-    const char* name = tmp;
-    if (P->rotmma) name = rotmma[P->rotmma == 2 ? 0 : P->rotmma == 4 ? 1 : P->rotmma == 10 ? 2 : 3];
-    else if (P->rotbig) snprintf(tmp, sizeof tmp, "k_column_rotbig<%d,25>", P->rotbig_nt);
-    else if (P->rot2000) name = "k_column_rot2000";
-    else if (P->rotsplit) snprintf(tmp, sizeof tmp, "k_column_rotsplit<%d,%d>", P->d.num_coh, P->d.num_blocks);
-    else if (P->col_pair) name = P->tile_half ? "k_column_c160_pair<32,512,fp16>" : "k_column_c160_pair<32,512>";
-    else if (P->col_static) name = P->tile_half ? "k_column_c160<32,512,fp16>" : "k_column_c160<32,512>";
-    else if (P->col_reg) snprintf(tmp, sizeof tmp, "k_column_reg<%d>", P->d.num_doppler_bins);
-    else if (P->simple_kernel) name = P->col_onebuf ? "k_column_simple<onebuf>" : "k_column_simple";
-    else if (P->d.path == FMDBZP_PATH_ROTATION) name = "k_column_rotation";
-    else if (P->bitsplit) snprintf(tmp, sizeof tmp, "k_column_bitsplit<%d>", P->d.num_blocks);
-    else name = "k_column_sign";
-    snprintf(buf, buflen, "%s", name);
+    if (full_call(P, eltype, (flags & FMDBZP_FLAG_STORE_SURFACES) != 0)) {
+        if (P->fp31.n) snprintf(buf, buflen, "k_full31_corr<%d>", P->full_nthr);
+        else snprintf(buf, buflen, "k_full_corr<%d,%s>", P->full_nthr, P->d.num_noncoherent > 1 ? "true" : "false");
+        return FMDBZP_OK;
+    }
+    const char* half = P->tile_half || (P->tile_auto && int_samples(eltype)) ? ",fp16" : "";
+    static const char* const corr_of[] = {"1,false", "1,true", "2,true", "2,true,2048", "1,true,2500", "2,true,500",
+                                          "10,true,400", "5,true,800", "2,true,2000", "1,true,4000"};
+    char corr[64], col[64];
+    if (P->corr_variant == 10) snprintf(corr, sizeof corr, "k_corr_fc<%d%s>", P->fc_nthr, half);
+    else snprintf(corr, sizeof corr, "k_corr_tile<%s%s>", corr_of[P->corr_variant], half);
+    if (P->rot25 && !P->rotmma) snprintf(col, sizeof col, "k_column_rot25<%d>", P->d.num_blocks);
+    else if (P->col_static) snprintf(col, sizeof col, "k_column_c160%s<32,512%s>", P->col_pair ? "_pair" : "", half);
+    else column_name(P, col, sizeof col);
+    snprintf(buf, buflen, "%s %s", corr, col);
     return FMDBZP_OK;
 }
 
@@ -1614,19 +1659,6 @@ struct Work {
 
 int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t eltype, double interm_freq_hz,
                    int32_t nreq, uint32_t flags, float* const* out_surfaces);
-
-bool int_samples(int32_t eltype)
-{
-    return eltype == FMDBZP_I16 || eltype == FMDBZP_CI8 || eltype == FMDBZP_CI16 || eltype == FMDBZP_C2BIT;
-}
-
-// Whether a call runs the full-period correlation: not with surfaces (their
-// time is the copy to the caller, and the tile path's column kernels stay the
-// ones that write them), nor where FMDBZP_PREC_AUTO takes the FP16 tile.
-bool full_call(const fmdbzp_plan* P, int32_t eltype, bool store)
-{
-    return P->full && !store && !(P->tile_auto && int_samples(eltype));
-}
 
 // Enqueue one search on the plan's stream; statistics land in the plan's
 // pinned staging buffer and are returned by acquire_finish. The caller holds

@@ -1560,7 +1560,7 @@ __device__ __forceinline__ void rows_stage_any(int R, float2* rows, int rp, int 
 
 // CPT: accumulator cells (sorted rows) per thread, ceil(ndop / NT); rgrp:
 // rows a wave transforms together (both checked on the host). Serves the row
-// lengths that k_column_rot25 has no instance of (10, 25, 125) and more than 64
+// lengths that k_column_rot25 has no instance of (10 rows) and more than 64
 // rotations.
 template <int NT, int CPT>
 __global__ void __launch_bounds__(NT)

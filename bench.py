@@ -174,6 +174,7 @@ def _run_c5_group(grp, precision, timing):
     sub-submissions when the plans would not fit device memory together.
     Returns (seconds, results per request, kernel times per plan geometry)."""
     from acquisition import acquire_batch, plan_acquire
+    from acquisition._native import ELTYPE
 
     budget = C5_WORKSPACE_GB * 2**30
     subs, cur, cur_b = [], [], 0.0
@@ -220,7 +221,8 @@ def _run_c5_group(grp, precision, timing):
     for k, (pl, kt) in ktimes.items():
         ktimes[k] = ({"ndop": pl.num_doppler_bins, "spc": pl.samples_per_code, "nb": pl.num_blocks,
                       "bs": pl.block_size, "F": pl.fft_size, "R": pl.num_secondary_rotations,
-                      "nnc": pl.num_noncoherent_accumulations, "kernel": pl.native.column_kernel()}, kt)
+                      "nnc": pl.num_noncoherent_accumulations,
+                      "kernel": pl.native.call_kernels(ELTYPE["cf32"], 1).split()[-1]}, kt)
         pl.close()
     return tot, results, ktimes
 

@@ -347,11 +347,21 @@ int fmdbzp_plan_set_timing(fmdbzp_plan* plan, int32_t enable);
 int fmdbzp_plan_tuning(fmdbzp_plan* plan, char* buf, size_t buflen);
 /* Graphs captured and replayed by a FMDBZP_OPT_GRAPH plan so far. */
 int fmdbzp_plan_graph_counts(fmdbzp_plan* plan, int64_t* captures, int64_t* replays);
-/* Name of the kernel that runs the plan's column stage on the coherent tile
- * (the column Doppler transforms, sign or rotation search and accumulation), e.g.
- * "k_column_rotmma<8,3,20>". No counterpart in the reference (which has one
- * CPU implementation); for tests and reports. */
+/* Form of the column stage that the plan selects on the coherent tile (the
+ * column Doppler transforms, sign or rotation search and accumulation), by the
+ * name of a kernel, e.g. "k_column_rotmma<8,3,20>". A form keeps its name where
+ * a later kernel serves part of its geometries: k_column_rot2000 and
+ * k_column_rotbig are also the forms of the searches that k_column_rot25 runs.
+ * fmdbzp_plan_call_kernels names the kernels themselves. No counterpart in the
+ * reference (which has one CPU implementation); for tests and reports. */
 int fmdbzp_plan_column_kernel(fmdbzp_plan* plan, char* buf, size_t buflen);
+/* Kernels that a call of fmdbzp_acquire with these samples, PRN count and flags
+ * launches for the search: the full-period correlation ("k_full31_corr<512>"),
+ * or the block correlation and the column kernel, separated by a space
+ * ("k_corr_tile<1,true,2500> k_column_rot25<80>"; ",fp16" with an FP16 tile).
+ * No counterpart in the reference; for tests and reports. */
+int fmdbzp_plan_call_kernels(fmdbzp_plan* plan, int32_t eltype, int32_t nreq, uint32_t flags, char* buf,
+                             size_t buflen);
 int fmdbzp_plan_kernel_times(fmdbzp_plan* plan, double* total_ms, int64_t* launches, int32_t n);
 
 /*
