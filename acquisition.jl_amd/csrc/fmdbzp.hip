@@ -742,12 +742,22 @@ bool int_samples(int32_t eltype)
     return eltype == FMDBZP_I16 || eltype == FMDBZP_CI8 || eltype == FMDBZP_CI16 || eltype == FMDBZP_C2BIT;
 }
 
-// Whether a call runs the full-period correlation: not with surfaces (their
-// time is the copy to the caller, and the tile path's column kernels stay the
-// ones that write them), nor where FMDBZP_PREC_AUTO takes the FP16 tile.
-bool full_call(const fmdbzp_plan* P, int32_t eltype, bool store)
+// Whether a call over nreq PRNs runs the full-period correlation: not with
+// surfaces (their time is the copy to the caller, and the tile path's column
+// kernels stay the ones that write them), nor where FMDBZP_PREC_AUTO takes the
+// FP16 tile, nor with few rows of long periods: a row is one workgroup there,
+// and up to 32 of them leave most of the device idle over 13 to 18 us of
+// transform per step, where the tile's kernels split every row. Call times at 20 MHz
+// in us, full-period and tile: 16 rows 73 / 65 (one step), 208 / 161 (8 steps);
+// 32 rows 74 / 70, 208 / 181; 48 rows 76 / 74, 210 / 200; at 16.384 MHz 16 rows
+// 66 / 60, 156 / 145; 32 rows 67 / 63, 158 / 159; at 15 MHz 20 rows 65 / 67, 151 / 209.
+// The 31-axis form is the faster one from two steps on (16.368 MHz, 16 rows: 67 / 60, 141 / 149).
+bool full_call(const fmdbzp_plan* P, int32_t eltype, int32_t nreq, bool store)
 {
-    return P->full && !store && !(P->tile_auto && int_samples(eltype));
+    if (!P->full || store || (P->tile_auto && int_samples(eltype))) return false;
+    const bool several = P->d.num_noncoherent > 1;
+    const int64_t rows = (int64_t)P->d.num_doppler_bins * nreq;
+    return !(P->d.samples_per_code > 15360 && rows < (several ? 33 : 32) && !(several && P->fp31.n));
 }
 
 // Column-stage form of the plan on the tile (fmdbzp_plan_column_kernel).
@@ -1542,7 +1552,7 @@ int fmdbzp_plan_call_kernels(fmdbzp_plan* plan, int32_t eltype, int32_t nreq, ui
     if (!elsize(eltype) && eltype != FMDBZP_C2BIT) return set_err(FMDBZP_EINVAL, "unknown eltype %d", eltype);
     std::lock_guard<std::mutex> lk(plan->mu);
     const fmdbzp_plan* P = plan;
-    if (full_call(P, eltype, (flags & FMDBZP_FLAG_STORE_SURFACES) != 0)) {
+    if (full_call(P, eltype, nreq, (flags & FMDBZP_FLAG_STORE_SURFACES) != 0)) {
         if (P->fp31.n) snprintf(buf, buflen, "k_full31_corr<%d>", P->full_nthr);
         else snprintf(buf, buflen, "k_full_corr<%d,%s>", P->full_nthr, P->d.num_noncoherent > 1 ? "true" : "false");
         return FMDBZP_OK;
@@ -1729,7 +1739,7 @@ int acquire_enqueue(fmdbzp_plan* P, const void* signal, int32_t eltype, int64_t 
     if (store && !P->d_export && !(flags & FMDBZP_FLAG_DEVICE_OUTPUT))
         HIP_TRY(hipMalloc((void**)&P->d_export, sizeof(float) * (size_t)ndop * surf_cols * kLanes));
 
-    if (!full_call(P, eltype, store)) {
+    if (!full_call(P, eltype, nreq, store)) {
         const int rc = ensure_tile(P);
         if (rc) return rc;
     }
@@ -2011,7 +2021,7 @@ int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t elt
     const int spc = d.samples_per_code, spc_eff = d.samples_per_code_eff, nnc = d.num_noncoherent;
     const int64_t seglen = (int64_t)d.num_coh * spc;
     const size_t surf_cols = P->surf_bins > 0 ? (size_t)P->surf_bins : (size_t)spc_eff;
-    if (full_call(P, eltype, store)) return launch_full(P, W, d_sig, eltype, interm_freq_hz, nreq);
+    if (full_call(P, eltype, nreq, store)) return launch_full(P, W, d_sig, eltype, interm_freq_hz, nreq);
 
     // 1. downconvert + double-block FFTs of every segment
     {

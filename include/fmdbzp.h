@@ -128,9 +128,10 @@ enum fmdbzp_precision {
 /* Run every call of a simple-path plan on the coherent tile (block correlation,
  * then the column stage). By default calls that return statistics only run the
  * full-period correlation where the plan admits it (one circular correlation
- * of the code period per Doppler row, no tile); calls with surfaces run on the
- * tile either way. For measuring the tile kernels. Results agree to FP32
- * rounding. No counterpart in the reference. */
+ * of the code period per Doppler row, no tile); calls with surfaces, and calls
+ * of few Doppler rows over all their PRNs at long code periods, run on the
+ * tile either way (fmdbzp_plan_call_kernels tells). For measuring the tile
+ * kernels. Results agree to FP32 rounding. No counterpart in the reference. */
 #define FMDBZP_OPT_TILE_PATH 0x10
 
 /* fmdbzp_acquire flags */
