@@ -280,6 +280,7 @@ struct fmdbzp_plan {
     FftPlanDev pf8{};  // F-point plan without radix 16 (forward signal / code FFTs: fewer live inputs per thread)
     float2* d_twF = nullptr;
     float2* d_twD = nullptr;
+    char* d_arena = nullptr;     // one allocation: code FFTs, signal FFTs, tiles, accumulator, code spectra
     float2* d_prnconj = nullptr;
     float* d_patterns = nullptr;
     int32_t* d_pset = nullptr;
@@ -287,9 +288,9 @@ struct fmdbzp_plan {
     // workspace
     void* d_signal = nullptr;
     size_t signal_cap = 0;
+    int8_t* d_codes = nullptr;   // code samples, during creation
     float2* d_sigfft = nullptr;
     float2* d_tile = nullptr;
-    size_t tile_elems = 0;
     float2* d_tile2 = nullptr;   // second step's tile of a two-step column launch (col_pair)
     float* d_acc = nullptr;
     double* d_rowsum = nullptr;
@@ -338,13 +339,13 @@ struct fmdbzp_plan {
     int fc_nthr = 0;
     size_t fc_lds = 0;
     float2* d_fc_tw = nullptr;
-    // full-period correlation (full_corr.hpp): statistics-only calls of simple
-    // plans; the tile, if other calls need it, is allocated by the first of them
+    // full-period correlation (full_corr.hpp): statistics-only calls of simple plans
     bool full = false;
     FullPlanDev fp{};
     Full31Dev fp31{};                // the chip-rate multiples' form (fp31.n != 0)
     int full_nthr = 0;
     size_t full_lds = 0;
+    std::vector<float2> full_tw;
     float2* d_full_tw = nullptr;
     float2* d_full_code = nullptr;   // [nprn][ndop][spc] code spectra
     uint16_t* d_full_map = nullptr;  // [spc] column of delay tau
@@ -590,19 +591,15 @@ void free_plan(fmdbzp_plan* P)
     if (P->stream) hipStreamSynchronize(P->stream);
     hipFree(P->d_twF);
     hipFree(P->d_twD);
-    hipFree(P->d_prnconj);
+    hipFree(P->d_arena);
     hipFree(P->d_patterns);
     hipFree(P->d_pset);
     hipFree(P->d_shifts);
     hipFree(P->d_signal);
-    hipFree(P->d_sigfft);
-    hipFree(P->d_tile);
-    hipFree(P->d_tile2);
+    hipFree(P->d_codes);
     hipFree(P->d_full_tw);
     hipFree(P->d_fc_tw);
-    hipFree(P->d_full_code);
     hipFree(P->d_full_map);
-    hipFree(P->d_acc);
     hipFree(P->d_rowsum);
     hipFree(P->d_rowbest_v);
     hipFree(P->d_rowbest_k);
@@ -650,17 +647,6 @@ size_t workspace_budget()
     return want;
 }
 
-// The coherent tile (and the second one of two-step column launches). Plans
-// whose calls normally run the full-period correlation allocate it with the
-// first call that needs it.
-int ensure_tile(fmdbzp_plan* P)
-{
-    int rc;
-    if (!P->d_tile && (rc = dev_alloc(&P->d_tile, P->tile_elems))) return rc;
-    if (P->col_pair && !P->d_tile2 && (rc = dev_alloc(&P->d_tile2, P->tile_elems))) return rc;
-    return FMDBZP_OK;
-}
-
 // Most coherent periods of the full-period correlation. Its fold costs
 // num_coh^2 n and adds num_coh samples one after the other in FP32, where the
 // tile's column transform grows and rounds with the logarithm. At 2.048 MHz, full-
@@ -672,48 +658,55 @@ constexpr int kFullMaxCoh = 32;
 // Full-period correlation of a plan, where it admits it: simple column stage
 // (any E with one data bit included), the code period's transform in one LDS
 // buffer with the axes of make_full31_plan or the radices of make_full_plan,
-// and the code spectra, plan data like the code FFTs, within a quarter of the
-// free memory (else, or when their allocation fails, the plan keeps to the
-// tile path; not by the workspace budget, which must not change results).
-int full_create(fmdbzp_plan* P, const int8_t* d_codes)
+// and the code spectra, plan data like the code FFTs, within
+// FMDBZP_FULL_SPECTRA_MAX_BYTES. That limit is a constant, so that neither the
+// workspace budget nor the memory in use decides how a search rounds; only if
+// the device cannot hold admitted spectra beside the plan's workspace does the
+// plan keep to the tile path (fmdbzp_plan_call_kernels tells). The size of the
+// spectra; 0: the plan does not admit it.
+size_t full_plan(fmdbzp_plan* P)
 {
     const fmdbzp_plan_desc& d = P->d;
     const int n = d.samples_per_code, ndop = d.num_doppler_bins;
-    if (!P->simple_kernel || P->tile_half || n > 65535 || (d.options & FMDBZP_OPT_TILE_PATH)) return FMDBZP_OK;
-    if (d.num_coh > kFullMaxCoh) return FMDBZP_OK;
-    if ((int64_t)d.num_coh * n > INT32_MAX || (size_t)P->ap * 4 > UINT32_MAX) return FMDBZP_OK;
+    if (!P->simple_kernel || P->tile_half || n > 65535 || (d.options & FMDBZP_OPT_TILE_PATH)) return 0;
+    if (d.num_coh > kFullMaxCoh) return 0;
+    if ((int64_t)d.num_coh * n > INT32_MAX || (size_t)P->ap * 4 > UINT32_MAX) return 0;
     // 32 elements behind the last spectrum: k_full31_corr's groups read past a row's end
     const size_t spec = ((size_t)P->nprn * ndop * n + 32) * sizeof(float2);
-    size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || spec > free_b / 4) return FMDBZP_OK;
-    const int nb = d.num_blocks, bs = d.block_size;
-    auto column = [&](int tau) { return (uint16_t)(((nb - tau / bs) % nb) * bs + tau % bs); };
-    std::vector<float2> tw;
-    std::vector<uint16_t> map((size_t)n);
-    int rc;
+    if (spec > FMDBZP_FULL_SPECTRA_MAX_BYTES) return 0;
     if (make_full31_plan(n, &P->fp31)) {
         const Full31Dev& q = P->fp31;
-        map.assign((size_t)(q.rc + 1) / 2 * 2 * 31 * q.rb, 0);
         P->full_lds = (size_t)fc31_lds_span(q) * sizeof(float2);
         // one butterfly of the last stage per thread, 24 or 32 cells per thread
         P->full_nthr = (31 * q.rb > 256 || n > 6144) ? 512 : 256;
-        if (31 * q.rb > P->full_nthr || n > 32 * P->full_nthr) {
-            P->fp31.n = 0;
-            return FMDBZP_OK;
-        }
-        for (int tau = 0; tau < n; tau++)
-            map[((size_t)(tau % q.rc / 2) * 31 * q.rb + (tau % 31) * q.rb + tau % q.rb) * 2 + (tau % q.rc) % 2] = column(tau);
+        if (31 * q.rb > P->full_nthr || n > 32 * P->full_nthr) return 0;
     } else {
         P->fp31.n = 0;
         P->full_nthr = n > 10240 ? 1024 : n > 5120 ? 512 : 256;  // at most FC_CELLS cells per thread
-        if (!make_full_plan(n, P->full_nthr, d.num_noncoherent > 1, &P->fp, &tw)) return FMDBZP_OK;
+        if (!make_full_plan(n, P->full_nthr, d.num_noncoherent > 1, &P->fp, &P->full_tw)) return 0;
         P->full_lds = (size_t)fc_lds_span(P->fp) * sizeof(float2);
-        for (int tau = 0; tau < n; tau++) map[(size_t)tau] = column(tau);
     }
     // the cell exchange reads whole groups of four cells per thread
     const size_t group = (size_t)4 * P->full_nthr;
     P->full_lds = std::max(P->full_lds, ((size_t)n + group - 1) / group * group * sizeof(float));
-    if (P->full_lds > kLdsMax) return FMDBZP_OK;
+    return P->full_lds > kLdsMax ? 0 : spec;
+}
+
+// Tables and code spectra of the full-period correlation (d_codes on the device).
+int full_spectra(fmdbzp_plan* P)
+{
+    const fmdbzp_plan_desc& d = P->d;
+    const int n = d.samples_per_code, ndop = d.num_doppler_bins, nb = d.num_blocks, bs = d.block_size;
+    auto column = [&](int tau) { return (uint16_t)(((nb - tau / bs) % nb) * bs + tau % bs); };
+    std::vector<uint16_t> map((size_t)n);
+    if (P->fp31.n) {
+        const Full31Dev& q = P->fp31;
+        map.assign((size_t)(q.rc + 1) / 2 * 2 * 31 * q.rb, 0);
+        for (int tau = 0; tau < n; tau++)
+            map[((size_t)(tau % q.rc / 2) * 31 * q.rb + (tau % 31) * q.rb + tau % q.rb) * 2 + (tau % q.rc) % 2] = column(tau);
+    } else
+        for (int tau = 0; tau < n; tau++) map[(size_t)tau] = column(tau);
+    int rc;
     if ((rc = set_lds_attr((const void*)k_full_corr<256, true>, P->full_lds)) ||
         (rc = set_lds_attr((const void*)k_full_corr<256, false>, P->full_lds)) ||
         (rc = set_lds_attr((const void*)k_full_corr<512, true>, P->full_lds)) ||
@@ -727,22 +720,16 @@ int full_create(fmdbzp_plan* P, const int8_t* d_codes)
         (rc = set_lds_attr((const void*)k_full_code, P->full_lds)) ||
         (rc = set_lds_attr((const void*)k_full31_code, P->full_lds)))
         return rc;
-    if (hipMalloc((void**)&P->d_full_code, spec) != hipSuccess) {
-        (void)hipGetLastError();
-        P->d_full_code = nullptr;
-        return FMDBZP_OK;
-    }
-    if ((rc = dev_alloc(&P->d_full_tw, tw.size())) || (rc = dev_alloc(&P->d_full_map, map.size()))) return rc;
-    HIP_TRY(hipMemcpy(P->d_full_tw, tw.data(), sizeof(float2) * tw.size(), hipMemcpyHostToDevice));
+    if ((rc = dev_alloc(&P->d_full_tw, P->full_tw.size())) || (rc = dev_alloc(&P->d_full_map, map.size()))) return rc;
+    HIP_TRY(hipMemcpy(P->d_full_tw, P->full_tw.data(), sizeof(float2) * P->full_tw.size(), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(P->d_full_map, map.data(), sizeof(uint16_t) * map.size(), hipMemcpyHostToDevice));
     if (P->fp31.n)
         k_full31_code<<<dim3(ndop, P->nprn), FC_FWD_NTHR, P->full_lds, P->stream>>>(
-            d_codes, P->d_full_code, P->fp31, bs, d.num_coh, 1.0f / (float)n);
+            P->d_codes, P->d_full_code, P->fp31, bs, d.num_coh, 1.0f / (float)n);
     else
         k_full_code<<<dim3(ndop, P->nprn), FC_FWD_NTHR, P->full_lds, P->stream>>>(
-            d_codes, P->d_full_code, P->fp, P->d_full_tw, bs, d.num_coh, 1.0f / (float)n);
+            P->d_codes, P->d_full_code, P->fp, P->d_full_tw, bs, d.num_coh, 1.0f / (float)n);
     HIP_TRY(hipGetLastError());
-    P->full = true;
     return FMDBZP_OK;
 }
 
@@ -1228,7 +1215,6 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         if (hipMemcpy(P->d_twR, twR.data(), sizeof(float2) * nb, hipMemcpyHostToDevice) != hipSuccess)
             return fail(set_err(FMDBZP_EHIP, "row twiddle upload failed"));
     }
-    if ((rc = dev_alloc(&P->d_prnconj, (size_t)nprn * nb * F))) return fail(rc);
     if ((rc = dev_alloc(&P->d_shifts, (size_t)d.num_noncoherent * ndop))) return fail(rc);
     if (hipMemcpy(P->d_shifts, drift_shifts, sizeof(int32_t) * (size_t)d.num_noncoherent * ndop,
                   hipMemcpyHostToDevice) != hipSuccess)
@@ -1255,39 +1241,7 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
                 return fail(set_err(FMDBZP_EHIP, "pattern upload failed"));
         }
     }
-    // code samples -> conj sub-block FFTs on the device
-    {
-        for (int64_t i = 0; i < (int64_t)nprn * spc; i++)
-            if (code_samples[i] != 1 && code_samples[i] != -1)
-                return fail(set_err(FMDBZP_EINVAL, "code samples must be +1/-1"));
-        int8_t* d_codes = nullptr;
-        if ((rc = dev_alloc(&d_codes, (size_t)nprn * spc))) return fail(rc);
-        hipError_t e = hipMemcpy(d_codes, code_samples, (size_t)nprn * spc, hipMemcpyHostToDevice);
-        if (e == hipSuccess) {
-            Timed t(P, FMDBZP_K_CODE_FFT, P->stream);
-            if (P->corr_variant != 10)
-                k_code_fft<<<dim3(nb, nprn), FMDBZP_NTHR, P->fft_lds, P->stream>>>(
-                    d_codes, P->d_prnconj, P->pf8, P->d_twF, spc, nb, bs, P->pscale);
-            else if (P->fc_nthr == 512)
-                k_fc_code<512><<<dim3(nb, nprn), 512, P->fc_lds, P->stream>>>(d_codes, P->d_prnconj, P->fc, P->d_fc_tw,
-                                                                             spc, nb, bs, P->pscale);
-            else
-                k_fc_code<256><<<dim3(nb, nprn), 256, P->fc_lds, P->stream>>>(d_codes, P->d_prnconj, P->fc, P->d_fc_tw,
-                                                                             spc, nb, bs, P->pscale);
-            e = hipGetLastError();
-        }
-        if (e == hipSuccess && (rc = full_create(P, d_codes))) {
-            hipStreamSynchronize(P->stream);
-            hipFree(d_codes);
-            return fail(rc);
-        }
-        if (e == hipSuccess) e = hipStreamSynchronize(P->stream);
-        hipFree(d_codes);
-        if (e != hipSuccess) return fail(set_err(FMDBZP_EHIP, "code FFT failed: %s", hipGetErrorString(e)));
-        collect_timing(P);
-    }
     // workspace: signal FFT cache for all segments + PRN-batch tile/accumulator
-    if ((rc = dev_alloc(&P->d_sigfft, (size_t)d.num_noncoherent * ndop * F))) return fail(rc);
     const int tile_blocks = P->rotbig ? P->nrb_max : nb;
     {
         size_t per_prn = (size_t)tile_blocks * ndop * P->tp * sizeof(float2) * (P->col_pair ? 2 : 1) +
@@ -1318,9 +1272,36 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         while ((size_t)nchunk() * kRedPart > (size_t)nb * P->tp * sizeof(float2)) P->red_cw *= 2;
         P->red_nchunk = nchunk();
     }
-    P->tile_elems = (size_t)P->batch * tile_blocks * ndop * P->tp;
-    if ((!P->full && (rc = ensure_tile(P))) || (rc = dev_alloc(&P->d_acc, (size_t)P->batch * P->acc_ps)) ||
-        (rc = dev_alloc(&P->d_rowsum, (size_t)P->batch * ndop)) ||
+    // The large buffers are one allocation: a free of each (200 to 300 us from
+    // about 30 MB on) would cost more than all of a small plan's creation. The
+    // code spectra come last: where they do not fit beside the rest, the plan
+    // does without the full-period correlation.
+    {
+        const size_t tile_bytes = (size_t)P->batch * tile_blocks * ndop * P->tp * sizeof(float2);
+        size_t total = 0;
+        auto place = [&](size_t bytes) {  // large ones on 2 MiB pages, as an allocation of their own
+            const size_t page = bytes >= (2u << 20) ? (2u << 20) : 256, at = (total + page - 1) / page * page;
+            total = at + bytes;
+            return at;
+        };
+        const size_t o_prn = place((size_t)nprn * nb * F * sizeof(float2));
+        const size_t o_sig = place((size_t)d.num_noncoherent * ndop * F * sizeof(float2));
+        const size_t o_tile = place(tile_bytes), o_tile2 = P->col_pair ? place(tile_bytes) : 0;
+        const size_t o_acc = place((size_t)P->batch * P->acc_ps * sizeof(float));
+        const size_t without = total, spec = full_plan(P), o_spec = place(spec);
+        if (spec) {
+            P->full = hipMalloc((void**)&P->d_arena, total) == hipSuccess;
+            if (!P->full) (void)hipGetLastError();
+        }
+        if (!P->full && (rc = dev_alloc(&P->d_arena, without))) return fail(rc);
+        P->d_prnconj = (float2*)(P->d_arena + o_prn);
+        P->d_sigfft = (float2*)(P->d_arena + o_sig);
+        P->d_tile = (float2*)(P->d_arena + o_tile);
+        if (P->col_pair) P->d_tile2 = (float2*)(P->d_arena + o_tile2);
+        P->d_acc = (float*)(P->d_arena + o_acc);
+        if (P->full) P->d_full_code = (float2*)(P->d_arena + o_spec);
+    }
+    if ((rc = dev_alloc(&P->d_rowsum, (size_t)P->batch * ndop)) ||
         (rc = dev_alloc(&P->d_rowbest_v, (size_t)P->batch * ndop)) ||
         (rc = dev_alloc(&P->d_rowbest_k, (size_t)P->batch * ndop)))
         return fail(rc);
@@ -1333,6 +1314,36 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         if (d.noise_estimator == FMDBZP_NOISE_GLOBAL_MEAN &&
             (rc = dev_alloc(&P->d_colsum, (size_t)P->batch * spc_eff)))
             return fail(rc);
+    }
+    // code samples -> conj sub-block FFTs on the device
+    {
+        for (int64_t i = 0; i < (int64_t)nprn * spc; i++)
+            if (code_samples[i] != 1 && code_samples[i] != -1)
+                return fail(set_err(FMDBZP_EINVAL, "code samples must be +1/-1"));
+        if ((rc = dev_alloc(&P->d_codes, (size_t)nprn * spc))) return fail(rc);
+        hipError_t e = hipMemcpy(P->d_codes, code_samples, (size_t)nprn * spc, hipMemcpyHostToDevice);
+        if (e == hipSuccess) {
+            Timed t(P, FMDBZP_K_CODE_FFT, P->stream);
+            if (P->corr_variant != 10)
+                k_code_fft<<<dim3(nb, nprn), FMDBZP_NTHR, P->fft_lds, P->stream>>>(
+                    P->d_codes, P->d_prnconj, P->pf8, P->d_twF, spc, nb, bs, P->pscale);
+            else if (P->fc_nthr == 512)
+                k_fc_code<512><<<dim3(nb, nprn), 512, P->fc_lds, P->stream>>>(P->d_codes, P->d_prnconj, P->fc,
+                                                                             P->d_fc_tw, spc, nb, bs, P->pscale);
+            else
+                k_fc_code<256><<<dim3(nb, nprn), 256, P->fc_lds, P->stream>>>(P->d_codes, P->d_prnconj, P->fc,
+                                                                             P->d_fc_tw, spc, nb, bs, P->pscale);
+            e = hipGetLastError();
+        }
+        if (e != hipSuccess) return fail(set_err(FMDBZP_EHIP, "code FFT failed: %s", hipGetErrorString(e)));
+    }
+    if (P->full && (rc = full_spectra(P))) return fail(rc);
+    {
+        const hipError_t e = hipStreamSynchronize(P->stream);
+        if (e != hipSuccess) return fail(set_err(FMDBZP_EHIP, "code spectra failed: %s", hipGetErrorString(e)));
+        hipFree(P->d_codes);
+        P->d_codes = nullptr;
+        collect_timing(P);
     }
     const char* at = getenv("FMDBZP_AUTOTUNE");
     if ((d.options & FMDBZP_OPT_AUTOTUNE) || (at && atoi(at) != 0))
@@ -1748,10 +1759,6 @@ int acquire_enqueue(fmdbzp_plan* P, const void* signal, int32_t eltype, int64_t 
     if (store && !P->d_export && !(flags & FMDBZP_FLAG_DEVICE_OUTPUT))
         HIP_TRY(hipMalloc((void**)&P->d_export, sizeof(float) * (size_t)ndop * surf_cols * kLanes));
 
-    if (!full_call(P, eltype, nreq, store)) {
-        const int rc = ensure_tile(P);
-        if (rc) return rc;
-    }
     Work W{P->d_sigfft, P->d_tile, P->d_acc, P->d_rowsum, P->d_rowbest_v, P->d_rowbest_k, P->d_psum,
            P->d_pbest_v, P->d_pbest_k, P->d_req, P->d_stats, P->batch, P->nlanes, true,
            P->col_pair ? P->d_tile2 : nullptr};
@@ -2322,7 +2329,6 @@ int autotune(fmdbzp_plan* P)
                 return FMDBZP_OK;
             }
     }
-    if (const int rc = ensure_tile(P)) return rc;
     std::vector<int> variants;
     if (P->corr_variant >= 3) variants.push_back(P->corr_variant);  // compile-time transform
     else {

@@ -133,6 +133,12 @@ enum fmdbzp_precision {
  * tile either way (fmdbzp_plan_call_kernels tells). For measuring the tile
  * kernels. Results agree to FP32 rounding. No counterpart in the reference. */
 #define FMDBZP_OPT_TILE_PATH 0x10
+/* Largest size of the code spectra of the full-period correlation, plan data
+ * of 8 bytes x samples_per_code x num_doppler_bins per PRN held beside the
+ * workspace (the L1 C/A search at 16.368 MHz, 160 bins, 32 PRNs: 0.67 GB).
+ * Plans that would exceed it run on the tile. The limit depends neither on the
+ * workspace budget nor on the memory in use. */
+#define FMDBZP_FULL_SPECTRA_MAX_BYTES (4ull << 30)
 
 /* fmdbzp_acquire flags */
 #define FMDBZP_FLAG_STORE_SURFACES 0x1u  /* copy (ndop, spc_eff) power surfaces out */
