@@ -1260,13 +1260,14 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
     }
     if (P->acc_cm && !P->rotbig) {
         // columns per workgroup of the column-major reduction: about 1024
-        // workgroups over the batch, 32 to 4096 columns each. With 4096
-        // columns always, 8 PRNs of 4000 columns (640 Doppler rows) ran on 8
-        // workgroups, 1430 us; a 2.5 M-column surface keeps 4096. The
-        // partials (20 bytes per row and chunk) live in the batch's tile,
-        // which is consumed by then: wider chunks where they would not fit.
+        // workgroups per PRN, 32 to 4096 columns each. With 4096 columns
+        // always, 8 PRNs of 4000 columns (640 Doppler rows) ran on 8
+        // workgroups, 1430 us; a 2.5 M-column surface keeps 4096. Not by the
+        // batch: the FP64 sums of a search round by its chunks. The partials
+        // (20 bytes per row and chunk) live in the batch's tile, which is
+        // consumed by then: wider chunks where they would not fit.
         const size_t rb4 = (ndop + 4 * FMDBZP_NTHR - 1) / (4 * FMDBZP_NTHR);
-        const size_t cw = (size_t)spc_eff * rb4 * P->batch / 1024;
+        const size_t cw = (size_t)spc_eff * rb4 / 1024;
         P->red_cw = (int)std::min<size_t>(4096, std::max<size_t>(32, (cw + 31) / 32 * 32));
         auto nchunk = [&]() { return (spc_eff + P->red_cw - 1) / P->red_cw; };
         while ((size_t)nchunk() * kRedPart > (size_t)nb * P->tp * sizeof(float2)) P->red_cw *= 2;
