@@ -128,7 +128,7 @@ constexpr size_t kLdsMax = 160 * 1024;   // gfx950 LDS per workgroup
 // radix is odd unless n is a power of two (bank spread); with one noncoherent
 // step 25 may run first and 20 and 22 in the middle, else at most 16. false: n has a
 // prime factor above 13, more than FC_MAX_STAGES stages, or fewer than two.
-bool make_full_plan(int n, int nthr, bool multi, FullPlanDev* f, std::vector<float2>* tw)
+bool make_full_plan(int n, int nthr, bool multi, FullPlanDev* f)
 {
     struct Radix {
         int r;
@@ -171,21 +171,14 @@ bool make_full_plan(int n, int nthr, bool multi, FullPlanDev* f, std::vector<flo
     f->nst = (int)best.size();
     f->pad_shift = 31;
     if (best[0] % 2 == 0) f->pad_shift = __builtin_ctz((unsigned)best[0]);
-    int ns = 1;
-    tw->clear();
+    int ns = 1, at = 0;
     for (int t = 0; t < f->nst; t++) {
         const int R = best[(size_t)t];
         f->radix[t] = R;
         f->ns[t] = ns;
         f->inv_ns[t] = 1.0f / (float)ns;
-        f->twoff[t] = (int)tw->size();
-        if (t > 0)
-            for (int r = 1; r < R; r++)
-                for (int k = 0; k < ns; k++) {
-                    double s, c;
-                    sincospi_d(2.0 * (double)((int64_t)r * k) / ((double)ns * R), &s, &c);
-                    tw->push_back(make_float2((float)c, (float)(-s)));
-                }
+        f->twoff[t] = at;
+        if (t > 0) at += (R - 1) * ns;
         ns *= R;
     }
     return true;
@@ -345,7 +338,6 @@ struct fmdbzp_plan {
     Full31Dev fp31{};                // the chip-rate multiples' form (fp31.n != 0)
     int full_nthr = 0;
     size_t full_lds = 0;
-    std::vector<float2> full_tw;
     float2* d_full_tw = nullptr;
     float2* d_full_code = nullptr;   // [nprn][ndop][spc] code spectra
     uint16_t* d_full_map = nullptr;  // [spc] column of delay tau
@@ -655,6 +647,21 @@ size_t workspace_budget()
 // error against 64 bits 3.2e-7 / 1.4e-7 at 1000 periods and 4.9e-7 / 1.3e-7 at 2000.
 constexpr int kFullMaxCoh = 32;
 
+// Few rows of long periods over nreq PRNs: a row is one workgroup of the full-
+// period correlation, and up to 32 of them leave most of the device idle over 13
+// to 18 us of transform per step, where the tile's kernels split every row. Call
+// times in us, full-period and tile: at 20 MHz 16 rows 73 / 65 (one step),
+// 208 / 161 (8 steps); 32 rows 74 / 70, 208 / 181; 48 rows 76 / 74, 210 / 200; at
+// 16.384 MHz 16 rows 66 / 60, 156 / 145; 32 rows 67 / 63, 158 / 159; at 15 MHz 20
+// rows 65 / 67, 151 / 209. The 31-axis form is the faster one from two steps on
+// (16.368 MHz, 16 rows: 67 / 60, 141 / 149).
+bool full_few_rows(const fmdbzp_plan* P, int nreq)
+{
+    const bool several = P->d.num_noncoherent > 1;
+    const int64_t rows = (int64_t)P->d.num_doppler_bins * nreq;
+    return P->d.samples_per_code > 15360 && rows < (several ? 33 : 32) && !(several && P->fp31.n);
+}
+
 // Full-period correlation of a plan, where it admits it: simple column stage
 // (any E with one data bit included), the code period's transform in one LDS
 // buffer with the axes of make_full31_plan or the radices of make_full_plan,
@@ -683,13 +690,14 @@ size_t full_plan(fmdbzp_plan* P)
     } else {
         P->fp31.n = 0;
         P->full_nthr = n > 10240 ? 1024 : n > 5120 ? 512 : 256;  // at most FC_CELLS cells per thread
-        if (!make_full_plan(n, P->full_nthr, d.num_noncoherent > 1, &P->fp, &P->full_tw)) return 0;
+        if (!make_full_plan(n, P->full_nthr, d.num_noncoherent > 1, &P->fp)) return 0;
         P->full_lds = (size_t)fc_lds_span(P->fp) * sizeof(float2);
     }
     // the cell exchange reads whole groups of four cells per thread
     const size_t group = (size_t)4 * P->full_nthr;
     P->full_lds = std::max(P->full_lds, ((size_t)n + group - 1) / group * group * sizeof(float));
-    return P->full_lds > kLdsMax ? 0 : spec;
+    if (P->full_lds > kLdsMax || full_few_rows(P, P->nprn)) return 0;  // the latter: no call would use them
+    return spec;
 }
 
 // Tables and code spectra of the full-period correlation (d_codes on the device).
@@ -697,15 +705,6 @@ int full_spectra(fmdbzp_plan* P)
 {
     const fmdbzp_plan_desc& d = P->d;
     const int n = d.samples_per_code, ndop = d.num_doppler_bins, nb = d.num_blocks, bs = d.block_size;
-    auto column = [&](int tau) { return (uint16_t)(((nb - tau / bs) % nb) * bs + tau % bs); };
-    std::vector<uint16_t> map((size_t)n);
-    if (P->fp31.n) {
-        const Full31Dev& q = P->fp31;
-        map.assign((size_t)(q.rc + 1) / 2 * 2 * 31 * q.rb, 0);
-        for (int tau = 0; tau < n; tau++)
-            map[((size_t)(tau % q.rc / 2) * 31 * q.rb + (tau % 31) * q.rb + tau % q.rb) * 2 + (tau % q.rc) % 2] = column(tau);
-    } else
-        for (int tau = 0; tau < n; tau++) map[(size_t)tau] = column(tau);
     int rc;
     if ((rc = set_lds_attr((const void*)k_full_corr<256, true>, P->full_lds)) ||
         (rc = set_lds_attr((const void*)k_full_corr<256, false>, P->full_lds)) ||
@@ -720,15 +719,22 @@ int full_spectra(fmdbzp_plan* P)
         (rc = set_lds_attr((const void*)k_full_code, P->full_lds)) ||
         (rc = set_lds_attr((const void*)k_full31_code, P->full_lds)))
         return rc;
-    if ((rc = dev_alloc(&P->d_full_tw, P->full_tw.size())) || (rc = dev_alloc(&P->d_full_map, map.size()))) return rc;
-    HIP_TRY(hipMemcpy(P->d_full_tw, P->full_tw.data(), sizeof(float2) * P->full_tw.size(), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(P->d_full_map, map.data(), sizeof(uint16_t) * map.size(), hipMemcpyHostToDevice));
-    if (P->fp31.n)
-        k_full31_code<<<dim3(ndop, P->nprn), FC_FWD_NTHR, P->full_lds, P->stream>>>(
+    auto grid = [](int count) { return dim3((count + 255) / 256); };
+    hipStream_t st = P->stream;
+    const size_t nmap = P->fp31.n ? (size_t)(P->fp31.rc + 1) / 2 * 2 * 31 * P->fp31.rb : (size_t)n;
+    if ((rc = dev_alloc(&P->d_full_map, nmap))) return rc;
+    if (P->fp31.n) {
+        k_full31_map<<<grid(n), 256, 0, st>>>(P->d_full_map, P->fp31, nb, bs);
+        k_full31_code<<<dim3(ndop, P->nprn), FC_FWD_NTHR, P->full_lds, st>>>(
             P->d_codes, P->d_full_code, P->fp31, bs, d.num_coh, 1.0f / (float)n);
-    else
-        k_full_code<<<dim3(ndop, P->nprn), FC_FWD_NTHR, P->full_lds, P->stream>>>(
+    } else {
+        const int ntw = fc_tw_count(P->fp);
+        if ((rc = dev_alloc(&P->d_full_tw, (size_t)ntw))) return rc;
+        k_fc_twiddles<<<grid(ntw), 256, 0, st>>>(P->fp, P->d_full_tw, ntw);
+        k_full_map<<<grid(n), 256, 0, st>>>(P->d_full_map, n, nb, bs);
+        k_full_code<<<dim3(ndop, P->nprn), FC_FWD_NTHR, P->full_lds, st>>>(
             P->d_codes, P->d_full_code, P->fp, P->d_full_tw, bs, d.num_coh, 1.0f / (float)n);
+    }
     HIP_TRY(hipGetLastError());
     return FMDBZP_OK;
 }
@@ -741,19 +747,10 @@ bool int_samples(int32_t eltype)
 // Whether a call over nreq PRNs runs the full-period correlation: not with
 // surfaces (their time is the copy to the caller, and the tile path's column
 // kernels stay the ones that write them), nor where FMDBZP_PREC_AUTO takes the
-// FP16 tile, nor with few rows of long periods: a row is one workgroup there,
-// and up to 32 of them leave most of the device idle over 13 to 18 us of
-// transform per step, where the tile's kernels split every row. Call times at 20 MHz
-// in us, full-period and tile: 16 rows 73 / 65 (one step), 208 / 161 (8 steps);
-// 32 rows 74 / 70, 208 / 181; 48 rows 76 / 74, 210 / 200; at 16.384 MHz 16 rows
-// 66 / 60, 156 / 145; 32 rows 67 / 63, 158 / 159; at 15 MHz 20 rows 65 / 67, 151 / 209.
-// The 31-axis form is the faster one from two steps on (16.368 MHz, 16 rows: 67 / 60, 141 / 149).
+// FP16 tile, nor with few rows.
 bool full_call(const fmdbzp_plan* P, int32_t eltype, int32_t nreq, bool store)
 {
-    if (!P->full || store || (P->tile_auto && int_samples(eltype))) return false;
-    const bool several = P->d.num_noncoherent > 1;
-    const int64_t rows = (int64_t)P->d.num_doppler_bins * nreq;
-    return !(P->d.samples_per_code > 15360 && rows < (several ? 33 : 32) && !(several && P->fp31.n));
+    return P->full && !store && !(P->tile_auto && int_samples(eltype)) && !full_few_rows(P, nreq);
 }
 
 // Column-stage form of the plan on the tile (fmdbzp_plan_column_kernel).
@@ -897,10 +894,9 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
     else if (fft_inplace_ok(P->pf) && 2 * F <= FMDBZP_CORR_MAXV * FMDBZP_NTHR) P->corr_variant = 2;
     else if (fft_inplace_ok(P->pf) && F <= FMDBZP_CORR_MAXV * FMDBZP_NTHR) P->corr_variant = 1;
     else P->corr_variant = 0;
-    std::vector<float2> fc_tw;
     if (P->corr_variant < 2) {  // one transform per pass, runtime radices: in place instead, where F factors
         P->fc_nthr = F > 5120 ? 512 : 256;
-        if (make_full_plan(F, P->fc_nthr, false, &P->fc, &fc_tw)) {
+        if (make_full_plan(F, P->fc_nthr, false, &P->fc)) {
             P->corr_variant = 10;
             P->fc_lds = (size_t)fc_lds_span(P->fc) * sizeof(float2);
             P->pscale = P->inv_f;  // 1/F in the code spectra for every F
@@ -1197,8 +1193,8 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
             return fail(set_err(FMDBZP_EHIP, "twiddle upload failed"));
     }
     if (P->corr_variant == 10) {
-        if ((rc = dev_alloc(&P->d_fc_tw, fc_tw.size()))) return fail(rc);
-        if (hipMemcpy(P->d_fc_tw, fc_tw.data(), sizeof(float2) * fc_tw.size(), hipMemcpyHostToDevice) != hipSuccess ||
+        const int count = fc_tw_count(P->fc);
+        if ((rc = dev_alloc(&P->d_fc_tw, (size_t)count)) ||
             (rc = set_lds_attr((const void*)k_fc_code<256>, P->fc_lds)) ||
             (rc = set_lds_attr((const void*)k_fc_code<512>, P->fc_lds)) ||
             (rc = set_lds_attr((const void*)k_fc_signal<256>, P->fc_lds)) ||
@@ -1207,7 +1203,9 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
             (rc = set_lds_attr((const void*)k_corr_fc<512, float2>, P->fc_lds)) ||
             (rc = set_lds_attr((const void*)k_corr_fc<256, __half2>, P->fc_lds)) ||
             (rc = set_lds_attr((const void*)k_corr_fc<512, __half2>, P->fc_lds)))
-            return fail(rc ? rc : set_err(FMDBZP_EHIP, "transform twiddle upload failed"));
+            return fail(rc);
+        k_fc_twiddles<<<dim3((count + 255) / 256), 256, 0, P->stream>>>(P->fc, P->d_fc_tw, count);
+        if (hipGetLastError() != hipSuccess) return fail(set_err(FMDBZP_EHIP, "transform twiddles failed"));
     }
     if (P->rotbig) {
         std::vector<float2> twR = twiddles(nb);

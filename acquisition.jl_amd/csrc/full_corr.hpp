@@ -389,11 +389,50 @@ __device__ __forceinline__ void fc_forward(float2* lds, const FullPlanDev& f, co
 }
 
 // ---------------------------------------------------------------------------
+// Tables (plan time), FP64 angles on the device: on the host the sines of a
+// 20000-point plan took 0.4 ms, as long as the rest of its creation.
+// ---------------------------------------------------------------------------
+inline int fc_tw_count(const FullPlanDev& f)
+{
+    const int t = f.nst - 1;
+    return f.twoff[t] + (f.radix[t] - 1) * f.ns[t];
+}
+// twiddles of the stages, in their order. grid (ceil(fc_tw_count / 256))
+__global__ void __launch_bounds__(256)
+k_fc_twiddles(FullPlanDev f, float2* __restrict__ tw, int count)
+{
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= count) return;
+    int t = f.nst - 1;
+    while (t > 1 && e < f.twoff[t]) t--;
+    const int ns = f.ns[t], r = (e - f.twoff[t]) / ns + 1, k = (e - f.twoff[t]) % ns;
+    double sn, cs;
+    sincospi(-2.0 * (double)((int64_t)r * k) / ((double)ns * f.radix[t]), &sn, &cs);
+    tw[e] = make_float2((float)cs, (float)sn);
+}
+// column of delay tau: block (nb - tau / bs) mod nb, lag tau mod bs
+__device__ __forceinline__ uint16_t full_column(int tau, int nb, int bs)
+{
+    const int r = tau / bs;
+    return (uint16_t)((r ? nb - r : 0) * bs + tau % bs);
+}
+// grid (ceil(n / 256))
+__global__ void __launch_bounds__(256)
+k_full_map(uint16_t* __restrict__ map, int n, int nb, int bs)
+{
+    const int tau = blockIdx.x * 256 + threadIdx.x;
+    if (tau < n) map[tau] = full_column(tau, nb, bs);
+}
+
+// ---------------------------------------------------------------------------
 // Code spectra (plan time): conj(DFT(conj a_w)) / spc. grid (ndop, nprn)
 // ---------------------------------------------------------------------------
 #define FC_FWD_NTHR 512
 // conj a_w[m]: exp(2 pi i (w bs floor(m / bs) - s m) / (ncoh spc)) times the
-// code sample, the angle an exact integer over ncoh spc
+// code sample, the angle an exact integer over ncoh spc. (The sincospi is not
+// what bounds these kernels: with the angle's two factors from tables they took
+// 50.9 instead of 56.9 us at 8 x 80 rows of 10000 points and 543 instead of 538 at
+// 32 x 160 of 16368.)
 __device__ __forceinline__ float2 full_code_in(const int8_t* c, int m, int w, int s, int bs, double two_over_d)
 {
     const double t = (double)((int64_t)w * ((m / bs) * bs) - (int64_t)s * m);
@@ -1569,6 +1608,19 @@ k_full31_code(const int8_t* __restrict__ codes, float2* __restrict__ spec, Full3
     fc31_forward<FC_FWD_NTHR>(
         lds, f, threadIdx.x, [&](int m) { return full_code_in(c, m, w, s, bs, two_over_d); },
         [&](int i, float2 x) { out[i] = make_float2(x.x * scale, -x.y * scale); });
+}
+// columns of k_full31_corr's last stage: [(rc + 1) / 2][31 rb] pairs of outputs
+// c = 2 i, 2 i + 1 of (k, b); the partner of an odd rc's last output is 0.
+// grid (ceil(n / 256))
+__global__ void __launch_bounds__(256)
+k_full31_map(uint16_t* __restrict__ map, Full31Dev f, int nb, int bs)
+{
+    const int tau = blockIdx.x * 256 + threadIdx.x;
+    if (tau >= f.n) return;
+    const int c = tau % f.rc;
+    uint16_t* at = map + ((size_t)(c / 2) * 31 * f.rb + (tau % 31) * f.rb + tau % f.rb) * 2;
+    at[c & 1] = full_column(tau, nb, bs);
+    if (c == f.rc - 1 && !(c & 1)) at[1] = 0;
 }
 
 template <int NTHR>
