@@ -319,7 +319,8 @@ def plan_acquire(system: GNSSSystem, sampling_freq: float, prns: Sequence[int], 
                  tile_precision: str = "fp32",
                  graphs: bool = False,
                  autotune: bool = False,
-                 fp64_carrier_phase: bool = False) -> AcquisitionPlan:
+                 fp64_carrier_phase: bool = False,
+                 _tile_path: bool = False) -> AcquisitionPlan:
     """Pre-compute an FM-DBZP acquisition plan (src/plan.jl:312-324).
 
     Keyword arguments and validation errors are the reference's; frequencies
@@ -376,6 +377,7 @@ def plan_acquire(system: GNSSSystem, sampling_freq: float, prns: Sequence[int], 
     plan.graphs = bool(graphs)
     plan.autotune = bool(autotune)
     plan.fp64_carrier_phase = bool(fp64_carrier_phase)
+    plan.tile_path = bool(_tile_path)
     if tile_precision not in ("fp32", "fp16", "auto", "mfma"):
         raise ArgumentError(f"tile_precision must be 'fp32', 'fp16', 'mfma' or 'auto', got {tile_precision!r}")
     plan.tile_precision = tile_precision
