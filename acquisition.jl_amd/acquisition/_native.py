@@ -148,6 +148,7 @@ EXPORTED_SYMBOLS = (
     "fmdbzp_plan_tuning",
     "fmdbzp_plan_column_kernel",
     "fmdbzp_plan_call_kernels",
+    "fmdbzp_full_period_form",
     "fmdbzp_plan_kernel_times",
     "fmdbzp_synthesize",
     "fmdbzp_plan_set_surface_layout",
@@ -201,6 +202,8 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
     if hasattr(lib, "fmdbzp_plan_column_kernel"):
         lib.fmdbzp_plan_column_kernel.argtypes = [P, ctypes.c_char_p, ctypes.c_size_t]
         lib.fmdbzp_plan_column_kernel.restype = ctypes.c_int
+    lib.fmdbzp_full_period_form.argtypes = [I, I, I, I, I]
+    lib.fmdbzp_full_period_form.restype = ctypes.c_int
     if hasattr(lib, "fmdbzp_plan_call_kernels"):
         lib.fmdbzp_plan_call_kernels.argtypes = [P, ctypes.c_int32, ctypes.c_int32, ctypes.c_uint32, ctypes.c_char_p,
                                                  ctypes.c_size_t]
@@ -223,6 +226,14 @@ def prn_results(stats, n: int, spc: int, nb: int, bs: int, fs: float, fc: float,
     """`fmdbzp_prn_results` over a ctypes array of `PrnStats`."""
     _check(lib().fmdbzp_prn_results(stats, n, spc, nb, bs, fs, fc, code_length, tcoh, spacing, interpolate, out_ptr),
            "fmdbzp_prn_results")
+
+
+def full_period_form(samples_per_code: int, num_blocks: int, num_coh: int, num_noncoherent: int, nprn: int) -> str:
+    """Form of the full-period correlation of a statistics-only call: "radix",
+    "axis31", or "" where the call runs on the tile (`fmdbzp_full_period_form`)."""
+    rc = lib().fmdbzp_full_period_form(samples_per_code, num_blocks, num_coh, num_noncoherent, nprn)
+    _check(min(rc, 0), "fmdbzp_full_period_form")
+    return ("", "radix", "axis31")[rc]
 
 
 def acquire_batch(reqs):

@@ -655,17 +655,46 @@ constexpr int kFullMaxCoh = 32;
 // 16.384 MHz 16 rows 66 / 60, 156 / 145; 32 rows 67 / 63, 158 / 159; at 15 MHz 20
 // rows 65 / 67, 151 / 209. The 31-axis form is the faster one from two steps on
 // (16.368 MHz, 16 rows: 67 / 60, 141 / 149).
+bool full_few_rows(int n, bool several, bool axis31, int64_t rows)
+{
+    return n > 15360 && rows < (several ? 33 : 32) && !(several && axis31);
+}
 bool full_few_rows(const fmdbzp_plan* P, int nreq)
 {
-    const bool several = P->d.num_noncoherent > 1;
-    const int64_t rows = (int64_t)P->d.num_doppler_bins * nreq;
-    return P->d.samples_per_code > 15360 && rows < (several ? 33 : 32) && !(several && P->fp31.n);
+    return full_few_rows(P->d.samples_per_code, P->d.num_noncoherent > 1, P->fp31.n != 0,
+                         (int64_t)P->d.num_doppler_bins * nreq);
+}
+
+// 32 elements behind the last spectrum: k_full31_corr's groups read past a row's end
+size_t full_spectra_bytes(int64_t nprn, int64_t ndop, int64_t n) { return ((size_t)(nprn * ndop * n) + 32) * sizeof(float2); }
+
+// The full-period transform of n points: the axes of make_full31_plan
+// (FMDBZP_FULL_AXIS31) or the radices of make_full_plan (FMDBZP_FULL_RADIX) in
+// one LDS buffer, its threads and LDS; FMDBZP_FULL_NONE where neither fits.
+int full_form(int n, bool several, FullPlanDev* fp, Full31Dev* fp31, int* nthr, size_t* lds)
+{
+    if (n > 65535) return FMDBZP_FULL_NONE;
+    const bool axis31 = make_full31_plan(n, fp31);
+    if (axis31) {
+        *lds = (size_t)fc31_lds_span(*fp31) * sizeof(float2);
+        // one butterfly of the last stage per thread, 24 or 32 cells per thread
+        *nthr = (31 * fp31->rb > 256 || n > 6144) ? 512 : 256;
+        if (31 * fp31->rb > *nthr || n > 32 * *nthr) return FMDBZP_FULL_NONE;
+    } else {
+        fp31->n = 0;
+        *nthr = n > 10240 ? 1024 : n > 5120 ? 512 : 256;  // at most FC_CELLS cells per thread
+        if (!make_full_plan(n, *nthr, several, fp)) return FMDBZP_FULL_NONE;
+        *lds = (size_t)fc_lds_span(*fp) * sizeof(float2);
+    }
+    // the cell exchange reads whole groups of four cells per thread
+    const size_t group = (size_t)4 * *nthr;
+    *lds = std::max(*lds, ((size_t)n + group - 1) / group * group * sizeof(float));
+    return *lds > kLdsMax ? FMDBZP_FULL_NONE : axis31 ? FMDBZP_FULL_AXIS31 : FMDBZP_FULL_RADIX;
 }
 
 // Full-period correlation of a plan, where it admits it: simple column stage
-// (any E with one data bit included), the code period's transform in one LDS
-// buffer with the axes of make_full31_plan or the radices of make_full_plan,
-// and the code spectra, plan data like the code FFTs, within
+// (any E with one data bit included), a full_form, up to kFullMaxCoh periods and
+// the code spectra, plan data like the code FFTs, within
 // FMDBZP_FULL_SPECTRA_MAX_BYTES. That limit is a constant, so that neither the
 // workspace budget nor the memory in use decides how a search rounds; only if
 // the device cannot hold admitted spectra beside the plan's workspace does the
@@ -674,29 +703,13 @@ bool full_few_rows(const fmdbzp_plan* P, int nreq)
 size_t full_plan(fmdbzp_plan* P)
 {
     const fmdbzp_plan_desc& d = P->d;
-    const int n = d.samples_per_code, ndop = d.num_doppler_bins;
-    if (!P->simple_kernel || P->tile_half || n > 65535 || (d.options & FMDBZP_OPT_TILE_PATH)) return 0;
-    if (d.num_coh > kFullMaxCoh) return 0;
-    if ((int64_t)d.num_coh * n > INT32_MAX || (size_t)P->ap * 4 > UINT32_MAX) return 0;
-    // 32 elements behind the last spectrum: k_full31_corr's groups read past a row's end
-    const size_t spec = ((size_t)P->nprn * ndop * n + 32) * sizeof(float2);
-    if (spec > FMDBZP_FULL_SPECTRA_MAX_BYTES) return 0;
-    if (make_full31_plan(n, &P->fp31)) {
-        const Full31Dev& q = P->fp31;
-        P->full_lds = (size_t)fc31_lds_span(q) * sizeof(float2);
-        // one butterfly of the last stage per thread, 24 or 32 cells per thread
-        P->full_nthr = (31 * q.rb > 256 || n > 6144) ? 512 : 256;
-        if (31 * q.rb > P->full_nthr || n > 32 * P->full_nthr) return 0;
-    } else {
-        P->fp31.n = 0;
-        P->full_nthr = n > 10240 ? 1024 : n > 5120 ? 512 : 256;  // at most FC_CELLS cells per thread
-        if (!make_full_plan(n, P->full_nthr, d.num_noncoherent > 1, &P->fp)) return 0;
-        P->full_lds = (size_t)fc_lds_span(P->fp) * sizeof(float2);
-    }
-    // the cell exchange reads whole groups of four cells per thread
-    const size_t group = (size_t)4 * P->full_nthr;
-    P->full_lds = std::max(P->full_lds, ((size_t)n + group - 1) / group * group * sizeof(float));
-    if (P->full_lds > kLdsMax || full_few_rows(P, P->nprn)) return 0;  // the latter: no call would use them
+    if (!P->simple_kernel || P->tile_half || (d.options & FMDBZP_OPT_TILE_PATH) || d.num_coh > kFullMaxCoh) return 0;
+    const size_t spec = full_spectra_bytes(P->nprn, d.num_doppler_bins, d.samples_per_code);
+    if (spec > FMDBZP_FULL_SPECTRA_MAX_BYTES ||
+        full_form(d.samples_per_code, d.num_noncoherent > 1, &P->fp, &P->fp31, &P->full_nthr, &P->full_lds) ==
+            FMDBZP_FULL_NONE ||
+        full_few_rows(P, P->nprn))  // no call would use them
+        return 0;
     return spec;
 }
 
@@ -1560,6 +1573,26 @@ int fmdbzp_plan_column_kernel(fmdbzp_plan* plan, char* buf, size_t buflen)
     if (!buf || buflen == 0) return set_err(FMDBZP_EINVAL, "null buffer");
     column_name(plan, buf, buflen);
     return FMDBZP_OK;
+}
+
+int fmdbzp_full_period_form(int32_t samples_per_code, int32_t num_blocks, int32_t num_coh, int32_t num_noncoherent,
+                            int32_t nprn)
+{
+    if (samples_per_code <= 0 || num_blocks <= 0 || num_coh <= 0 || num_noncoherent <= 0 || nprn <= 0)
+        return set_err(FMDBZP_EINVAL, "fmdbzp_full_period_form: sizes must be positive");
+    const int64_t ndop = (int64_t)num_coh * num_blocks;
+    if (num_coh > kFullMaxCoh || samples_per_code > 65535 ||
+        ndop * nprn > (int64_t)(FMDBZP_FULL_SPECTRA_MAX_BYTES / sizeof(float2)) ||
+        full_spectra_bytes(nprn, ndop, samples_per_code) > FMDBZP_FULL_SPECTRA_MAX_BYTES)
+        return FMDBZP_FULL_NONE;
+    FullPlanDev fp{};
+    Full31Dev fp31{};
+    int nthr = 0;
+    size_t lds = 0;
+    const int form = full_form(samples_per_code, num_noncoherent > 1, &fp, &fp31, &nthr, &lds);
+    if (full_few_rows(samples_per_code, num_noncoherent > 1, form == FMDBZP_FULL_AXIS31, ndop * nprn))
+        return FMDBZP_FULL_NONE;
+    return form;
 }
 
 int fmdbzp_plan_call_kernels(fmdbzp_plan* plan, int32_t eltype, int32_t nreq, uint32_t flags, char* buf, size_t buflen)

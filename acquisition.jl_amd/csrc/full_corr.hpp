@@ -1458,8 +1458,11 @@ k_column_bitsplit(ColumnArgs A)
 #define BITSPLIT_ALL(OP) OP(10) OP(11) OP(12) OP(15) OP(16) OP(20) OP(22)
 
 // ---------------------------------------------------------------------------
-// Code periods of 31 RB RC samples with 31, RB and RC pairwise coprime: every
-// multiple of the 1.023 MHz chip rate up to 20.46 MHz (1023 = 3 11 31). By
+// Code periods of 31 RB RC samples with 31, RB and RC pairwise coprime, RB and
+// RC radices of the switches below, at most 16384 samples: of the multiples of
+// the 1.023 MHz chip rate (1023 = 3 11 31) the 2, 3, 4, 5, 6, 8, 10 and 16 fold. The
+// others (7, 9, 11 to 15, 17 to 20) have no such axes or do not fit, and a
+// factor 31 no radix in k_full_corr: they run on the tile. By
 // Good-Thomas the transform is three independent DFTs along the axes of a
 // 31 x RB x RC array, with no twiddles: f = sum_i f_i N / q_i, n and tau by
 // their residues. The 31-point DFTs, the largest part of the arithmetic on

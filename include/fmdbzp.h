@@ -369,6 +369,20 @@ int fmdbzp_plan_column_kernel(fmdbzp_plan* plan, char* buf, size_t buflen);
  * No counterpart in the reference; for tests and reports. */
 int fmdbzp_plan_call_kernels(fmdbzp_plan* plan, int32_t eltype, int32_t nreq, uint32_t flags, char* buf,
                              size_t buflen);
+/* Form of the full-period correlation that a statistics-only FP32 call over
+ * nprn PRNs runs, on a simple-path plan of those PRNs; host only, for cost models.
+ * FMDBZP_FULL_NONE: the tile. It depends on the factors of the code period, not
+ * on the FFT size. 31-axis: 31 a b samples, a and b coprime radices of its
+ * stages, up to 16384 samples: of the multiples of 1023 the 2, 3, 4, 5, 6, 8, 10
+ * and 16 fold. Radices: no prime factor above 13, up to 20480 samples.
+ * FMDBZP_EINVAL on a non-positive size. */
+enum fmdbzp_full_form {
+    FMDBZP_FULL_NONE = 0,
+    FMDBZP_FULL_RADIX = 1,
+    FMDBZP_FULL_AXIS31 = 2
+};
+int fmdbzp_full_period_form(int32_t samples_per_code, int32_t num_blocks, int32_t num_coh, int32_t num_noncoherent,
+                            int32_t nprn);
 int fmdbzp_plan_kernel_times(fmdbzp_plan* plan, double* total_ms, int64_t* launches, int32_t n);
 
 /*
