@@ -22,6 +22,7 @@ from typing import Dict, List, Optional, Sequence, Tuple
 
 import numpy as np
 
+from ._native import full_period_form
 from .plan import ArgumentError, nextprod
 from .systems import GNSSSystem
 
@@ -216,10 +217,19 @@ def format_recommendations(rs: Sequence[SamplingFreqRecommendation]) -> str:
 # ---------------------------------------------------------------------------
 # Cost model of this engine
 # ---------------------------------------------------------------------------
+# transform sizes of compile-time block correlations
+_CORR_STATIC = (400, 500, 800, 2000, 2048, 2500, 4000)
+
+
 def _corr_variant(F: int) -> str:
     """The block-correlation kernel the engine runs for transform size F:
-    compile-time transforms for 500, 2048 and 2500, the runtime-radix one
+    compile-time transforms for 500, 2048 and 2500 (and for 400, 800, 2000 and
+    4000, counted with the generic one), in-place stages ("fc", k_corr_fc) above
+    2048 points or with a prime above 5 in a middle stage, the runtime-radix one
     otherwise."""
+    if F not in _CORR_STATIC and 64 <= F <= 10240 and (F > 2048 or any(r > 5 and r not in (8, 16)
+                                                                       for r in _engine_radices(F, True)[1:-1])):
+        return "fc"
     return {500: "f500", 2048: "f2048", 2500: "f2500"}.get(F, "generic")
 
 
@@ -260,8 +270,10 @@ def _transform_work(n: int, radix16: bool) -> float:
 
 
 def _corr_work(nb: int, F: int, ndop: int) -> float:
-    """ndop·nb inverse transforms of F points per PRN-step."""
-    return ndop * nb * _transform_work(F, True)
+    """ndop·nb inverse transforms of F points per PRN-step. The in-place form
+    has no direct DFT of a large prime: its work counts as F·log2(F)."""
+    w = F * math.log2(F) if _corr_variant(F) == "fc" else _transform_work(F, True)
+    return ndop * nb * w
 
 
 def _column_work(spc: int, ndop: int) -> Tuple[float, float]:
@@ -271,41 +283,58 @@ def _column_work(spc: int, ndop: int) -> Tuple[float, float]:
     return float(ndop) * spc, spc * _transform_work(ndop, False) if ndop > 1 else 0.0
 
 
+def _full_work(spc: int, ndop: int, nprn: int) -> List[float]:
+    """Regressors of a full-period step: launch, one transform, all rows."""
+    v = spc * math.log2(spc)
+    return [1.0, v, nprn * ndop * v, float(nprn * ndop)]
+
+
 # Coefficients measured on one MI355X by GpuCostModel.calibrate() with its
-# default geometry set (GPS L1 C/A rates 4-20 MHz, N_coh 1-10, 8 and 32 PRNs):
-# per launch, corr = a0 + nprn·work·a1 and column = b0 + nprn·(cells·b1 +
-# work·b2), in seconds, with the work terms of _corr_work and _column_work.
+# default geometry sets (GPS L1 C/A rates 2-30 MHz, N_coh 1-10, 8 and 32 PRNs),
+# in seconds, in the form stated at GpuCostModel. On rates left out of the fit
+# the full-period steps come out within 25 %, the tile's launches mostly within 25 %
+# (k_corr_fc within a factor of 2: it covers 686 to 10240 points in one line).
 MI355X_COEFFS: Dict[str, Dict[str, Tuple[float, ...]]] = {
-    "corr": {"f500": (6.847e-06, 7.705e-14), "f2048": (1.676e-05, 3.355e-14), "f2500": (1.333e-05, 5.584e-14),
-             "generic": (1.019e-05, 8.947e-14)},
-    "column": {"c160": (2.381e-06, 2.469e-12, 0.0), "generic": (6.004e-06, 5.246e-12, 0.0)},
+    "corr": {"f500": (7.069e-06, 7.716e-14), "f2048": (1.756e-05, 3.345e-14), "f2500": (1.376e-05, 5.515e-14),
+             "generic": (1.042e-05, 8.898e-14), "fc": (1.463e-05, 3.270e-13)},
+    "column": {"c160": (3.447e-06, 2.429e-12, 0.0), "generic": (4.706e-06, 0.0, 1.371e-13)},
+    "full": {"radix": (7.005e-06, 1.244e-11, 2.912e-13, 0.0), "axis31": (3.885e-06, 1.905e-11, 2.192e-13, 1.207e-08)},
 }
 
 
 @dataclass
 class GpuCostModel:
-    """Predicted engine time of one PRN through one noncoherent step.
+    """Predicted engine time of one PRN through one noncoherent step of a
+    search that returns statistics (N_nc > 1).
 
-    Per kernel launch over `nprn` PRNs:
+    Where the full-period correlation serves the geometry (`full_period_form`),
+    its one kernel, per step over `nprn` PRNs:
+      t = c0 + V · c1 + nprn · ndop · (V · c2 + c3), V = spc · log2(spc)
+    (the second term is one row's transform, which few rows cannot hide).
+    Elsewhere the two kernels of the tile, per launch:
       block correlation  t = a0 + nprn · ndop·nb·W(F) · a1
       column stage       t = b0 + nprn · (ndop·spc · b1 + spc·W(ndop) · b2)
     where W(n) counts the float operations of one n-point transform over the
-    radix stages the engine plans for it (a direct DFT for primes above 5).
-    with (a0, a1) per correlation variant and (b0, b1, b2) per column variant,
-    all in seconds. The variant is the kernel the engine selects for the
-    geometry. `predict_step` returns (t_corr + t_column) / nprn.
+    radix stages the engine plans for it (a direct DFT for primes above 5; n log2(n)
+    in the in-place form), with (a0, a1) per correlation variant, (b0, b1, b2)
+    per column variant and (c0, ..., c3) per full-period form, all in seconds.
+    The variant is the kernel the engine selects for the geometry. `predict_launches` gives the tile's two
+    kernels for any geometry, `predict_step` the time of the kernels that a call
+    runs, divided by `nprn`. A model without full-period coefficients predicts
+    the tile throughout.
     """
     corr: Dict[str, Tuple[float, float]]
     column: Dict[str, Tuple[float, float, float]]
     nprn: int = 32
     device: str = ""
+    full: Dict[str, Tuple[float, float, float, float]] = field(default_factory=dict)
 
     @classmethod
     def mi355x(cls, nprn: int = 32) -> "GpuCostModel":
         if not MI355X_COEFFS["corr"]:
             raise RuntimeError("no MI355X coefficients recorded; use GpuCostModel.calibrate()")
-        return cls({k: tuple(v) for k, v in MI355X_COEFFS["corr"].items()},
-                   {k: tuple(v) for k, v in MI355X_COEFFS["column"].items()}, nprn, "MI355X")
+        t = {k: {v: tuple(c) for v, c in MI355X_COEFFS[k].items()} for k in ("corr", "column", "full")}
+        return cls(t["corr"], t["column"], nprn, "MI355X", t["full"])
 
     def _coef(self, table: dict, key: str):
         if key in table:
@@ -323,8 +352,11 @@ class GpuCostModel:
         return a0 + n * _corr_work(nb, F, ndop) * a1, b0 + n * (cells * b1 + work * b2)
 
     def predict_step(self, spc: int, nb: int, F: int, ndop: int, nprn: Optional[int] = None) -> float:
-        """Seconds per PRN and noncoherent step."""
+        """Seconds per PRN and noncoherent step of a call that returns statistics."""
         n = self.nprn if nprn is None else nprn
+        form = full_period_form(spc, nb, ndop // nb, 2, n) if self.full else ""
+        if form in self.full:
+            return float(np.dot(self.full[form], _full_work(spc, ndop, n))) / n
         tc, tk = self.predict_launches(spc, nb, F, ndop, n)
         return (tc + tk) / n
 
@@ -336,45 +368,60 @@ class GpuCostModel:
     # -- calibration on the device -------------------------------------------------
     DEFAULT_GEOMETRIES = ((4e6, 1), (5e6, 1), (5e6, 4), (8e6, 2), (10e6, 1), (10e6, 5), (12e6, 2),
                           (16.368e6, 1), (16.368e6, 4), (16.368e6, 10), (20e6, 1), (20e6, 10))
+    # further periods of 31 a b samples and sizes of the in-place correlation,
+    # which the set above has too few of
+    EXTRA_GEOMETRIES = ((2.046e6, 2), (3.069e6, 1), (5.115e6, 1), (5.115e6, 4), (8.184e6, 2), (10.23e6, 1), (10.23e6, 5),
+                        (9.207e6, 1), (14.7e6, 2), (24e6, 1), (30e6, 2))
 
     @staticmethod
     def measure(system: GNSSSystem, sampling_freq: float, num_coherently_integrated_code_periods: int,
                 nprn: int, *, min_doppler_coverage: float = 7000.0, repeats: int = 3, seed: int = 1) -> dict:
-        """Run the engine's tile kernels (the model's two stages) at one
-        geometry on the device (noise input, N_nc 2, `nprn` PRNs) and return
-        the geometry with the mean correlation and column kernel time per
+        """Run the engine at one geometry on the device (noise input, N_nc 2,
+        `nprn` PRNs) and return the geometry with the mean kernel times per
         noncoherent step and PRN batch (seconds), from the engine's HIP-event
-        timing. One correlation launch runs per step
-        and batch; a column launch may carry two steps (k_column_c160_pair),
-        so both totals are divided by the correlation launch count."""
+        timing: `corr_s` and `column_s` of the tile, `step_s` of the kernels that
+        a call returning statistics runs, and their `form` ("" for the tile).
+        One correlation launch runs per step and batch; a column launch may carry
+        two steps (k_column_c160_pair), so both totals are divided by the
+        correlation launch count. A full-period launch carries all steps."""
         from . import _native
         from .acquire import acquire_
-        from .plan import _plan_host
+        from .plan import plan_acquire
 
         N = num_coherently_integrated_code_periods
         prns = list(range(1, nprn + 1))
-        plan = _plan_host(system, sampling_freq, prns, min_doppler_coverage=min_doppler_coverage,
-                          num_coherently_integrated_code_periods=N, num_noncoherent_accumulations=2)
-        plan.tile_path = True
-        plan.native = _native.NativePlan.create(plan)
-        try:
-            spc, nb, F, ndop = plan.samples_per_code, plan.num_blocks, plan.fft_size, plan.num_doppler_bins
-            n = 2 * N * spc + spc
-            rng = np.random.default_rng(seed)
-            sig = (rng.standard_normal(n) + 1j * rng.standard_normal(n)).astype(np.complex64)
-            acquire_(plan, sig, prns, interm_freq=0.0)  # warm-up
-            plan.native.set_timing(True)
-            for _ in range(repeats):
-                acquire_(plan, sig, prns, interm_freq=0.0)
-            kt = plan.native.kernel_times()
-            plan.native.set_timing(False)
-        finally:
-            plan.close()
-        (mc, nc), (mk, nk) = kt["corr_tile"], kt["column"]
+
+        def times(tile):
+            plan = plan_acquire(system, sampling_freq, prns, min_doppler_coverage=min_doppler_coverage,
+                                num_coherently_integrated_code_periods=N, num_noncoherent_accumulations=2,
+                                _tile_path=tile)
+            try:
+                n = 2 * N * plan.samples_per_code + plan.samples_per_code
+                rng = np.random.default_rng(seed)
+                sig = (rng.standard_normal(n) + 1j * rng.standard_normal(n)).astype(np.complex64)
+                acquire_(plan, sig, prns, interm_freq=0.0)  # warm-up
+                plan.native.set_timing(True)
+                for _ in range(repeats):
+                    acquire_(plan, sig, prns, interm_freq=0.0)
+                kt = plan.native.kernel_times()
+                full = plan.native.call_kernels(_native.ELTYPE["cf32"], nprn).startswith("k_full")
+                return plan, kt["corr_tile"], kt["column"], full
+            finally:
+                plan.close()
+
+        plan, (mc, nc), (mk, nk), _ = times(True)
         if nc <= 0 or nk <= 0:
             raise RuntimeError("engine recorded no correlation or column launches")
-        return dict(fs=sampling_freq, N=N, nprn=nprn, spc=spc, nb=nb, F=F, ndop=ndop,
-                    corr_s=1e-3 * mc / nc, column_s=1e-3 * mk / nc)
+        spc, nb, F, ndop = plan.samples_per_code, plan.num_blocks, plan.fft_size, plan.num_doppler_bins
+        out = dict(fs=sampling_freq, N=N, nprn=nprn, spc=spc, nb=nb, F=F, ndop=ndop, corr_s=1e-3 * mc / nc,
+                   column_s=1e-3 * mk / nc, form="")
+        out["step_s"] = out["corr_s"] + out["column_s"]
+        if full_period_form(spc, nb, N, 2, nprn):
+            _, _, (mf, nf), full = times(False)
+            if full:
+                # launches per call: one per PRN batch, over both steps
+                out.update(form=full_period_form(spc, nb, N, 2, nprn), step_s=1e-3 * mf / nf / 2)
+        return out
 
     @classmethod
     def fit(cls, points: Sequence[dict], nprn: int = 32, device: str = "") -> "GpuCostModel":
@@ -384,12 +431,17 @@ class GpuCostModel:
 
         corr_rows: Dict[str, list] = {}
         col_rows: Dict[str, list] = {}
+        full_rows: Dict[str, list] = {}
         for p in points:
-            corr_rows.setdefault(_corr_variant(p["F"]), []).append(
-                ([1.0, p["nprn"] * _corr_work(p["nb"], p["F"], p["ndop"])], p["corr_s"]))
-            cells, work = _column_work(p["spc"], p["ndop"])
-            col_rows.setdefault(_column_variant(p["ndop"], p["spc"] // p["nb"]), []).append(
-                ([1.0, p["nprn"] * cells, p["nprn"] * work], p["column_s"]))
+            if p.get("form"):
+                full_rows.setdefault(p["form"], []).append((_full_work(p["spc"], p["ndop"], p["nprn"]), p["step_s"]))
+            if "corr_s" in p:
+                corr_rows.setdefault(_corr_variant(p["F"]), []).append(
+                    ([1.0, p["nprn"] * _corr_work(p["nb"], p["F"], p["ndop"])], p["corr_s"]))
+            if "column_s" in p:
+                cells, work = _column_work(p["spc"], p["ndop"])
+                col_rows.setdefault(_column_variant(p["ndop"], p["spc"] // p["nb"]), []).append(
+                    ([1.0, p["nprn"] * cells, p["nprn"] * work], p["column_s"]))
 
         def solve(rows, ncoef):
             A = np.array([r[0] for r in rows], dtype=np.float64)
@@ -402,7 +454,8 @@ class GpuCostModel:
 
         corr = {k: solve(v, 2) for k, v in corr_rows.items()}
         column = {k: solve(v, 3) for k, v in col_rows.items()}
-        return cls(corr, column, nprn, device)
+        full = {k: solve(v, 4) for k, v in full_rows.items()}
+        return cls(corr, column, nprn, device, full)
 
     @classmethod
     def calibrate(cls, system: Optional[GNSSSystem] = None, geometries=None, nprns=(8, 32),
@@ -415,6 +468,12 @@ class GpuCostModel:
         system = GPSL1CA() if system is None else system
         points = [cls.measure(system, fs, N, n, repeats=repeats)
                   for fs, N in (geometries or cls.DEFAULT_GEOMETRIES) for n in nprns]
+        if not geometries:
+            for fs, N in cls.EXTRA_GEOMETRIES:
+                for n in nprns:
+                    m = cls.measure(system, fs, N, n, repeats=repeats)
+                    drop = ("column_s",) if _corr_variant(m["F"]) == "fc" else ("corr_s", "column_s")
+                    points.append({k: v for k, v in m.items() if k not in drop})
         return cls.fit(points, nprn=max(nprns), device="calibrated"), points
 
 
@@ -510,8 +569,9 @@ def recommend_sampling_freqs(code_length_or_system, code_freq: Optional[float] =
 
 
 def _measure_and_rerank(cands, k, system, code_length, code_freq_hz, cov, N, nprn, key):
-    """Time the k best candidates on the device; their cost becomes the
-    measured microseconds per PRN-step and they are re-sorted ahead of the rest."""
+    """Time the k best candidates on the device, in the form that a call
+    returning statistics runs; their cost becomes the measured microseconds per
+    PRN-step and they are re-sorted ahead of the rest."""
     if system is None:
         from .systems import SeededCodeSystem
         system = SeededCodeSystem("seeded", code_length, code_freq_hz, 1575.42e6, 1, seed=0x5EED0006)
@@ -521,6 +581,6 @@ def _measure_and_rerank(cands, k, system, code_length, code_freq_hz, cov, N, npr
         if (m["spc"], m["nb"], m["F"], m["ndop"]) != (c.samples_per_code, c.num_blocks, c.inner_fft_size,
                                                       c.num_doppler_bins):
             raise RuntimeError(f"plan geometry at {c.sampling_freq} Hz differs from the recommender's: {m}")
-        head.append(replace(c, cost=1e6 * (m["corr_s"] + m["column_s"]) / nprn))
+        head.append(replace(c, cost=1e6 * m["step_s"] / nprn))
     head.sort(key=key)
     return head + cands[k:]
