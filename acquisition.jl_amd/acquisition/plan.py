@@ -342,9 +342,10 @@ def plan_acquire(system: GNSSSystem, sampling_freq: float, prns: Sequence[int], 
     FP16-operand complex DFT-matrix products on the matrix cores with FP32
     accumulation (direct rotation plans with 25 coherent periods and
     num_doppler_bins = 625 n1, n1 in {2, 4, 10, 20}: the E1-like searches at
-    +-5 to +-50 kHz). "auto" takes the FP16 tile per call where the plan and
-    the samples admit it, the matrix-core form where the plan admits it, else
-    FP32.
+    +-5 to +-50 kHz). "auto" runs FP32 where the full-period correlation serves
+    the call, else the FP16 tile where the plan and the samples admit it, the
+    matrix-core form at n1 = 10 and 20, else FP32. At n1 = 10 and 20 FP32 is the
+    faster form (32.3 and 72 ms per PRN-step at 25 MHz against 47.7 and 109).
 
     `graphs` (engine option): capture each call's kernel sequence in a hipGraph
     and replay it while calls repeat the same device signal buffer, sample

@@ -759,11 +759,12 @@ bool int_samples(int32_t eltype)
 
 // Whether a call over nreq PRNs runs the full-period correlation: not with
 // surfaces (their time is the copy to the caller, and the tile path's column
-// kernels stay the ones that write them), nor where FMDBZP_PREC_AUTO takes the
-// FP16 tile, nor with few rows.
-bool full_call(const fmdbzp_plan* P, int32_t eltype, int32_t nreq, bool store)
+// kernels stay the ones that write them), nor with few rows. Under
+// FMDBZP_PREC_AUTO it comes before the FP16 tile, being the faster form (2.00
+// against 3.40 ms for the 16.368 MHz search of 32 PRNs and 8 steps) and FP32.
+bool full_call(const fmdbzp_plan* P, int32_t nreq, bool store)
 {
-    return P->full && !store && !(P->tile_auto && int_samples(eltype)) && !full_few_rows(P, nreq);
+    return P->full && !store && !full_few_rows(P, nreq);
 }
 
 // Column-stage form of the plan on the tile (fmdbzp_plan_column_kernel).
@@ -1067,9 +1068,9 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
         }
     }
     // the matrix-core form of the E1-like search (nb = 25 n1, n1 = 2, 4, 10, 20);
-    // FMDBZP_PREC_AUTO takes it at n1 = 10 and 20, its documented choice (47.7
-    // and 109 ms per PRN-step at 25 MHz; k_column_rotbig took 55.6 and 132
-    // there, k_column_rot25 takes 32.3 and 72 in FP32)
+    // FMDBZP_PREC_AUTO takes it at n1 = 10 and 20, a fixed choice from when it
+    // was the faster one (47.7 and 109 ms per PRN-step at 25 MHz, k_column_rotbig
+    // 55.6 and 132); k_column_rot25 takes 32.3 and 72 in FP32
     if ((d.precision == FMDBZP_PREC_MFMA || d.precision == FMDBZP_PREC_AUTO) && P->rotbig && nb % 25 == 0 &&
         ndop == 25 * nb &&
         (nb / 25 == 2 || nb / 25 == 4 || nb / 25 == 10 || nb / 25 == 20) && d.num_secondary_rotations <= 32 &&
@@ -1604,7 +1605,7 @@ int fmdbzp_plan_call_kernels(fmdbzp_plan* plan, int32_t eltype, int32_t nreq, ui
     if (!elsize(eltype) && eltype != FMDBZP_C2BIT) return set_err(FMDBZP_EINVAL, "unknown eltype %d", eltype);
     std::lock_guard<std::mutex> lk(plan->mu);
     const fmdbzp_plan* P = plan;
-    if (full_call(P, eltype, nreq, (flags & FMDBZP_FLAG_STORE_SURFACES) != 0)) {
+    if (full_call(P, nreq, (flags & FMDBZP_FLAG_STORE_SURFACES) != 0)) {
         if (P->fp31.n) snprintf(buf, buflen, "k_full31_corr<%d>", P->full_nthr);
         else snprintf(buf, buflen, "k_full_corr<%d,%s>", P->full_nthr, P->d.num_noncoherent > 1 ? "true" : "false");
         return FMDBZP_OK;
@@ -2069,7 +2070,7 @@ int acquire_launch(fmdbzp_plan* P, const Work& W, const void* d_sig, int32_t elt
     const int spc = d.samples_per_code, spc_eff = d.samples_per_code_eff, nnc = d.num_noncoherent;
     const int64_t seglen = (int64_t)d.num_coh * spc;
     const size_t surf_cols = P->surf_bins > 0 ? (size_t)P->surf_bins : (size_t)spc_eff;
-    if (full_call(P, eltype, nreq, store)) return launch_full(P, W, d_sig, eltype, interm_freq_hz, nreq);
+    if (full_call(P, nreq, store)) return launch_full(P, W, d_sig, eltype, interm_freq_hz, nreq);
 
     // 1. downconvert + double-block FFTs of every segment
     {

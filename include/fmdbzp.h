@@ -82,10 +82,13 @@ enum fmdbzp_precision {
      * samples (I16, CI8, CI16, C2BIT) only; other plans are rejected at
      * creation and float samples at the search call (FMDBZP_EINVAL). */
     FMDBZP_PREC_TILE_FP16 = 1,
-    /* Per call: FMDBZP_PREC_TILE_FP16 when the plan admits it and the samples
-     * are integers, FMDBZP_PREC_MFMA on the plans that admit it with n1 = 10
-     * or 20, else FP32; never rejected. For
-     * batches of requests whose plans and sample types differ. */
+    /* Per call: FP32 where the full-period correlation runs (the faster form),
+     * else FMDBZP_PREC_TILE_FP16 when the plan admits it and the samples are
+     * integers, FMDBZP_PREC_MFMA on the plans that admit it with n1 = 10 or 20,
+     * else FP32; never rejected. For batches of requests whose plans and sample
+     * types differ. At n1 = 10 and 20 the choice is fixed, not the faster one:
+     * the matrix-core kernel takes 47.7 and 109 ms per PRN-step at 25 MHz, FP32
+     * (k_column_rot25) 32.3 and 72; take FMDBZP_PREC_FP32 for speed there. */
     FMDBZP_PREC_AUTO = 2,
     /* Mixed, on matrix cores: the column Doppler transforms of the secondary-
      * code rotation search run as complex DFT-matrix products on

@@ -68,7 +68,8 @@ def test_names_follow_samples_and_flags():
         q = plan.native.call_kernels
         assert q(CF32, 2) == "k_full31_corr<512>"
         assert q(CF32, 2, FLAG_STORE_SURFACES) == "k_corr_tile<2,true,2048> k_column_c160_pair<32,512>"
-        assert q(ELTYPE["i16"], 2) == "k_corr_tile<2,true,2048,fp16> k_column_c160_pair<32,512,fp16>"
+        want = "k_corr_tile<2,true,2048,fp16> k_column_c160_pair<32,512,fp16>"
+        assert q(ELTYPE["i16"], 2, FLAG_STORE_SURFACES) == want
         with pytest.raises(EngineError, match="eltype"):
             q(99, 1)
         with pytest.raises(EngineError, match="nreq"):
