@@ -345,7 +345,7 @@ def plan_acquire(system: GNSSSystem, sampling_freq: float, prns: Sequence[int], 
     +-5 to +-50 kHz). "auto" runs FP32 where the full-period correlation serves
     the call, else the FP16 tile where the plan and the samples admit it, the
     matrix-core form at n1 = 10 and 20, else FP32. At n1 = 10 and 20 FP32 is the
-    faster form (32.3 and 72 ms per PRN-step at 25 MHz against 47.7 and 109).
+    faster form (34.5 and 79 ms per PRN-step at 25 MHz against 48.4 and 109).
 
     `graphs` (engine option): capture each call's kernel sequence in a hipGraph
     and replay it while calls repeat the same device signal buffer, sample

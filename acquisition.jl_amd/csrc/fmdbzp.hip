@@ -1092,8 +1092,8 @@ int fmdbzp_plan_create(const fmdbzp_plan_desc* desc, int32_t nprn, const int8_t*
     }
     // the matrix-core form of the E1-like search (nb = 25 n1, n1 = 2, 4, 10, 20);
     // FMDBZP_PREC_AUTO takes it at n1 = 10 and 20, a fixed choice from when it
-    // was the faster one (47.7 and 109 ms per PRN-step at 25 MHz, k_column_rotbig
-    // 55.6 and 132); k_column_rot25 takes 32.3 and 72 in FP32
+    // was the faster one (48.4 and 109 ms per PRN-step at 25 MHz over two steps,
+    // k_column_rotbig 57.4 and 132); k_column_rot25 takes 34.5 and 79 in FP32
     if ((d.precision == FMDBZP_PREC_MFMA || d.precision == FMDBZP_PREC_AUTO) && P->rotbig && nb % 25 == 0 &&
         ndop == 25 * nb &&
         (nb / 25 == 2 || nb / 25 == 4 || nb / 25 == 10 || nb / 25 == 20) && d.num_secondary_rotations <= 32 &&

@@ -320,8 +320,7 @@ def run_mixed_batch(args):
     if "mixed" in legs:
         mx = legs["mixed"]
         mixed = {"form": "per request: FP16-operand DFT-matrix products on the matrix cores for the E1-like "
-                         "rotation searches at +-25 and +-50 kHz (n1 = 10, 20), FP16 coherent tile for integer-"
-                         "sample 160-bin plans, else the FP32 path",
+                         "rotation searches at +-25 and +-50 kHz (n1 = 10, 20), else the FP32 path",
                  "value": round(cells_all / mx["t"], 1), "seconds": round(mx["t"], 3),
                  "kernel_seconds": {k: round(v / 1e3, 3) for k, v in mx["kern"].items() if v},
                  "detections": dict(mx["det"]), "roofline": leg_roofline(mx)}

@@ -87,8 +87,8 @@ enum fmdbzp_precision {
      * integers, FMDBZP_PREC_MFMA on the plans that admit it with n1 = 10 or 20,
      * else FP32; never rejected. For batches of requests whose plans and sample
      * types differ. At n1 = 10 and 20 the choice is fixed, not the faster one:
-     * the matrix-core kernel takes 47.7 and 109 ms per PRN-step at 25 MHz, FP32
-     * (k_column_rot25) 32.3 and 72; take FMDBZP_PREC_FP32 for speed there. */
+     * the matrix-core kernel takes 48.4 and 109 ms per PRN-step at 25 MHz, FP32
+     * (k_column_rot25) 34.5 and 79 (two steps); take FMDBZP_PREC_FP32 for speed. */
     FMDBZP_PREC_AUTO = 2,
     /* Mixed, on matrix cores: the column Doppler transforms of the secondary-
      * code rotation search run as complex DFT-matrix products on
@@ -116,7 +116,8 @@ enum fmdbzp_precision {
 /* At plan creation, time the admissible launch configurations of the block
  * correlation (buffering, transforms per pass, pass split) and of the generic
  * simple column kernel (columns per workgroup) on the plan's workspace and
- * keep the fastest; choices are cached per geometry for the process. The
+ * keep the fastest, for the calls that run on the tile (the full-period
+ * correlation has none); choices are cached per geometry for the process. The
  * reference plans its FFTs by measurement (FFTW MEASURE, src/plan.jl:468-483).
  * The environment variable FMDBZP_AUTOTUNE=1 turns it on for every plan. */
 #define FMDBZP_OPT_AUTOTUNE 0x4
